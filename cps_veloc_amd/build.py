@@ -11,6 +11,7 @@ LIB = os.path.join(HERE, "libcps_dwf_gpu.so")
 SOURCES = [os.path.join(HERE, "csrc", "dwf_gpu.hip"), os.path.join(HERE, "csrc", "synth.cpp"),
            os.path.join(HERE, "csrc", "nersc.cpp")]
 HEADERS = [os.path.join(HERE, "csrc", "dwf_kernels.hpp"),
+           os.path.join(HERE, "csrc", "hop64.hpp"),
            os.path.join(HERE, "csrc", "ptc_kernels.hpp"),
            os.path.join(ROOT, "include", "dwf_gpu.h"),
            os.path.join(ROOT, "include", "roofline.h"),

@@ -19,6 +19,7 @@
 #include "dwf_gpu.h"
 #include "dwf_synth.h"
 #include "dwf_kernels.hpp"
+#include "hop64.hpp"
 #include "ptc_kernels.hpp"
 #include "roofline.h"
 
@@ -99,6 +100,9 @@ struct dwfgpu_s {
   double* dalpha = nullptr;  // alphas of the pending sloppy CG steps (device)
   double* hring = nullptr;   // pinned copies of the sloppy CG scalars, per step
   int grid_hop = 0;
+  // the small-lattice FP64 hop kernels (hop64.hpp): sites per work-group (0:
+  // this lattice takes the general ones) and work-groups
+  int ns64 = 0, grid64 = 0;
   int ns = 16;  // sites per work-group of the hopping kernels (x); y = all slices
   int max_lds = 65536;
   // launch shape of the many-RHS operator chosen by the autotuner, per
@@ -365,6 +369,80 @@ struct Scratch {
   double* dscal;
 };
 
+// Launch shape of the small-lattice FP64 hop kernels.  They win while the
+// chip has SIMDs to spare for four threads per (site, slice).  FP64
+// MatPcDagMatPc, general / small-lattice us: Mobius 8^4 Ls 8 60.3 / 48.0, DWF
+// 8^3x16 Ls 8 60.4 / 56.0, Mobius 8^3x16 Ls 12 71.8 / 83.3, DWF 8^3x32 Ls 12
+// 91.1 / 122, Mobius 12^4 Ls 12 126 / 175: the line is at 32 Ki (site, slice)
+// pairs.  8 sites a work-group (128-byte rows; 4 cost DWF 8^4 45.5 -> 48.2 us),
+// 4 where 8 would leave most CUs without one (4^3x8 39.8 -> 37.2 us) or Ls is
+// too long for 8 (512 threads).
+constexpr size_t SMALL64_MAX = 32768;
+size_t lds64(const dwfgpu_s* h, int ns) {
+  return std::max(dwfk::lds64_cols(ns, h->ls), h->action == DWFGPU_DWF
+                                                   ? dwfk::lds64_links(ns, 2)
+                                                   : dwfk::lds64_tx(ns, h->ls));
+}
+void set_shape64(dwfgpu_s* h) {
+  h->ns64 = h->grid64 = 0;
+  if ((size_t)h->g.vh * h->ls > SMALL64_MAX) return;
+  int ns = h->g.vh > 512 ? 8 : 4;
+  while (ns > 4 && (4 * ns * h->ls > 512 || lds64(h, ns) > (size_t)h->max_lds)) ns /= 2;
+  if (4 * ns * h->ls > 512 || lds64(h, ns) > (size_t)h->max_lds) return;
+  h->ns64 = ns;
+  h->grid64 = (h->g.vh + ns - 1) / ns;
+}
+
+// Small-lattice FP64 DWF pass: out = D in (epi 0), x0 + alpha D in (epi 1,
+// |.|^2 partials if norm), or (scal) r -= alpha_cg of the latter with |r|^2
+// partials.  masses: nrhs right-hand sides, n/2 components apart (device).
+int dwf64(dwfgpu_s* h, const Geom& g, cx<double>* out, const cx<double>* in, const cx<double>* x0,
+          int cb_in, int dag, int epi, bool norm, double nm, double alpha, double* partial,
+          cx<double>* r, const double* scal, const double* masses = nullptr, int nrhs = 1) {
+  const dim3 grid(h->grid64, nrhs), block(2 * h->ns64, h->ls, 2);
+  const size_t lds = lds64(h, h->ns64);
+  const cx<double>* u = (const cx<double>*)h->f[DWFGPU_F64].U;
+#define DWF64_LAUNCH(DAG, EPI, NORM, CG)                                                         \
+  hipLaunchKernelGGL((dwfk::k_dwf64<DAG, EPI, NORM, CG>), grid, block, lds, h->st, out, in, u,   \
+                     x0, partial, g, cb_in, 2.0 * h->a5inv, nm, alpha, r, scal, masses, h->n / 2)
+  if (scal) DWF64_LAUNCH(1, 1, false, true);
+  else if (epi == 0 && dag) DWF64_LAUNCH(1, 0, false, false);
+  else if (epi == 0) DWF64_LAUNCH(0, 0, false, false);
+  else if (norm && dag) DWF64_LAUNCH(1, 1, true, false);
+  else if (norm) DWF64_LAUNCH(0, 1, true, false);
+  else if (dag) DWF64_LAUNCH(1, 1, false, false);
+  else DWF64_LAUNCH(0, 1, false, false);
+#undef DWF64_LAUNCH
+  HIPCHK(hipGetLastError());
+  return DWFGPU_OK;
+}
+
+// Small-lattice FP64 Mobius pass; fl: dwfk::FL_*, with FL_CG r and scal as above
+int mob64(dwfgpu_s* h, const Geom& g, const MobArgs& a, cx<double>* out, const cx<double>* in,
+          const cx<double>* psi, int p_out, int dag, int epi, int fl, double* partial,
+          cx<double>* r, const double* scal) {
+  using namespace dwfk;
+  const dim3 grid(h->grid64), block(2 * h->ns64, h->ls, 2);
+  const size_t lds = std::max(lds64_cols(h->ns64, h->ls), !dag && !(fl & FL_PRE_T)
+                                                               ? lds64_tx(h->ns64, h->ls)
+                                                               : lds64_links(h->ns64, 1));
+  const cx<double>* u = (const cx<double>*)h->f[DWFGPU_F64].U;
+#define MOB64_LAUNCH(DAG, EPI, FL)                                                              \
+  hipLaunchKernelGGL((k_mobius64<DAG, EPI, FL>), grid, block, lds, h->st, out, in, psi, u,      \
+                     partial, g, p_out, a, r, scal)
+  if (!dag && epi == EPI_M5INV) MOB64_LAUNCH(0, EPI_M5INV, FL_POST_T);
+  else if (!dag && epi == EPI_SCHUR && (fl & FL_NORM)) MOB64_LAUNCH(0, EPI_SCHUR, FL_PRE_T | FL_NORM);
+  else if (!dag && epi == EPI_SCHUR) MOB64_LAUNCH(0, EPI_SCHUR, FL_PRE_T);
+  else if (!dag) MOB64_LAUNCH(0, EPI_PLAIN, 0);
+  else if (epi == EPI_M5INV) MOB64_LAUNCH(1, EPI_M5INV, 0);
+  else if (epi == EPI_SCHUR && (fl & FL_CG)) MOB64_LAUNCH(1, EPI_SCHUR, FL_CG);
+  else if (epi == EPI_SCHUR) MOB64_LAUNCH(1, EPI_SCHUR, 0);
+  else MOB64_LAUNCH(1, EPI_PLAIN, 0);
+#undef MOB64_LAUNCH
+  HIPCHK(hipGetLastError());
+  return DWFGPU_OK;
+}
+
 // ---------------------------------------------------------------------------
 // operator pieces for storage policy P
 // ---------------------------------------------------------------------------
@@ -381,9 +459,13 @@ struct Ops {
     const dim3 grid(h->grid_hop), block(h->ns, h->ls);
     const double two_a5 = 2.0 * h->a5inv, nm = -2.0 * mass * h->a5inv;
     const S* u = (const S*)F(h).U;
-    const size_t lds = link_lds_bytes(h, 2, sizeof(R));
     Geom gm = h->g;
     gm.rev = epi;  // the x0 + alpha D passes sweep backwards, as the Schur ones in mob()
+    if constexpr (std::is_same<P, P64>::value)
+      if (h->ns64)
+        return dwf64(h, gm, (cx<double>*)out.d, (const cx<double>*)in.d, (const cx<double>*)x0.d,
+                     cb_in, dag, epi, norm, nm, alpha, partial, nullptr, nullptr);
+    const size_t lds = link_lds_bytes(h, 2, sizeof(R));
 #define DWF_LAUNCH(DAG, EPI, NORM)                                                           \
   hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, DAG, EPI, NORM>), grid, block, lds, h->st,       \
                      fld<P>(out), cfld<P>(in), u, cfld<P>(x0), partial, gm, cb_in, two_a5,    \
@@ -413,6 +495,10 @@ struct Ops {
     Geom gm = h->g;
     gm.rev = epi == dwfk::EPI_SCHUR ? 1 : 0;
     const S* u = (const S*)F(h).U;
+    if constexpr (std::is_same<P, P64>::value)
+      if (h->ns64)
+        return mob64(h, gm, a, (cx<double>*)out.d, (const cx<double>*)in.d,
+                     (const cx<double>*)psi.d, p_out, dag, epi, fl, partial, nullptr, nullptr);
     const bool col = dag || epi == dwfk::EPI_M5INV || epi == dwfk::EPI_SCHUR;
     // exchange slots after the links; the M5^-1 / Schur s-columns reuse the
     // LDS from offset 0 once the hop is done
@@ -486,18 +572,28 @@ struct Ops {
   static int mob_cg_last(dwfgpu_s* h, double mass, const DVec& te, const DVec& t1,
                          const DVec& r, const DVec& p, const DVec& x, const double* scal,
                          double* partial, const int* active) {
-    const dim3 grid(h->grid_hop), block(h->ns, h->ls);
-    const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), scal};
     MobArgs a = mob_args(h, mass, 1);
     a.active = active;
-    const size_t lds = std::max(link_lds_bytes(h, 1, sizeof(R)), col_lds_bytes(h, sizeof(R)));
     Geom gm = h->g;
     gm.rev = 1;  // a Schur pass: backwards, as in mob()
+    if constexpr (std::is_same<P, P64>::value && std::is_same<PX, dwfk::NoX>::value) {
+      if (h->ns64)
+        return mob64(h, gm, a, nullptr, (const cx<double>*)te.d, (const cx<double>*)t1.d, 1, 1,
+                     dwfk::EPI_SCHUR, dwfk::FL_CG, partial, (cx<double>*)r.d, scal);
+    }
+    const dim3 grid(h->grid_hop), block(h->ns, h->ls);
+    const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), scal};
+    const size_t lds = std::max(link_lds_bytes(h, 1, sizeof(R)), col_lds_bytes(h, sizeof(R)));
     hipLaunchKernelGGL((dwfk::k_mobius<P, 1, dwfk::EPI_SCHUR, dwfk::FL_CG, PX>), grid, block,
                        lds, h->st, fld<P>(te), cfld<P>(te), cfld<P>(t1), (const S*)F(h).U,
                        partial, gm, 1, a, cg);
     HIPCHK(hipGetLastError());
     return DWFGPU_OK;
+  }
+
+  // work-groups of a hop pass: the partial sums it leaves
+  static int grid(const dwfgpu_s* h) {
+    return std::is_same<P, P64>::value && h->ns64 ? h->grid64 : h->grid_hop;
   }
 
   static int m5inv(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, int dag) {
@@ -539,7 +635,7 @@ struct Ops {
   static int mdagm_w(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, double* dot,
                      const Scratch& w) {
     TRY(matpc_w(h, mass, w.t1, in, 0, dot != nullptr, w));
-    if (dot) TRY(fetch_sum_to(h, w.partial, h->grid_hop, w.dscal, dot));
+    if (dot) TRY(fetch_sum_to(h, w.partial, grid(h), w.dscal, dot));
     TRY(matpc_w(h, mass, out, w.t1, 1, false, w));
     return DWFGPU_OK;
   }
@@ -552,31 +648,36 @@ struct Ops {
   // d = <p, A p> -> dscal[1], a = rr / d, x += a p, r -= a A p, and
   // |r|^2 -> dscal[0] (mdagm_cg; *rr_new, *d receive the two scalars).
   // mdagm_cg_launch issues the kernels only: the |r|^2 partials are left in
-  // h->partial (grid_hop of them) and <p, A p> in dscal[1].
+  // h->partial (grid(h) of them) and <p, A p> in dscal[1].
   template <class PX>
   static int mdagm_cg_launch(dwfgpu_s* h, double mass, const DVec& p, const DVec& r,
                              const DVec& x) {
     const DVec& te = F(h).te;
     const DVec& t1 = F(h).t1;
-    const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), h->dscal};
-    const dim3 grid(h->grid_hop), block(h->ns, h->ls);
-    const S* u = (const S*)F(h).U;
     if (h->action == DWFGPU_DWF) {
       const double mk2 = -dwf_kappa(h) * dwf_kappa(h);
       TRY(dwf(h, mass, te, p, 1, 0, 0, DVec(), 0.0, false));
       TRY(dwf(h, mass, t1, te, 0, 0, 1, p, mk2, true));
-      TRY(reduce_to(h, h->grid_hop, 1));
+      TRY(reduce_to(h, grid(h), 1));
       TRY(dwf(h, mass, te, t1, 1, 1, 0, DVec(), 0.0, false));
       Geom gm = h->g;
       gm.rev = 1;  // an x0 + alpha D pass: backwards, as in dwf()
-      hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, 1, 1, false, true, PX>), grid, block,
-                         link_lds_bytes(h, 2, sizeof(R)), h->st, fld<P>(te), cfld<P>(te), u,
-                         cfld<P>(t1), h->partial, gm, 0, 2.0 * h->a5inv,
-                         -2.0 * mass * h->a5inv, mk2, cg);
+      if constexpr (std::is_same<P, P64>::value && std::is_same<PX, dwfk::NoX>::value) {
+        if (h->ns64)
+          return dwf64(h, gm, nullptr, (const cx<double>*)te.d, (const cx<double>*)t1.d, 0, 1, 1,
+                       false, -2.0 * mass * h->a5inv, mk2, h->partial, (cx<double>*)r.d, h->dscal);
+      }
+      {
+        const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), h->dscal};
+        hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, 1, 1, false, true, PX>), dim3(h->grid_hop),
+                           dim3(h->ns, h->ls), link_lds_bytes(h, 2, sizeof(R)), h->st, fld<P>(te),
+                           cfld<P>(te), (const S*)F(h).U, cfld<P>(t1), h->partial, gm, 0,
+                           2.0 * h->a5inv, -2.0 * mass * h->a5inv, mk2, cg);
+      }
     } else {
       TRY(mob_first(h, mass, te, p, 0));
       TRY(mob_second(h, mass, t1, te, p, 0, true));
-      TRY(reduce_to(h, h->grid_hop, 1));
+      TRY(reduce_to(h, grid(h), 1));
       TRY(mob_first(h, mass, te, t1, 1));
       TRY(mob_cg_last<PX>(h, mass, te, t1, r, p, x, h->dscal, h->partial, nullptr));
     }
@@ -588,7 +689,7 @@ struct Ops {
   static int mdagm_cg(dwfgpu_s* h, double mass, const DVec& p, const DVec& r, const DVec& x,
                       double* rr_new, double* d) {
     TRY(mdagm_cg_launch<PX>(h, mass, p, r, x));
-    TRY(reduce_to(h, h->grid_hop, 0));
+    TRY(reduce_to(h, grid(h), 0));
     double sc[2];
     TRY(fetch_scalars(h, 2, sc));
     *rr_new = sc[0];
@@ -918,7 +1019,7 @@ int invcg_mixed(dwfgpu_s* h, const dwfgpu_cg_arg* arg, double delta, const DVec&
     // k_reduce_cg_step the scalars and the step's alpha (x_s += a p_s pending)
     TRY(L::template mdagm_cg_launch<dwfk::NoX>(h, mass, ps, rs, DVec()));
     hipLaunchKernelGGL(dwfk::k_reduce_cg_step, dim3(1), dim3(1024), 0, h->st, h->partial,
-                       h->grid_hop, h->dscal, h->dalpha + slot);
+                       L::grid(h), h->dscal, h->dalpha + slot);
     HIPCHK(hipGetLastError());
     double* hs = h->hring + 4 * (itr % NEV);
     HIPCHK(hipMemcpyAsync(hs, h->dscal, 2 * sizeof(double), hipMemcpyDeviceToHost, h->st));
@@ -1056,7 +1157,7 @@ int time_mdagm(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, int re
     rec(b + 4);
     if (!st) {
       hipLaunchKernelGGL(dwfk::k_reduce_partials, dim3(1), dim3(1024), 0, h->st, h->partial,
-                         h->grid_hop, h->dscal);
+                         O::grid(h), h->dscal);
       if (hipGetLastError() != hipSuccess) st = DWFGPU_HIP_ERROR;
     }
   }
@@ -1743,7 +1844,7 @@ int mr_partials_per_rhs(const dwfgpu_s* h) { return (h->g.vh + MR_MIN_NS - 1) / 
 // Mobius passes' grid (the handle's hop shape, which may hold fewer than
 // MR_MIN_NS sites per work-group at long Ls)
 int mr_partials_stride(const dwfgpu_s* h) {
-  return std::max(mr_partials_per_rhs(h), h->grid_hop);
+  return std::max(mr_partials_per_rhs(h), std::max(h->grid_hop, h->grid64));
 }
 
 bool mr_shape_ok(const dwfgpu_s* h, const MrShape& t, int nrhs, size_t creal) {
@@ -1850,7 +1951,7 @@ int mr_mdagm_mob(dwfgpu_s* h, int nrhs, const DVec& out, const DVec& in, const D
                  const DVec& t1, const double* masses, const int* active, double* partial,
                  double* scal, const DVec* r, const DVec* x, bool cg) {
   typedef Ops<P> O;
-  const int gx = h->grid_hop;
+  const int gx = O::grid(h);
   for (int j = 0; j < nrhs; ++j) {
     const DVec inj = mslice<P>(h, in, j), tej = mslice<P>(h, te, j), t1j = mslice<P>(h, t1, j);
     TRY(O::mob_first(h, masses[j], tej, inj, 0, active + j));
@@ -1896,6 +1997,20 @@ std::vector<MrShape> mr_candidates(const dwfgpu_s* h, int nrhs, size_t creal) {
   return c;
 }
 
+// the shape that DWFGPU_MRHS_SHAPE="ns,nr" pins (*t left alone without it)
+int mr_pinned(const dwfgpu_s* h, int nrhs, size_t creal, MrShape* t) {
+  const char* env = getenv("DWFGPU_MRHS_SHAPE");
+  if (!env) return DWFGPU_OK;
+  int ns = 0, nr = 0;
+  if (sscanf(env, "%d,%d", &ns, &nr) != 2 || !mr_shape_ok(h, MrShape{ns, nr}, nrhs, creal)) {
+    set_err("DWFGPU_MRHS_SHAPE=%s: need ns >= %d, 1 <= nr <= nrhs, ns*Ls*nr <= 512 and the "
+            "LDS of the shape within the device limit", env, MR_MIN_NS);
+    return DWFGPU_BAD_ARG;
+  }
+  *t = MrShape{ns, nr};
+  return DWFGPU_OK;
+}
+
 // Project-written autotuner: time one batched MatPcDagMatPc (all RHS active)
 // for every candidate shape, twice, and keep the fastest; cached per handle,
 // sloppy precision and RHS count.
@@ -1906,18 +2021,11 @@ int mr_tune(dwfgpu_s* h, int nrhs, MrState<P>& m, const int* all_active, MrShape
     *best = MrShape{h->mr_ns[pi], h->mr_nr[pi]};
     return DWFGPU_OK;
   }
-  const char* env = getenv("DWFGPU_MRHS_SHAPE");  // "ns,nr" pins the shape
-  if (env) {
-    int ns = 0, nr = 0;
-    if (sscanf(env, "%d,%d", &ns, &nr) != 2 ||
-        !mr_shape_ok(h, MrShape{ns, nr}, nrhs, sizeof(typename P::R))) {
-      set_err("DWFGPU_MRHS_SHAPE=%s: need ns >= %d, 1 <= nr <= nrhs, ns*Ls*nr <= 512 and the "
-              "LDS of the shape within the device limit", env, MR_MIN_NS);
-      return DWFGPU_BAD_ARG;
-    }
-    *best = MrShape{ns, nr};
-    h->mr_ns[pi] = ns;
-    h->mr_nr[pi] = nr;
+  *best = MrShape{0, 0};
+  TRY(mr_pinned(h, nrhs, sizeof(typename P::R), best));
+  if (best->ns) {
+    h->mr_ns[pi] = best->ns;
+    h->mr_nr[pi] = best->nr;
     h->mr_nrhs[pi] = nrhs;
     return DWFGPU_OK;
   }
@@ -3107,7 +3215,7 @@ int scratch_setup(int dev) {
 
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// carve te, t1 (with their scales in the 16-bit formats), grid_hop partials
+// carve te, t1 (with their scales in the 16-bit formats), the hop's partials
 // and one device scalar out of base (nullptr: only count); returns the bytes
 template <class P>
 size_t carve_scratch(const dwfgpu_s* h, unsigned char* base, Scratch* w) {
@@ -3124,7 +3232,7 @@ size_t carve_scratch(const dwfgpu_s* h, unsigned char* base, Scratch* w) {
   te.sc = P::kScaled ? (float*)take(sb) : nullptr;
   t1.d = take(vb);
   t1.sc = P::kScaled ? (float*)take(sb) : nullptr;
-  double* partial = (double*)take(round256((size_t)h->grid_hop * sizeof(double)));
+  double* partial = (double*)take(round256((size_t)std::max(h->grid_hop, h->grid64) * sizeof(double)));
   double* dscal = (double*)take(256);
   if (w) *w = Scratch{te, t1, partial, dscal};
   return off;
@@ -3232,7 +3340,8 @@ int dwfgpu_create(const double* gauge, const int dims[4], int ls, int action, do
     return DWFGPU_BAD_ARG;
   }
   h->grid_hop = (h->g.vh + h->ns - 1) / h->ns;
-  h->npartial = h->grid_hop > dwfk::BLAS_BLOCKS ? h->grid_hop : dwfk::BLAS_BLOCKS;
+  set_shape64(h);
+  h->npartial = std::max({h->grid_hop, h->grid64, dwfk::BLAS_BLOCKS});
   int r = DWFGPU_OK;
   auto fail = [&](int code) {
     free_all(h);
@@ -3733,7 +3842,23 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
                          fld<P>(mslice<P>(h, m.ps, j)), cfld<P64>(mslice<P64>(h, in->v, j)), h->g);
     HIPCHK(hipGetLastError());
     MrShape t{h->ns, 1};
-    if (h->action == DWFGPU_DWF) {
+    if (h->action == DWFGPU_DWF && pidx<P>() == DWFGPU_F64 && h->ns64) {
+      // the passes of a single right-hand side on this lattice, all in one launch
+      TRY(mr_pinned(h, nrhs, sizeof(double), &t));
+      const double mk2 = -dwf_kappa(h) * dwf_kappa(h);
+      Geom fwd = h->g, back = h->g;
+      back.rev = 1;
+      cx<double> *in = (cx<double>*)m.ps.d, *out = (cx<double>*)m.rs.d;
+      cx<double> *te = (cx<double>*)m.te.d, *t1 = (cx<double>*)m.t1.d;
+      auto pass = [&](const Geom& g, cx<double>* o, cx<double>* i, cx<double>* x0, int dag) {
+        return dwf64(h, g, o, i, x0, x0 ? 0 : 1, dag, x0 ? 1 : 0, false, 0.0, x0 ? mk2 : 0.0,
+                     nullptr, nullptr, nullptr, m.mass, nrhs);
+      };
+      TRY(pass(fwd, te, in, nullptr, 0));
+      TRY(pass(back, t1, te, in, 0));
+      TRY(pass(fwd, te, t1, nullptr, 1));
+      TRY(pass(back, out, te, t1, 1));
+    } else if (h->action == DWFGPU_DWF) {
       TRY(mr_tune<P>(h, nrhs, m, m.active(), &t));
       TRY(mr_mdagm<P>(h, t, nrhs, m.rs, m.ps, m.te, m.t1, m.mass, m.active(), m.partial,
                       nullptr, nullptr, nullptr, false));

@@ -1031,8 +1031,8 @@ __device__ __forceinline__ void hop4(cx<R>* acc, const LD& ld, const cx<R>* lu, 
 // sum over the work-group; result valid in thread 0.  Fixed order, so the
 // total is reproducible run to run.
 __device__ __forceinline__ double block_sum(double v, double* sh) {
-  const int tid = threadIdx.x + blockDim.x * threadIdx.y;
-  const int nthr = blockDim.x * blockDim.y;
+  const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
+  const int nthr = blockDim.x * blockDim.y * blockDim.z;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
   if ((tid & 63) == 0) sh[tid >> 6] = v;
@@ -1282,8 +1282,8 @@ __device__ __forceinline__ void m5inv_column_reg(cx<R>* v, bool upper, const M5S
 template <int DAG, typename R>
 __device__ __forceinline__ void m5inv_columns(cx<R>* col, int sst, int ns, int nvalid, int ls,
                                               const M5Side& k) {
-  const int tid = threadIdx.x + blockDim.x * threadIdx.y;
-  const int nthr = blockDim.x * blockDim.y;
+  const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
+  const int nthr = blockDim.x * blockDim.y * blockDim.z;
   for (int w = tid; w < ns * 12; w += nthr) {
     const int cc = w / ns, sl = w - cc * ns;
     if (sl >= nvalid) continue;
