@@ -12,6 +12,7 @@ SOURCES = [os.path.join(HERE, "csrc", "dwf_gpu.hip"), os.path.join(HERE, "csrc",
            os.path.join(HERE, "csrc", "nersc.cpp")]
 HEADERS = [os.path.join(HERE, "csrc", "dwf_kernels.hpp"),
            os.path.join(HERE, "csrc", "hop64.hpp"),
+           os.path.join(HERE, "csrc", "host_copy.hpp"),
            os.path.join(HERE, "csrc", "ptc_kernels.hpp"),
            os.path.join(ROOT, "include", "dwf_gpu.h"),
            os.path.join(ROOT, "include", "roofline.h"),

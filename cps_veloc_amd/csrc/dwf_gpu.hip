@@ -20,6 +20,7 @@
 #include "dwf_synth.h"
 #include "dwf_kernels.hpp"
 #include "hop64.hpp"
+#include "host_copy.hpp"
 #include "ptc_kernels.hpp"
 #include "roofline.h"
 
@@ -897,8 +898,7 @@ struct Ops {
   }
 
   static int to_device(dwfgpu_s* h, const DVec& dst, const double* host) {
-    HIPCHK(hipMemcpyAsync(h->cps_stage, host, h->n * sizeof(double), hipMemcpyHostToDevice,
-                          h->st));
+    HIPCHK(hostcopy::copy(h->cps_stage, (void*)host, h->n * sizeof(double), false, h->st));
     hipLaunchKernelGGL((dwfk::k_cps_to_field<P>), dim3(2048), dim3(256), 0, h->st, fld<P>(dst),
                        (const double*)h->cps_stage, h->g);
     HIPCHK(hipGetLastError());
@@ -909,9 +909,7 @@ struct Ops {
     hipLaunchKernelGGL((dwfk::k_field_to_cps<P>), dim3(2048), dim3(256), 0, h->st,
                        (double*)h->cps_stage, cfld<P>(src), h->g);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(host, h->cps_stage, h->n * sizeof(double), hipMemcpyDeviceToHost,
-                          h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
+    HIPCHK(hostcopy::copy(h->cps_stage, host, h->n * sizeof(double), true, h->st));
     return DWFGPU_OK;
   }
 
@@ -3378,6 +3376,7 @@ int dwfgpu_create(const double* gauge, const int dims[4], int ls, int action, do
     set_err("dwfgpu_create: stream synchronize failed");
     return fail(DWFGPU_HIP_ERROR);
   }
+  hostcopy::retain();
   *out = h;
   return DWFGPU_OK;
 }
@@ -3385,6 +3384,7 @@ int dwfgpu_create(const double* gauge, const int dims[4], int ls, int action, do
 int dwfgpu_destroy(dwfgpu_t h) {
   if (!h) return DWFGPU_BAD_ARG;
   (void)hipStreamSynchronize(h->st);
+  hostcopy::release();
   free_all(h);
   delete h;
   return DWFGPU_OK;
@@ -4226,8 +4226,8 @@ int dwfgpu_fermion_from_canonical(dwfgpu_t h, dwfgpu_vec_t first, dwfgpu_vec_t s
   TRY(ensure_stage4d(h));
   const size_t v4r = (size_t)2 * h->g.vh * 24;
   for (int s = 0; s < h->ls; ++s) {
-    HIPCHK(hipMemcpyAsync(h->stage4d, canon + (size_t)s * v4r, v4r * sizeof(double),
-                          hipMemcpyHostToDevice, h->st));
+    HIPCHK(hostcopy::copy(h->stage4d, (void*)(canon + (size_t)s * v4r), v4r * sizeof(double),
+                          false, h->st));
     TRY(DISPATCH(h, canon_to_halves(h, first->v, second->v, h->stage4d, s, 1, 1)));
   }
   HIPCHK(hipStreamSynchronize(h->st));
@@ -4241,8 +4241,8 @@ int dwfgpu_fermion_to_canonical(dwfgpu_t h, double* canon, dwfgpu_vec_t first,
   const size_t v4r = (size_t)2 * h->g.vh * 24;
   for (int s = 0; s < h->ls; ++s) {
     TRY(DISPATCH(h, halves_to_canon(h, h->stage4d, first->v, second->v, s, 1, 1)));
-    HIPCHK(hipMemcpyAsync(canon + (size_t)s * v4r, h->stage4d, v4r * sizeof(double),
-                          hipMemcpyDeviceToHost, h->st));
+    HIPCHK(hostcopy::copy(h->stage4d, canon + (size_t)s * v4r, v4r * sizeof(double), true,
+                          h->st));
   }
   HIPCHK(hipStreamSynchronize(h->st));
   return DWFGPU_OK;
@@ -4254,7 +4254,7 @@ int dwfgpu_four2five(dwfgpu_t h, dwfgpu_vec_t first, dwfgpu_vec_t second, const 
   if (s_u < 0 || s_u >= h->ls || s_l < 0 || s_l >= h->ls) return DWFGPU_BAD_ARG;
   TRY(ensure_stage4d(h));
   const size_t v4r = (size_t)2 * h->g.vh * 24;
-  HIPCHK(hipMemcpyAsync(h->stage4d, four, v4r * sizeof(double), hipMemcpyHostToDevice, h->st));
+  HIPCHK(hostcopy::copy(h->stage4d, (void*)four, v4r * sizeof(double), false, h->st));
   for (int s = 0; s < h->ls; ++s)
     TRY(DISPATCH(h, canon_to_halves(h, first->v, second->v, h->stage4d, s, s == s_u ? 1 : 0,
                                     s == s_l ? 1 : 0)));
@@ -4271,8 +4271,7 @@ int dwfgpu_five2four(dwfgpu_t h, double* four, dwfgpu_vec_t first, dwfgpu_vec_t 
   HIPCHK(hipMemsetAsync(h->stage4d, 0, v4r * sizeof(double), h->st));
   TRY(DISPATCH(h, halves_to_canon(h, h->stage4d, first->v, second->v, s_u, 1, 0)));
   TRY(DISPATCH(h, halves_to_canon(h, h->stage4d, first->v, second->v, s_l, 0, 1)));
-  HIPCHK(hipMemcpyAsync(four, h->stage4d, v4r * sizeof(double), hipMemcpyDeviceToHost, h->st));
-  HIPCHK(hipStreamSynchronize(h->st));
+  HIPCHK(hostcopy::copy(h->stage4d, four, v4r * sizeof(double), true, h->st));
   return DWFGPU_OK;
 }
 

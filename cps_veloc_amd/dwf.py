@@ -448,8 +448,8 @@ class _DiracOpGpu:
         al = None if alpha is None else np.ascontiguousarray(alpha, np.float64)
         if psi is None:
             psi = np.zeros((ns if multi else 1) * self.n)
-        # the result goes into a copy: the caller's starting vector is kept
-        psi = np.array(psi, dtype=np.float64, copy=True).reshape(-1)
+        else:  # the result goes into a copy: the caller's starting vector is kept
+            psi = np.array(psi, dtype=np.float64, copy=True).reshape(-1)
         its = np.zeros(ns, dtype=np.int32)
         k = C.c_int()
         st = _chk(lib().dwfgpu_minvcg(self.h, mass, shifts, ns, psi, _arr(chi), -1.0, rs,
