@@ -2291,140 +2291,209 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
 // ===========================================================================
 namespace {
 
-// psi: MULTI nshift vectors (mvec layout), SINGLE one vector; scalars and
-// stop tests exactly as minvcg.C, the vector updates of all shifts fused
-// into one pass per iteration (k_minv_update).
+// psi: MULTI nshift vectors (mvec layout), SINGLE one vector; the recurrences
+// and stop tests of minvcg.C.  A step runs on the device alone (k_ms_*); the
+// host follows LAG steps behind with the shifts' coefficients, which only the
+// flushes need (k_ms_flush), and the stop tests, so up to LAG steps past the
+// last are run and thrown away.
+struct MsWork {
+  DVec p;              // directions of all shifts
+  void* mem = nullptr;  // the ring of residuals and the live p0
+  dwfk::MsStep* steps = nullptr;   // device
+  dwfk::MsStep* hsteps = nullptr;  // pinned, MS_SLOTS flushes
+  hipEvent_t ev[4] = {};
+  ~MsWork() {
+    free_vec(&p);
+    if (mem) (void)hipFree(mem);
+    if (steps) (void)hipFree(steps);
+    if (hsteps) (void)hipHostFree(hsteps);
+    for (auto e : ev)
+      if (e) (void)hipEventDestroy(e);
+  }
+};
+
 int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const DVec& psi,
                int multi, const double* alpha, const DVec& chi, double chi_norm, double* rsdcg,
                int max_num_iter, int* iters, int* k_out) {
   typedef Ops<P64> H;
+  typedef cx<double> C;
+  using namespace dwfk;
   TRY(ensure_work<P64>(h, 2));
-  const DVec& r = h->f[DWFGPU_F64].work[0];
-  const DVec& ap = h->f[DWFGPU_F64].work[1];
-  DVec pv;
-  TRY(alloc_mvec<P64>(h, nshift, &pv));
-  struct Free {
-    DVec* v;
-    ~Free() { free_vec(v); }
-  } fr{&pv};
-  const size_t vbytes = h->n / 2 * sizeof(cx<double>);
-  dwfk::ShiftArgs<P64> A;
-  std::memset(&A, 0, sizeof A);
-  A.nshift = nshift;
-  A.single = multi ? 0 : 1;
-  for (int s = 0; s < nshift; ++s) {
-    A.p[s] = (cx<double>*)mslice<P64>(h, pv, s).d;
-    A.psi[s] = (cx<double>*)(multi ? mslice<P64>(h, psi, s).d : psi.d);
+  const size_t n = h->n / 2, vbytes = n * sizeof(C);
+  constexpr int NEV = 4, MS_SLOTS = 4;
+  struct Drain {  // nothing queued outlives the work buffers
+    hipStream_t st;
+    ~Drain() { (void)hipStreamSynchronize(st); }
+  };
+  MsWork w;
+  Drain drain{h->st};
+  HIPCHK(hipMalloc(&w.p.d, (size_t)nshift * vbytes));
+  HIPCHK(hipMalloc((void**)&w.steps, MS_MAXK * sizeof(MsStep)));
+  HIPCHK(hipHostMalloc((void**)&w.hsteps, MS_SLOTS * MS_MAXK * sizeof(MsStep),
+                       hipHostMallocDefault));
+  for (auto& e : w.ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  // K pending steps and LAG steps ahead need K + LAG + 1 residuals; the live
+  // p0 is one vector more.  Where they do not fit, or the solve is too short to
+  // gain from them: every step flushed at once, the residual in place and p0
+  // the first shift's own direction.
+  int K = MS_MAXK, LAG = 2, NR = K + LAG + 1;
+  if (max_num_iter <= 4 || hipMalloc(&w.mem, (size_t)(NR + 1) * vbytes) != hipSuccess) {
+    (void)hipGetLastError();
+    w.mem = nullptr;
+    K = NR = 1;
+    LAG = 0;
   }
-  auto launch = [&](unsigned psi_mask, unsigned p_mask) -> int {
-    A.psi_mask = psi_mask;
-    A.p_mask = p_mask;
-    hipLaunchKernelGGL((dwfk::k_minv_update<P64>), blas_grid(), blas_block(), 0, h->st, A,
-                       cfld<P64>(r), h->g);
+  C* const ring = w.mem ? (C*)w.mem : (C*)h->f[DWFGPU_F64].work[0].d;
+  C* const ap = (C*)h->f[DWFGPU_F64].work[1].d;
+  C* const p0 = w.mem ? ring + (size_t)NR * n : (C*)w.p.d;
+  auto res = [&](int k) { return ring + (size_t)(k % NR) * n; };
+  DVec vp0, vap;
+  vp0.d = p0;
+  vap.d = ap;
+  const double sigma = shift[0] > 0 ? shift[0] : 0.0;  // the operator's own shift
+  const DVec& t1 = h->f[DWFGPU_F64].t1;
+
+  MsFlush F{};
+  F.psi = (C*)psi.d;
+  F.p = (C*)w.p.d;
+  F.chi = (const C*)chi.d;
+  F.vs = F.n = n;
+  F.nshift = nshift;
+  F.single = multi ? 0 : 1;
+  int slot = 0;
+  auto pending = [&]() { return w.hsteps + (size_t)slot * MS_MAXK + F.cnt; };
+  auto flush = [&]() -> int {
+    if (F.cnt == 0) return DWFGPU_OK;
+    HIPCHK(hipMemcpyAsync(w.steps, w.hsteps + (size_t)slot * MS_MAXK, F.cnt * sizeof(MsStep),
+                          hipMemcpyHostToDevice, h->st));
+    if (F.chi) F.active = nshift == 32 ? ~0u : (1u << nshift) - 1;  // every vector is first written
+    hipLaunchKernelGGL((F.cnt == 1 ? k_ms_flush<1> : k_ms_flush<MS_MAXK>), dim3(2048), dim3(256),
+                       0, h->st, F, w.steps);
     HIPCHK(hipGetLastError());
+    F.cnt = 0;
+    F.active = 0;
+    F.chi = nullptr;
+    slot = (slot + 1) % MS_SLOTS;
     return DWFGPU_OK;
   };
-  // d = <p0, (A + shift0) p0>
-  DVec p0 = mslice<P64>(h, pv, 0);
-  auto shifted_a = [&](double* d) -> int {
-    if (shift[0] > 0) {
-      TRY(H::mdagm(h, mass, ap, p0, nullptr));
-      TRY(H::axpby(h, ap, p0, shift[0], 1.0));
-      return dot<P64>(h, p0, ap, d);
-    }
-    return H::mdagm(h, mass, ap, p0, d);
+  // step k: p0 = r_k + a p0, then r_{k+1} = r_k + b (A + sigma) p0
+  auto step = [&](int k) -> int {
+    hipLaunchKernelGGL(k_ms_p, blas_grid(), blas_block(), 0, h->st, p0, res(k), h->dscal,
+                       k == 0 ? 1 : 0, n, h->partial);
+    HIPCHK(hipGetLastError());
+    TRY(reduce_to(h, BLAS_BLOCKS, MS_PP));
+    TRY(H::matpc(h, mass, t1, vp0, 0, true));
+    TRY(reduce_to(h, H::grid(h), MS_MP));
+    TRY(H::matpc(h, mass, vap, t1, 1, false));
+    hipLaunchKernelGGL(k_ms_r, blas_grid(), blas_block(), 0, h->st, res(k + 1), res(k), ap, p0,
+                       sigma, h->dscal, n, h->partial);
+    hipLaunchKernelGGL(k_ms_reduce, dim3(1), dim3(1024), 0, h->st, h->partial, (int)BLAS_BLOCKS,
+                       sigma, h->dscal);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(h->hring + 8 * (k % NEV), h->dscal, 5 * sizeof(double),
+                          hipMemcpyDeviceToHost, h->st));
+    HIPCHK(hipEventRecord(w.ev[k % NEV], h->st));
+    return DWFGPU_OK;
   };
-  if (multi) HIPCHK(hipMemsetAsync(psi.d, 0, (size_t)nshift * vbytes, h->st));  // :118-121
-  HIPCHK(hipMemcpyAsync(r.d, chi.d, vbytes, hipMemcpyDeviceToDevice, h->st));
-  for (int s = 0; s < nshift; ++s)
-    HIPCHK(hipMemcpyAsync(A.p[s], chi.d, vbytes, hipMemcpyDeviceToDevice, h->st));
-  double cp = chi_norm;
-  std::vector<double> rsd_sq(nshift), bs(nshift), z0(nshift), z1(nshift), fin(nshift);
+  HIPCHK(hipMemcpyAsync(res(0), chi.d, vbytes, hipMemcpyDeviceToDevice, h->st));
+  h->hscal[0] = chi_norm;
+  HIPCHK(hipMemcpyAsync(h->dscal + MS_C, h->hscal, sizeof(double), hipMemcpyHostToDevice, h->st));
+
+  double cp = chi_norm, c = chi_norm, b = 0.0, a = 0.0;
+  std::vector<double> rsd_sq(nshift), bs(nshift), z0(nshift, 1.0), z1(nshift, 1.0), fin(nshift),
+      f(nshift);
   double* z[2] = {z0.data(), z1.data()};
   std::vector<int> convs(nshift, 0), conv_at(nshift, 0);
-  for (int s = 0; s < nshift; ++s) rsd_sq[s] = cp * rsdcg[s] * rsdcg[s];
-  double d;
-  TRY(shifted_a(&d));
-  double b = -cp / d;
-  z[0][0] = 1.0;
-  z[1][0] = 1.0;
-  bs[0] = b;
-  int iz = 1;
-  for (int s = 1; s < nshift; ++s) {
-    z[1 - iz][s] = 1.0;
-    z[iz][s] = 1.0 / (1.0 - b * (shift[s] - shift[0]));
-    bs[s] = b * z[iz][s];
-  }
-  TRY(H::axpy_to(h, r, ap, r, b, true));  // r += b A p0
-  double c;
-  TRY(fetch_sum(h, dwfk::BLAS_BLOCKS, &c));
-  // the solution update of the first step is pending (psi_s -= bs_s chi with
-  // p_s = chi): it is applied with the next direction update or at the end
-  unsigned pending = 0;
-  for (int s = 0; s < nshift; ++s) {
-    A.fpsi[s] = multi ? -bs[s] : -bs[s] * alpha[s];
-    pending |= 1u << s;
-  }
-  int convp = c < rsd_sq[0] ? 1 : 0;
-  double a = c / cp;
-  int k;
-  for (k = 1; k <= max_num_iter && !convp; k++) {
-    a = c / cp;
-    unsigned pmask = 0;
+  for (int s = 0; s < nshift; ++s) rsd_sq[s] = chi_norm * rsdcg[s] * rsdcg[s];
+  int iz = 1, convp = 0;
+  unsigned todo = 0;  // shifts whose psi update by f is pending
+  // the entry of step k for the flush: the pending psi update, and the
+  // directions of step k from r_k
+  auto entry = [&](int k, bool directions) {
+    MsStep* e = pending();
+    unsigned moves = todo;
     for (int s = 0; s < nshift; ++s) {
-      if (convs[s]) continue;
-      pmask |= 1u << s;
-      if (s == 0) {
-        A.zr[0] = 1.0;
-        A.ap[0] = a;
-      } else {
-        A.zr[s] = z[iz][s];
-        A.ap[s] = a * (z[iz][s] * bs[s]) / (z[1 - iz][s] * b);
-      }
+      e->f[s] = (todo >> s) & 1u ? f[s] : 0.0;
+      e->zr[s] = 0.0;
+      e->ap[s] = 1.0;
+      // without a ring the first shift's direction is the live one
+      if (!directions || convs[s] || (s == 0 && !w.mem)) continue;
+      moves |= 1u << s;
+      e->zr[s] = s == 0 ? 1.0 : z[iz][s];
+      e->ap[s] = s == 0 ? a : a * (z[iz][s] * bs[s]) / (z[1 - iz][s] * b);
     }
-    TRY(launch(pending, pmask));
-    pending = 0;
+    F.r[F.cnt++] = res(k);
+    F.active |= moves;
+    todo = 0;
+  };
+  // the recurrences of step k from its scalars
+  auto follow = [&](int k, double c_new, double d) {
     cp = c;
-    TRY(shifted_a(&d));
     const double bp = b;
     b = -cp / d;
-    bs[0] = b;
-    iz = 1 - iz;
-    for (int s = 1; s < nshift; ++s) {
-      if (convs[s]) continue;
-      const double ztmp = z[1 - iz][s] * z[iz][s] * bp /
-                          (b * a * (z[iz][s] - z[1 - iz][s]) +
-                           z[iz][s] * bp * (1 - b * (shift[s] - shift[0])));
-      bs[s] = b * ztmp / z[1 - iz][s];
-      z[iz][s] = ztmp;
-    }
-    TRY(H::axpy_to(h, r, ap, r, b, true));
-    TRY(fetch_sum(h, dwfk::BLAS_BLOCKS, &c));
-    for (int s = 0; s < nshift; ++s) {
-      if (convs[s]) continue;
-      A.fpsi[s] = multi ? -bs[s] : -bs[s] * alpha[s];
-      pending |= 1u << s;
-    }
-    for (int s = 0; s < nshift; ++s) {
-      if (convs[s]) continue;
-      const double css = c * z[iz][s] * z[iz][s];
-      convs[s] = css < rsd_sq[s] ? 1 : 0;
-      if (convs[s]) {
-        fin[s] = css;
-        conv_at[s] = k;
+    if (k == 0) {
+      bs[0] = b;
+      for (int s = 1; s < nshift; ++s) {
+        z[iz][s] = 1.0 / (1.0 - b * (shift[s] - shift[0]));
+        bs[s] = b * z[iz][s];
+      }
+    } else {
+      bs[0] = b;
+      iz = 1 - iz;
+      for (int s = 1; s < nshift; ++s) {
+        if (convs[s]) continue;
+        const double ztmp = z[1 - iz][s] * z[iz][s] * bp /
+                            (b * a * (z[iz][s] - z[1 - iz][s]) +
+                             z[iz][s] * bp * (1 - b * (shift[s] - shift[0])));
+        bs[s] = b * ztmp / z[1 - iz][s];
+        z[iz][s] = ztmp;
       }
     }
-    convp = convs[0];
-    if (convp)
+    c = c_new;
+    for (int s = 0; s < nshift; ++s)
+      if (!convs[s]) {
+        f[s] = multi ? -bs[s] : -bs[s] * alpha[s];
+        todo |= 1u << s;
+      }
+    if (k == 0) {
+      convp = c < rsd_sq[0] ? 1 : 0;
+    } else {
+      for (int s = 0; s < nshift; ++s) {
+        if (convs[s]) continue;
+        const double css = c * z[iz][s] * z[iz][s];
+        convs[s] = css < rsd_sq[s] ? 1 : 0;
+        if (convs[s]) {
+          fin[s] = css;
+          conv_at[s] = k;
+        }
+      }
+      convp = 1;
       for (int s = 0; s < nshift; ++s)
         if (!convs[s]) convp = 0;
+    }
+    a = c / cp;
+  };
+  int done = -1;  // the last step the host has followed
+  for (int k = 0;; ++k) {
+    if (k <= max_num_iter || k == 0) TRY(step(k));
+    if (k < LAG) continue;
+    const int j = k - LAG;
+    HIPCHK(hipEventSynchronize(w.ev[j % NEV]));
+    const double* hs = h->hring + 8 * (j % NEV);
+    follow(j, hs[MS_C], hs[MS_D]);
+    done = j;
+    if (convp || j + 1 > max_num_iter) break;
+    entry(j + 1, true);
+    if (F.cnt == K) TRY(flush());
   }
-  if (pending) TRY(launch(pending, 0u));
+  entry(done + 1, false);  // the last step's solution update
+  TRY(flush());
   HIPCHK(hipStreamSynchronize(h->st));
-  for (int s = nshift - 1; s >= 0; s--) rsdcg[s] = std::sqrt(convs[s] ? fin[s] : c * z[iz][s] * z[iz][s]);
+  for (int s = nshift - 1; s >= 0; s--)
+    rsdcg[s] = std::sqrt(convs[s] ? fin[s] : c * z[iz][s] * z[iz][s]);
   if (iters)
     for (int s = 0; s < nshift; ++s) iters[s] = conv_at[s];
-  if (k_out) *k_out = k;
+  if (k_out) *k_out = done + 1;
   for (int s = 0; s < nshift; ++s)
     if (!convs[s]) return DWFGPU_MAXITER;
   return DWFGPU_OK;
