@@ -328,6 +328,42 @@ int ensure_ring(dwfgpu_s* h, int count) {
   return DWFGPU_OK;
 }
 
+// vectors of a ring (*n = count), or one where they would take more than a
+// quarter of the device's free memory
+template <class P>
+int ring_fits(dwfgpu_s* h, int count, int* n) {
+  size_t have = 0, total = 0, need = 0;
+  const std::vector<DVec>& ring = h->f[pidx<P>()].ring;
+  for (const DVec& v : ring) have += v.d ? 1 : 0;
+  *n = count;
+  if (have >= (size_t)count) return DWFGPU_OK;
+  need = (count - have) * (size_t)half_bytes<P>(h);
+  size_t avail = 0;
+  HIPCHK(hipMemGetInfo(&avail, &total));
+  if (need > avail / 4) *n = 1;
+  return DWFGPU_OK;
+}
+
+// events that mark the end of the last few steps
+template <int N>
+struct EventSet {
+  hipEvent_t e[N] = {};
+  int create() {
+    for (auto& x : e) HIPCHK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
+    return DWFGPU_OK;
+  }
+  ~EventSet() {
+    for (auto& x : e)
+      if (x) (void)hipEventDestroy(x);
+  }
+};
+
+// Pending solution updates of the plain CG.  Each is a vector of memory; the
+// flush moves (K + 2) / K vectors a step, 1.25 at 8 and 1.125 at 16.
+constexpr int CG_KRING = 8;
+// a solve capped at this many steps is too short for a ring of directions
+constexpr int CG_SHORT = 4;
+
 // ---------------------------------------------------------------------------
 // reductions
 // ---------------------------------------------------------------------------
@@ -765,19 +801,15 @@ struct Ops {
     TRY(axpy_to(h, res, mmp, src, -1.0, true));  // res = src - mmp
     double rr;
     TRY(fetch_sum(h, dwfk::BLAS_BLOCKS, &rr));
-    TRY(copy(h, dir, res));
     int itr = 0;
     int max_itr = arg->max_num_iter - 1;
     if (rr <= stp_cnd) max_itr = 0;
     int status = DWFGPU_OK;
-    // dscal[0] holds rr (fetch_sum above); each step replaces it by the new
-    // rr.  The hop epilogue updates res only; sol += a dir and dir = res + b
-    // dir follow in one pass (k_cg_xp), which reads dir once for both
-    for (int k = 0; k < max_itr; ++k) {
-      itr = itr + 1;
-      const double rr_prv = rr;
-      double d;
-      if (shift) {
+    if (shift) {
+      TRY(copy(h, dir, res));
+      for (int k = 0; k < max_itr; ++k) {
+        itr = itr + 1;
+        double d;
         bool stop = false;
         TRY(invcg_shifted_step(h, mass, *shift, sol, dir, res, mmp, stp_cnd, &rr, &d, &stop));
         if (d == 0.0) {
@@ -785,24 +817,9 @@ struct Ops {
           break;
         }
         if (stop) break;
-        continue;
       }
-      TRY(mdagm_cg<dwfk::NoX>(h, mass, dir, res, DVec(), &rr, &d));
-      if (d == 0.0) {  // a = 0 was used: res is unchanged
-        status = DWFGPU_BREAKDOWN;
-        break;
-      }
-      const double a = rr_prv / d;  // the epilogue's alpha (cg_alpha)
-      if (rr <= stp_cnd) {
-        hipLaunchKernelGGL((dwfk::k_cg_xp<P, P, false>), blas_grid(), blas_block(), 0, h->st,
-                           fld<P>(sol), fld<P>(dir), cfld<P>(res), a, 0.0, h->g);
-        HIPCHK(hipGetLastError());
-        break;
-      }
-      const double b = rr / rr_prv;
-      hipLaunchKernelGGL((dwfk::k_cg_xp<P, P, true>), blas_grid(), blas_block(), 0, h->st,
-                         fld<P>(sol), fld<P>(dir), cfld<P>(res), a, b, h->g);
-      HIPCHK(hipGetLastError());
+    } else if (max_itr > 0) {
+      TRY(invcg_steps(h, mass, sol, dir, res, stp_cnd, max_itr, &itr, &status));
     }
     // true residual |src - A sol| / |src|  (inv_cg.C:403-415)
     TRY(mdagm(h, mass, mmp, sol, nullptr));
@@ -814,6 +831,92 @@ struct Ops {
     if (iters) *iters = itr + 1;
     if (status == DWFGPU_OK && itr == arg->max_num_iter - 1) status = DWFGPU_MAXITER;
     return status;
+  }
+
+  // The steps of the plain CG: res holds the residual and dscal[0] its square.
+  // alpha and beta stay on the device, and the host looks at the scalars of a
+  // step (CPS's stop test, inv_cg.C:354) while the GPU runs the next, so that the
+  // GPU never waits for the host; one step past the last is run and not used.
+  // The directions of the last steps stay in a ring and sol += alpha_j dir_j is
+  // applied CG_KRING steps at a time (k_x_flush, the order and rounding of one
+  // update per step): 4.3 vectors move per step beside the operator where
+  // sol += a dir and dir = res + b dir in every step moved 5, and no speculative
+  // step ever reaches sol.  Moebius 24^3x64 Ls 12: 1004 -> 836 us a step (5.1
+  // TB/s); DWF 8^4 Ls 8, where the wait for the host and k_cg_xp's 12 components
+  // a thread cost more than the traffic: 5.3 -> 4.3 ms for 92 steps.  Without room
+  // for the ring (a quarter of the free memory), or for CG_SHORT steps, every step
+  // is waited for and applied at once, dir in place.
+  static int invcg_steps(dwfgpu_s* h, double mass, const DVec& sol, const DVec& dir,
+                         const DVec& res, double stp_cnd, int max_itr, int* itr_out,
+                         int* status) {
+    constexpr int NEV = 4;
+    int K = CG_KRING, LAG = 1, NR = K + LAG + 1;
+    if (max_itr <= CG_SHORT)
+      NR = 1;
+    else
+      TRY(ring_fits<P>(h, NR, &NR));
+    if (NR == 1) {
+      K = 1;
+      LAG = 0;
+    } else {
+      TRY(ensure_ring<P>(h, NR));
+    }
+    auto slot = [&](int k) -> const DVec& { return NR == 1 ? dir : F(h).ring[k % NR]; };
+    EventSet<NEV> ev;
+    TRY(ev.create());
+    dwfk::XFlush<P> xf;
+    xf.cnt = 0;
+    xf.alpha = h->dalpha;
+    auto flush = [&]() -> int {
+      if (xf.cnt == 0) return DWFGPU_OK;
+      hipLaunchKernelGGL((dwfk::k_x_flush<P, P>), blas_grid(), blas_block(), 0, h->st, fld<P>(sol),
+                         xf, h->g);
+      HIPCHK(hipGetLastError());
+      xf.cnt = 0;
+      return DWFGPU_OK;
+    };
+    TRY(copy(h, slot(1), res));
+    int itr = 0;
+    for (int k = 1; k <= max_itr + LAG; ++k) {
+      if (k <= max_itr) {
+        TRY(mdagm_cg_launch<dwfk::NoX>(h, mass, slot(k), res, DVec()));
+        hipLaunchKernelGGL(dwfk::k_reduce_cg_step, dim3(1), dim3(1024), 0, h->st, h->partial,
+                           grid(h), h->dscal, h->dalpha + k % NR);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(h->hring + 4 * (k % NEV), h->dscal, 2 * sizeof(double),
+                              hipMemcpyDeviceToHost, h->st));
+        HIPCHK(hipEventRecord(ev.e[k % NEV], h->st));
+      }
+      // dir of step k + 1 = res + b dir; in place only after step k's update
+      auto next = [&]() -> int {
+        if (k >= max_itr) return DWFGPU_OK;
+        hipLaunchKernelGGL((dwfk::k_pnext<P>), blas_grid(), blas_block(), 0, h->st,
+                           fld<P>(slot(k + 1)), cfld<P>(res), cfld<P>(slot(k)), h->dscal, h->g);
+        HIPCHK(hipGetLastError());
+        return DWFGPU_OK;
+      };
+      if (LAG) TRY(next());
+      const int j = k - LAG;
+      if (j < 1) continue;
+      HIPCHK(hipEventSynchronize(ev.e[j % NEV]));
+      const double rr = h->hring[4 * (j % NEV)], d = h->hring[4 * (j % NEV) + 1];
+      itr = j;
+      if (d == 0.0) {  // alpha = 0 was used: res is unchanged
+        *status = DWFGPU_BREAKDOWN;
+        break;
+      }
+      const DVec& p = slot(j);
+      xf.p[xf.cnt] = (const typename P::C*)p.d;
+      xf.sc[xf.cnt] = p.sc;
+      xf.ai[xf.cnt] = j % NR;
+      xf.cnt++;
+      if (xf.cnt == K) TRY(flush());
+      if (rr <= stp_cnd) break;
+      if (!LAG) TRY(next());
+    }
+    TRY(flush());
+    *itr_out = itr;
+    return DWFGPU_OK;
   }
 
   // one step of the shifted CG in CPS's order (inv_cg.C:293-363): mmp = A dir
@@ -997,14 +1100,8 @@ int invcg_mixed(dwfgpu_s* h, const dwfgpu_cg_arg* arg, double delta, const DVec&
   // its recurrence loses conjugacy between updates, and two-step-late
   // updates more than doubled its iteration count at 24^3x64 (3178 -> 7019).
   constexpr int LAG = std::is_same<PS, PBF16>::value ? 0 : 2, NEV = 4;
-  struct Events {
-    hipEvent_t e[NEV] = {};
-    ~Events() {
-      for (auto& x : e)
-        if (x) (void)hipEventDestroy(x);
-    }
-  } ev;
-  for (auto& x : ev.e) HIPCHK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
+  EventSet<NEV> ev;
+  TRY(ev.create());
   double rr_update = rr;  // |r|^2 at the last reliable update
   int itr = 0, nrel = 0, status = DWFGPU_OK;
   int fresh_from = 1;  // steps before this one were covered by a reliable update

@@ -1672,7 +1672,16 @@ k_cg_xp(Fld<PX> x, Fld<P> p, CFld<P> r, double a, double b, Geom g) {
   }
 }
 
-// pn = r + b p (the next CG direction into another buffer)
+// one chunk of an unscaled field, non-temporal as ld_spinor_once
+template <class P>
+__device__ __forceinline__ void ld_chunk(const typename P::C* p, cx<typename P::R>* v) {
+  const u32x4_t w = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+  typename P::C c;
+  __builtin_memcpy(&c, &w, 16);
+  chunk_unpack<P>(c, 1.0f, v);
+}
+
+// pn = r + b p (the next CG direction into another buffer, or in place)
 template <class P>
 __global__ void __launch_bounds__(BLAS_THREADS)
 k_pnext(Fld<P> pn, CFld<P> r, CFld<P> p, const double* __restrict__ scal, Geom g) {
@@ -1680,6 +1689,27 @@ k_pnext(Fld<P> pn, CFld<P> r, CFld<P> p, const double* __restrict__ scal, Geom g
   // beta = |r|^2 / the previous |r|^2 from the device scalars (k_reduce_cg_step)
   const double rr = scal[0], ro = scal[2];
   const R br = (R)(ro != 0.0 ? rr / ro : 0.0);
+  if constexpr (!P::kScaled) {
+    // no scale per site: chunk by chunk, four in flight per thread
+    const size_t n = (size_t)nch<P>() * g.vh * g.ls, stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t e0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e0 < n; e0 += 4 * stride) {
+      cx<R> rv[4][P::kCPC], pv[4][P::kCPC];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (e0 + u * stride < n) {
+          ld_chunk<P>(r.d + e0 + u * stride, rv[u]);
+          ld_chunk<P>(p.d + e0 + u * stride, pv[u]);
+        }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (e0 + u * stride < n) {
+#pragma unroll
+          for (int c = 0; c < P::kCPC; ++c) pv[u][c] = rv[u][c] + br * pv[u][c];
+          st_stream<P>(pn.d + e0 + u * stride, chunk_pack<P>(pv[u], 1.0f));
+        }
+    }
+    return;
+  }
   DWFK_SITE_LOOP(k, g) {
     cx<R> rv[12], pv[12];
     ld_site<P>(rv, r, g, k);
@@ -1706,6 +1736,30 @@ __global__ void __launch_bounds__(BLAS_THREADS)
 k_x_flush(Fld<PX> x, XFlush<P> f, Geom g) {
   typedef typename P::R R;
   typedef typename PX::R RX;
+  if constexpr (!P::kScaled && std::is_same<P, PX>::value) {
+    const size_t n = (size_t)nch<P>() * g.vh * g.ls;
+    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
+         e += (size_t)gridDim.x * blockDim.x) {
+      cx<R> xv[P::kCPC];
+      ld_chunk<P>(x.d + e, xv);
+      for (int j = 0; j < f.cnt; j += 4) {  // four directions in flight
+        cx<R> pv[4][P::kCPC];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (j + u < f.cnt) ld_chunk<P>(f.p[j + u] + e, pv[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (j + u < f.cnt) {
+            const double a = f.alpha[f.ai[j + u]];
+#pragma unroll
+            for (int c = 0; c < P::kCPC; ++c)
+              xv[c] = cx<R>{(R)(a * pv[u][c].re) + xv[c].re, (R)(a * pv[u][c].im) + xv[c].im};
+          }
+      }
+      st_stream<P>(x.d + e, chunk_pack<P>(xv, 1.0f));
+    }
+    return;
+  }
   DWFK_SITE_LOOP(k, g) {
     cx<RX> xv[12];
     ld_site<PX>(xv, CFld<PX>{x.d, x.sc}, g, k);
