@@ -370,7 +370,7 @@ constexpr int CG_SHORT = 4;
 // sum of nparts partials into the device scalar dscal[slot] (no host sync)
 int reduce_to(dwfgpu_s* h, int nparts, int slot) {
   hipLaunchKernelGGL(dwfk::k_reduce_partials, dim3(1), dim3(1024), 0, h->st, h->partial, nparts,
-                     h->dscal + slot);
+                     h->dscal + slot, (double*)nullptr);
   HIPCHK(hipGetLastError());
   return DWFGPU_OK;
 }
@@ -383,13 +383,16 @@ int fetch_scalars(dwfgpu_s* h, int n, double* out) {
   return DWFGPU_OK;
 }
 
-// sum of nparts partials in `partial` through the device scalar `dscal`, to
-// the host (waits)
-int fetch_sum_to(dwfgpu_s* h, const double* partial, int nparts, double* dscal, double* out) {
+// sum of nparts partials in `partial` into the device scalar `dscal` and the
+// pinned hscal[0], which holds it after the next wait
+int sum_to_host(dwfgpu_s* h, const double* partial, int nparts, double* dscal) {
   hipLaunchKernelGGL(dwfk::k_reduce_partials, dim3(1), dim3(1024), 0, h->st, partial, nparts,
-                     dscal);
+                     dscal, h->hscal);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(h->hscal, dscal, sizeof(double), hipMemcpyDeviceToHost, h->st));
+  return DWFGPU_OK;
+}
+int fetch_sum_to(dwfgpu_s* h, const double* partial, int nparts, double* dscal, double* out) {
+  TRY(sum_to_host(h, partial, nparts, dscal));
   HIPCHK(hipStreamSynchronize(h->st));
   *out = h->hscal[0];
   return DWFGPU_OK;
@@ -650,30 +653,40 @@ struct Ops {
   // the handle's own temporaries of this precision
   static Scratch own(dwfgpu_s* h) { return Scratch{F(h).te, F(h).t1, h->partial, h->dscal}; }
 
-  // MatPc / MatPcDag: out = M in (out on the CG parity).  norm -> partials.
+  // MatPc / MatPcDag: out = M in (out on the CG parity).  sum (dag 0): device
+  // scalar that receives |out|^2, and host (pinned) if given
   static int matpc_w(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, int dag,
-                     bool norm, const Scratch& w) {
+                     double* sum, double* host, const Scratch& w) {
     if (h->action == DWFGPU_DWF) {
       const double mk2 = -dwf_kappa(h) * dwf_kappa(h);
       TRY(dwf(h, mass, w.te, in, 1, dag, 0, DVec(), 0.0, false, w.partial));
-      TRY(dwf(h, mass, out, w.te, 0, dag, 1, in, mk2, norm, w.partial));
+      TRY(dwf(h, mass, out, w.te, 0, dag, 1, in, mk2, sum != nullptr, w.partial));
     } else {
       TRY(mob_first(h, mass, w.te, in, dag));
-      TRY(mob_second(h, mass, out, w.te, in, dag, norm, w.partial));
+      TRY(mob_second(h, mass, out, w.te, in, dag, sum != nullptr, w.partial));
+    }
+    if (sum) {
+      hipLaunchKernelGGL(dwfk::k_reduce_partials, dim3(1), dim3(1024), 0, h->st, w.partial,
+                         grid(h), sum, host);
+      HIPCHK(hipGetLastError());
     }
     return DWFGPU_OK;
   }
   static int matpc(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, int dag,
-                   bool norm) {
-    return matpc_w(h, mass, out, in, dag, norm, own(h));
+                   double* sum = nullptr) {
+    return matpc_w(h, mass, out, in, dag, sum, nullptr, own(h));
   }
 
-  // MatPcDagMatPc; *dot (if requested) = |MatPc in|^2 (dwf_mdagm.C:49-55)
+  // MatPcDagMatPc; *dot (if requested) = |MatPc in|^2 (dwf_mdagm.C:49-55), for
+  // which the host waits once, at the end
   static int mdagm_w(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, double* dot,
                      const Scratch& w) {
-    TRY(matpc_w(h, mass, w.t1, in, 0, dot != nullptr, w));
-    if (dot) TRY(fetch_sum_to(h, w.partial, grid(h), w.dscal, dot));
-    TRY(matpc_w(h, mass, out, w.t1, 1, false, w));
+    TRY(matpc_w(h, mass, w.t1, in, 0, dot ? w.dscal : nullptr, h->hscal, w));
+    TRY(matpc_w(h, mass, out, w.t1, 1, nullptr, nullptr, w));
+    if (dot) {
+      HIPCHK(hipStreamSynchronize(h->st));
+      *dot = h->hscal[0];
+    }
     return DWFGPU_OK;
   }
   static int mdagm(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, double* dot) {
@@ -682,20 +695,16 @@ struct Ops {
 
   // One CG step around MatPcDagMatPc (inv_cg.C:318-349) with the vector
   // updates fused into the last kernel: with rr = dscal[0] on entry,
-  // d = <p, A p> -> dscal[1], a = rr / d, x += a p, r -= a A p, and
-  // |r|^2 -> dscal[0] (mdagm_cg; *rr_new, *d receive the two scalars).
-  // mdagm_cg_launch issues the kernels only: the |r|^2 partials are left in
-  // h->partial (grid(h) of them) and <p, A p> in dscal[1].
+  // d = <p, A p> -> dscal[1], a = rr / d, x += a p, r -= a A p.
+  // mdagm_cg_launch leaves the |r|^2 partials in h->partial (grid(h) of them).
   template <class PX>
   static int mdagm_cg_launch(dwfgpu_s* h, double mass, const DVec& p, const DVec& r,
                              const DVec& x) {
     const DVec& te = F(h).te;
     const DVec& t1 = F(h).t1;
+    TRY(matpc(h, mass, t1, p, 0, h->dscal + 1));
     if (h->action == DWFGPU_DWF) {
       const double mk2 = -dwf_kappa(h) * dwf_kappa(h);
-      TRY(dwf(h, mass, te, p, 1, 0, 0, DVec(), 0.0, false));
-      TRY(dwf(h, mass, t1, te, 0, 0, 1, p, mk2, true));
-      TRY(reduce_to(h, grid(h), 1));
       TRY(dwf(h, mass, te, t1, 1, 1, 0, DVec(), 0.0, false));
       Geom gm = h->g;
       gm.rev = 1;  // an x0 + alpha D pass: backwards, as in dwf()
@@ -704,20 +713,26 @@ struct Ops {
           return dwf64(h, gm, nullptr, (const cx<double>*)te.d, (const cx<double>*)t1.d, 0, 1, 1,
                        false, -2.0 * mass * h->a5inv, mk2, h->partial, (cx<double>*)r.d, h->dscal);
       }
-      {
-        const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), h->dscal};
-        hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, 1, 1, false, true, PX>), dim3(h->grid_hop),
-                           dim3(h->ns, h->ls), link_lds_bytes(h, 2, sizeof(R)), h->st, fld<P>(te),
-                           cfld<P>(te), (const S*)F(h).U, cfld<P>(t1), h->partial, gm, 0,
-                           2.0 * h->a5inv, -2.0 * mass * h->a5inv, mk2, cg);
-      }
+      const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), h->dscal};
+      hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, 1, 1, false, true, PX>), dim3(h->grid_hop),
+                         dim3(h->ns, h->ls), link_lds_bytes(h, 2, sizeof(R)), h->st, fld<P>(te),
+                         cfld<P>(te), (const S*)F(h).U, cfld<P>(t1), h->partial, gm, 0,
+                         2.0 * h->a5inv, -2.0 * mass * h->a5inv, mk2, cg);
     } else {
-      TRY(mob_first(h, mass, te, p, 0));
-      TRY(mob_second(h, mass, t1, te, p, 0, true));
-      TRY(reduce_to(h, grid(h), 1));
       TRY(mob_first(h, mass, te, t1, 1));
       TRY(mob_cg_last<PX>(h, mass, te, t1, r, p, x, h->dscal, h->partial, nullptr));
     }
+    HIPCHK(hipGetLastError());
+    return DWFGPU_OK;
+  }
+  // the same with x left alone, and the end of the step: |r|^2 -> dscal[0], its
+  // previous value -> dscal[2], the step's alpha -> *alpha, and host[0..1]
+  // (pinned) = |r|^2, <p, A p> (k_reduce_cg_step)
+  static int cg_step(dwfgpu_s* h, double mass, const DVec& p, const DVec& r, double* alpha,
+                     double* host) {
+    TRY(mdagm_cg_launch<dwfk::NoX>(h, mass, p, r, DVec()));
+    hipLaunchKernelGGL(dwfk::k_reduce_cg_step, dim3(1), dim3(1024), 0, h->st, h->partial, grid(h),
+                       h->dscal, alpha, host);
     HIPCHK(hipGetLastError());
     return DWFGPU_OK;
   }
@@ -879,12 +894,7 @@ struct Ops {
     int itr = 0;
     for (int k = 1; k <= max_itr + LAG; ++k) {
       if (k <= max_itr) {
-        TRY(mdagm_cg_launch<dwfk::NoX>(h, mass, slot(k), res, DVec()));
-        hipLaunchKernelGGL(dwfk::k_reduce_cg_step, dim3(1), dim3(1024), 0, h->st, h->partial,
-                           grid(h), h->dscal, h->dalpha + k % NR);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(h->hring + 4 * (k % NEV), h->dscal, 2 * sizeof(double),
-                              hipMemcpyDeviceToHost, h->st));
+        TRY(cg_step(h, mass, slot(k), res, h->dalpha + k % NR, h->hring + 4 * (k % NEV)));
         HIPCHK(hipEventRecord(ev.e[k % NEV], h->st));
       }
       // dir of step k + 1 = res + b dir; in place only after step k's update
@@ -963,7 +973,7 @@ struct Ops {
       TRY(mob(h, mass, temp2, temp, DVec(), 1, 0, dwfk::EPI_PLAIN, 0));
       TRY(axpy_to(h, temp, temp2, in_second, mob_kappa_b(h), false));
     }
-    return matpc(h, mass, src, temp, 1, false);
+    return matpc(h, mass, src, temp, 1);
   }
   // the half of the solution the CG did not give (DWF: even from odd;
   // Mobius: even from odd, then both halves times 2 kappa_b), d_op_dwf.C:
@@ -1110,14 +1120,9 @@ int invcg_mixed(dwfgpu_s* h, const dwfgpu_cg_arg* arg, double delta, const DVec&
   while (!converged && itr < max_itr) {
     itr = itr + 1;
     const DVec& ps = ring[slot];
-    // dscal[0] holds |r_s|^2; the fused step updates r_s, and
-    // k_reduce_cg_step the scalars and the step's alpha (x_s += a p_s pending)
-    TRY(L::template mdagm_cg_launch<dwfk::NoX>(h, mass, ps, rs, DVec()));
-    hipLaunchKernelGGL(dwfk::k_reduce_cg_step, dim3(1), dim3(1024), 0, h->st, h->partial,
-                       L::grid(h), h->dscal, h->dalpha + slot);
-    HIPCHK(hipGetLastError());
-    double* hs = h->hring + 4 * (itr % NEV);
-    HIPCHK(hipMemcpyAsync(hs, h->dscal, 2 * sizeof(double), hipMemcpyDeviceToHost, h->st));
+    // dscal[0] holds |r_s|^2; the fused step updates r_s, the scalars and the
+    // step's alpha (x_s += a p_s pending)
+    TRY(L::cg_step(h, mass, ps, rs, h->dalpha + slot, h->hring + 4 * (itr % NEV)));
     HIPCHK(hipEventRecord(ev.e[itr % NEV], h->st));
     xf.p[xf.cnt] = (const typename PS::C*)ps.d;
     xf.sc[xf.cnt] = ps.sc;
@@ -1252,7 +1257,7 @@ int time_mdagm(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, int re
     rec(b + 4);
     if (!st) {
       hipLaunchKernelGGL(dwfk::k_reduce_partials, dim3(1), dim3(1024), 0, h->st, h->partial,
-                         O::grid(h), h->dscal);
+                         O::grid(h), h->dscal, (double*)nullptr);
       if (hipGetLastError() != hipSuccess) st = DWFGPU_HIP_ERROR;
     }
   }
@@ -2479,16 +2484,13 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
                        k == 0 ? 1 : 0, n, h->partial);
     HIPCHK(hipGetLastError());
     TRY(reduce_to(h, BLAS_BLOCKS, MS_PP));
-    TRY(H::matpc(h, mass, t1, vp0, 0, true));
-    TRY(reduce_to(h, H::grid(h), MS_MP));
-    TRY(H::matpc(h, mass, vap, t1, 1, false));
+    TRY(H::matpc(h, mass, t1, vp0, 0, h->dscal + MS_MP));
+    TRY(H::matpc(h, mass, vap, t1, 1));
     hipLaunchKernelGGL(k_ms_r, blas_grid(), blas_block(), 0, h->st, res(k + 1), res(k), ap, p0,
                        sigma, h->dscal, n, h->partial);
     hipLaunchKernelGGL(k_ms_reduce, dim3(1), dim3(1024), 0, h->st, h->partial, (int)BLAS_BLOCKS,
-                       sigma, h->dscal);
+                       sigma, h->dscal, h->hring + 8 * (k % NEV));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(h->hring + 8 * (k % NEV), h->dscal, 5 * sizeof(double),
-                          hipMemcpyDeviceToHost, h->st));
     HIPCHK(hipEventRecord(w.ev[k % NEV], h->st));
     return DWFGPU_OK;
   };
@@ -2577,7 +2579,7 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
     const int j = k - LAG;
     HIPCHK(hipEventSynchronize(w.ev[j % NEV]));
     const double* hs = h->hring + 8 * (j % NEV);
-    follow(j, hs[MS_C], hs[MS_D]);
+    follow(j, hs[0], hs[1]);
     done = j;
     if (convp || j + 1 > max_num_iter) break;
     entry(j + 1, true);
@@ -3571,7 +3573,7 @@ int dwfgpu_matpc(dwfgpu_t h, double mass, double* out, const double* in, int dag
   if (!h || !out || !in || (dag != 0 && dag != 1)) return DWFGPU_BAD_ARG;
   TRY(ensure_api(h, 2));
   TRY(DISPATCH(h, to_device(h, api_work(h, 0), in)));
-  TRY(DISPATCH(h, matpc(h, mass, api_work(h, 1), api_work(h, 0), dag, false)));
+  TRY(DISPATCH(h, matpc(h, mass, api_work(h, 1), api_work(h, 0), dag)));
   return DISPATCH(h, to_host(h, out, api_work(h, 1)));
 }
 
@@ -4465,7 +4467,7 @@ int dwfgpu_plaquette(dwfgpu_t h, double* plaq, double* link_trace) {
   HIPCHK(hipGetLastError());
   TRY(reduce_to(h, nb, 0));
   hipLaunchKernelGGL(dwfk::k_reduce_partials, dim3(1), dim3(1024), 0, h->st, h->partial + nb, nb,
-                     h->dscal + 1);
+                     h->dscal + 1, (double*)nullptr);
   HIPCHK(hipGetLastError());
   double sc[2];
   TRY(fetch_scalars(h, 2, sc));

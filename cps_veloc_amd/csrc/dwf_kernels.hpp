@@ -1897,9 +1897,12 @@ k_bw_probe(u32x4_t* __restrict__ d, const u32x4_t* __restrict__ a,
 }
 
 // deterministic final sum of per-block partials (one work-group of 1024
-// threads, four independent accumulators per thread, fixed order)
+// threads, four independent accumulators per thread, fixed order).  host:
+// pinned memory that also receives the sum, or null; a copy of 8 bytes after
+// the kernel would be a launch of its own (2.7 us and a gap)
 __global__ void __launch_bounds__(1024)
-k_reduce_partials(const double* __restrict__ partial, int n, double* __restrict__ out) {
+k_reduce_partials(const double* __restrict__ partial, int n, double* __restrict__ out,
+                  double* __restrict__ host) {
   __shared__ double sh[16];
   double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
   int k = threadIdx.x;
@@ -1911,16 +1914,21 @@ k_reduce_partials(const double* __restrict__ partial, int n, double* __restrict_
   }
   for (; k < n; k += 1024) a0 += partial[k];
   const double t = block_sum((a0 + a1) + (a2 + a3), sh);
-  if (threadIdx.x == 0) out[0] = t;
+  if (threadIdx.x == 0) {
+    out[0] = t;
+    if (host) host[0] = t;
+  }
 }
 
-// End of one step of the sloppy CG: |r|^2 of the partials into scal[0],
-// its previous value into scal[2] (for beta), and the step's alpha =
-// |r|^2 / <p, A p> (the value cg_alpha gave the epilogue) into *alpha_out,
-// all on the device so that the host need not wait for the step.
+// End of one CG step: |r|^2 of the partials into scal[0], its previous value
+// into scal[2] (for beta), and the step's alpha = |r|^2 / <p, A p> (the value
+// cg_alpha gave the epilogue) into *alpha_out, all on the device so that the
+// host need not wait for the step; host (pinned) receives |r|^2 and <p, A p>.
+// (The pass's last work-group doing this cost 2.5-3 us on an 8^4 lattice, as
+// much as this kernel.)
 __global__ void __launch_bounds__(1024)
 k_reduce_cg_step(const double* __restrict__ partial, int n, double* __restrict__ scal,
-                 double* __restrict__ alpha_out) {
+                 double* __restrict__ alpha_out, double* __restrict__ host) {
   __shared__ double sh[16];
   double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
   int k = threadIdx.x;
@@ -1937,6 +1945,8 @@ k_reduce_cg_step(const double* __restrict__ partial, int n, double* __restrict__
     *alpha_out = cg_alpha(scal);
     scal[2] = rr;
     scal[0] = t;
+    host[0] = t;
+    host[1] = scal[1];
   }
 }
 
@@ -2195,9 +2205,9 @@ k_ms_flush(MsFlush a, const MsStep* __restrict__ st) {
   }
 }
 
-// Scalars of the step on the device: |r|^2, |MatPc p0|^2, |p0|^2, the previous
-// |r|^2 and d = <p0, (A + sigma) p0>.
-enum { MS_C = 0, MS_MP = 1, MS_PP = 2, MS_CP = 3, MS_D = 4 };
+// Scalars of the step on the device: |r|^2, |MatPc p0|^2, |p0|^2 and the
+// previous |r|^2; d = <p0, (A + sigma) p0> = |MatPc p0|^2 + sigma |p0|^2.
+enum { MS_C = 0, MS_MP = 1, MS_PP = 2, MS_CP = 3 };
 
 // ro = r + b (ap + sigma p), b = -|r|^2 / d; |ro|^2 partials
 __global__ void __launch_bounds__(BLAS_THREADS)
@@ -2237,15 +2247,18 @@ k_ms_p(cx<double>* __restrict__ p, const cx<double>* __restrict__ r,
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// the end of a step: |r|^2 of the partials becomes the current one
+// the end of a step: |r|^2 of the partials becomes the current one; host
+// (pinned) receives it and d
 __global__ void __launch_bounds__(1024)
-k_ms_reduce(const double* __restrict__ partial, int n, double sigma, double* __restrict__ scal) {
+k_ms_reduce(const double* __restrict__ partial, int n, double sigma, double* __restrict__ scal,
+            double* __restrict__ host) {
   __shared__ double sh[16];
   double a0 = 0.0;
   for (int k = threadIdx.x; k < n; k += 1024) a0 += partial[k];
   const double t = block_sum(a0, sh);
   if (threadIdx.x == 0) {
-    scal[MS_D] = scal[MS_MP] + sigma * scal[MS_PP];
+    host[1] = scal[MS_MP] + sigma * scal[MS_PP];
+    host[0] = t;
     scal[MS_CP] = scal[MS_C];
     scal[MS_C] = t;
   }
