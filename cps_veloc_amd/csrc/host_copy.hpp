@@ -17,7 +17,6 @@
 #include <memory>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -60,10 +59,11 @@ inline void release() {
   }
 }
 
+// (to the device: in order on st, whose work the callers wait for before they
+// return to their own)
 inline hipError_t direct(void* dev, void* host, size_t bytes, bool to_host, hipStream_t st) {
-  const hipError_t e =
-      to_host ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st)
-              : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+  if (!to_host) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+  const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
   return e != hipSuccess ? e : hipStreamSynchronize(st);
 }
 
@@ -76,7 +76,7 @@ inline bool pinned(const void* host) {
   return false;
 }
 
-// dev <-> host, after the work queued on st; complete on return
+// dev <-> host, after the work queued on st; to the host complete on return
 inline hipError_t copy(void* dev, void* host, size_t bytes, bool to_host, hipStream_t st) {
   if (bytes < (to_host ? MIN_TO_HOST : MIN_TO_DEVICE) || pinned(host))
     return direct(dev, host, bytes, to_host, st);
@@ -128,7 +128,7 @@ inline hipError_t copy(void* dev, void* host, size_t bytes, bool to_host, hipStr
   int started = 0;
   try {
     for (; started < WORKERS; ++started) pool[started] = std::thread(worker);
-  } catch (const std::system_error&) {  // fewer threads than asked for
+  } catch (...) {  // fewer threads than asked for
   }
   hipError_t err = hipSuccess;
   if (started == 0) {
