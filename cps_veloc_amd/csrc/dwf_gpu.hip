@@ -233,7 +233,6 @@ M5Side m5_side(const dwfgpu_s* h, double mass, int dag) {
 
 MobArgs mob_args(const dwfgpu_s* h, double mass, int dag) {
   MobArgs a;
-  a.active = nullptr;
   const double kb = mob_kappa_b(h), kc = mob_kappa_c(h);
   a.b = h->b;
   a.c = h->c;
@@ -522,14 +521,26 @@ struct Ops {
     return DWFGPU_OK;
   }
 
+  // LDS of a Mobius pass, and whether it takes the exchange gather
+  static size_t mob_lds(const dwfgpu_s* h, int dag, int epi, int fl, bool* split) {
+    const bool col = dag || epi == dwfk::EPI_M5INV || epi == dwfk::EPI_SCHUR;
+    const size_t cols = col ? col_lds_bytes(h, sizeof(R)) : 0;
+    // exchange slots after the links; the M5^-1 / Schur s-columns reuse the
+    // LDS from offset 0 once the hop is done
+    const size_t split_lds =
+        std::max(cols, dwfk::split_col_offset<R>(h->ns) +
+                           (size_t)h->ls * h->ns * dwfk::TX_SLOT * 2 * sizeof(R));
+    *split = dwfk::MobSplitT<P>::value && !dag && !(fl & dwfk::FL_PRE_T) &&
+             split_lds <= (size_t)h->max_lds;
+    return *split ? split_lds : std::max(link_lds_bytes(h, 1, sizeof(R)), cols);
+  }
+
   // Mobius hop kernel; fl: dwfk::FL_* flags
   static int mob(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, const DVec& psi,
-                 int p_out, int dag, int epi, int fl, double* partial = nullptr,
-                 const int* active = nullptr) {
+                 int p_out, int dag, int epi, int fl, double* partial = nullptr) {
     if (!partial) partial = h->partial;
     const dim3 grid(h->grid_hop), block(h->ns, h->ls);
-    MobArgs a = mob_args(h, mass, dag);
-    a.active = active;
+    const MobArgs a = mob_args(h, mass, dag);
     // the Schur passes sweep backwards: they start on the sites the pass
     // before them wrote last, which the last-level cache still holds
     Geom gm = h->g;
@@ -539,18 +550,8 @@ struct Ops {
       if (h->ns64)
         return mob64(h, gm, a, (cx<double>*)out.d, (const cx<double>*)in.d,
                      (const cx<double>*)psi.d, p_out, dag, epi, fl, partial, nullptr, nullptr);
-    const bool col = dag || epi == dwfk::EPI_M5INV || epi == dwfk::EPI_SCHUR;
-    // exchange slots after the links; the M5^-1 / Schur s-columns reuse the
-    // LDS from offset 0 once the hop is done
-    const size_t split_lds =
-        std::max(col ? col_lds_bytes(h, sizeof(R)) : (size_t)0,
-                 dwfk::split_col_offset<R>(h->ns) +
-                     (size_t)h->ls * h->ns * dwfk::TX_SLOT * 2 * sizeof(R));
-    const bool split = dwfk::MobSplitT<P>::value && !dag && !(fl & dwfk::FL_PRE_T) &&
-                       split_lds <= (size_t)h->max_lds;
-    const size_t lds = split ? split_lds
-                             : std::max(link_lds_bytes(h, 1, sizeof(R)),
-                                        col ? col_lds_bytes(h, sizeof(R)) : (size_t)0);
+    bool split;
+    const size_t lds = mob_lds(h, dag, epi, fl, &split);
 #define MOB_LAUNCH(DAG, EPI, FL)                                                              \
   hipLaunchKernelGGL((dwfk::k_mobius<P, DAG, EPI, FL>), grid, block, lds, h->st, fld<P>(out), \
                      cfld<P>(in), cfld<P>(psi), u, partial, gm, p_out, a, dwfk::CgEpi<P, P>{})
@@ -594,16 +595,13 @@ struct Ops {
 
   // first / second half of MatPc (dag 0) or MatPcDag (dag 1): the first writes
   // te (for dag 0 already multiplied by (b + c D5), consumed by the second)
-  static int mob_first(dwfgpu_s* h, double mass, const DVec& te, const DVec& in, int dag,
-                       const int* active = nullptr) {
-    return mob(h, mass, te, in, DVec(), 0, dag, dwfk::EPI_M5INV, dag ? 0 : dwfk::FL_POST_T,
-               nullptr, active);
+  static int mob_first(dwfgpu_s* h, double mass, const DVec& te, const DVec& in, int dag) {
+    return mob(h, mass, te, in, DVec(), 0, dag, dwfk::EPI_M5INV, dag ? 0 : dwfk::FL_POST_T);
   }
   static int mob_second(dwfgpu_s* h, double mass, const DVec& out, const DVec& te,
-                        const DVec& in, int dag, bool norm, double* partial = nullptr,
-                        const int* active = nullptr) {
+                        const DVec& in, int dag, bool norm, double* partial = nullptr) {
     const int fl = (dag ? 0 : dwfk::FL_PRE_T) | (norm && !dag ? dwfk::FL_NORM : 0);
-    return mob(h, mass, out, te, in, 1, dag, dwfk::EPI_SCHUR, fl, partial, active);
+    return mob(h, mass, out, te, in, 1, dag, dwfk::EPI_SCHUR, fl, partial);
   }
   // the last pass of a Mobius CG step: dagger hop of te, (b + c D5^dag) and
   // the Schur term with t1, then r -= alpha A p and |r|^2 partials (and
@@ -611,9 +609,8 @@ struct Ops {
   template <class PX>
   static int mob_cg_last(dwfgpu_s* h, double mass, const DVec& te, const DVec& t1,
                          const DVec& r, const DVec& p, const DVec& x, const double* scal,
-                         double* partial, const int* active) {
-    MobArgs a = mob_args(h, mass, 1);
-    a.active = active;
+                         double* partial) {
+    const MobArgs a = mob_args(h, mass, 1);
     Geom gm = h->g;
     gm.rev = 1;  // a Schur pass: backwards, as in mob()
     if constexpr (std::is_same<P, P64>::value && std::is_same<PX, dwfk::NoX>::value) {
@@ -720,7 +717,7 @@ struct Ops {
                          2.0 * h->a5inv, -2.0 * mass * h->a5inv, mk2, cg);
     } else {
       TRY(mob_first(h, mass, te, t1, 1));
-      TRY(mob_cg_last<PX>(h, mass, te, t1, r, p, x, h->dscal, h->partial, nullptr));
+      TRY(mob_cg_last<PX>(h, mass, te, t1, r, p, x, h->dscal, h->partial));
     }
     HIPCHK(hipGetLastError());
     return DWFGPU_OK;
@@ -1914,6 +1911,7 @@ struct MrState {
   double* partial = nullptr;
   double* scal = nullptr;
   double* mass = nullptr;
+  MobArgs* mob = nullptr;  // Mobius: of each RHS for dag 0, then for dag 1
   int* ibuf = nullptr;  // active | flag | iters
   int gx = 0;
   ~MrState() {
@@ -1922,7 +1920,7 @@ struct MrState {
     free_vec(&rs);
     free_vec(&ps);
     free_vec(&xs);
-    void* p[] = {partial, scal, mass, ibuf};
+    void* p[] = {partial, scal, mass, mob, ibuf};
     for (void* q : p)
       if (q) (void)hipFree(q);
   }
@@ -2039,47 +2037,62 @@ int mr_mdagm(dwfgpu_s* h, const MrShape& t, int nrhs, const DVec& out, const DVe
   return DWFGPU_OK;
 }
 
-// batched Mobius MatPcDagMatPc: the four hop passes of each RHS with its own
-// mass, launched per RHS (the M5^-1 and (b + c D5) epilogues keep every s-
-// column of a site in one work-group's LDS, so RHS share a launch shape but
-// not a work-group).  A paused RHS (active[j] == 0) costs four launches whose
-// work-groups leave at once.  Partials: grid_hop per RHS, RHS j at j*grid_hop.
-// cg: the CG step of every active RHS (r -= alpha A p, x += alpha p in the
-// last pass, alpha and |r|^2 on the device) instead of `out`.
+// the coefficients of every RHS of a batched Mobius operator, on the device
 template <class P>
-int mr_mdagm_mob(dwfgpu_s* h, int nrhs, const DVec& out, const DVec& in, const DVec& te,
-                 const DVec& t1, const double* masses, const int* active, double* partial,
-                 double* scal, const DVec* r, const DVec* x, bool cg) {
+int mr_mob_args(dwfgpu_s* h, const double* masses, MrState<P>& m) {
+  std::vector<MobArgs> a;
+  for (int dag = 0; dag < 2; ++dag)
+    for (int j = 0; j < m.nrhs; ++j) a.push_back(mob_args(h, masses[j], dag));
+  TRY(alloc(h, (void**)&m.mob, a.size() * sizeof(MobArgs)));
+  HIPCHK(hipMemcpyAsync(m.mob, a.data(), a.size() * sizeof(MobArgs), hipMemcpyHostToDevice,
+                        h->st));
+  HIPCHK(hipStreamSynchronize(h->st));
+  return DWFGPU_OK;
+}
+
+// batched Mobius MatPcDagMatPc: the four hop passes, each one launch for all
+// RHS (k_mobius_mrhs; the M5^-1 and (b + c D5) epilogues keep every s-column
+// of a site in one work-group's LDS, so RHS share a launch but not a
+// work-group).  cg: the CG step of every active RHS (r -= alpha A p,
+// x += alpha p in the last pass, alpha and |r|^2 on the device) instead of
+// `out`.  12^4 Ls 12, 4 RHS, int16: the passes of a step 198 -> 124 us against a launch per
+// RHS and pass, a batched MatInv 61 -> 48.5 ms.
+template <class P>
+int mr_mdagm_mob(dwfgpu_s* h, const MrState<P>& m, const DVec& out, const DVec& in, double* scal,
+                 bool cg) {
   typedef Ops<P> O;
-  const int gx = O::grid(h);
-  for (int j = 0; j < nrhs; ++j) {
-    const DVec inj = mslice<P>(h, in, j), tej = mslice<P>(h, te, j), t1j = mslice<P>(h, t1, j);
-    TRY(O::mob_first(h, masses[j], tej, inj, 0, active + j));
-    TRY(O::mob_second(h, masses[j], t1j, tej, inj, 0, scal != nullptr, partial + (size_t)j * gx,
-                      active + j));
+  using namespace dwfk;
+  const int nrhs = m.nrhs, gx = h->grid_hop;
+  const dim3 grid(gx, nrhs), block(h->ns, h->ls);
+  const size_t vs = h->n / 2 / P::kCPC;
+  const typename P::S* u = (const typename P::S*)h->f[pidx<P>()].U;
+  Geom fwd = h->g, back = h->g;
+  back.rev = 1;  // the Schur passes, as in Ops::mob()
+  bool split;
+#define MOB_MR(DAG, EPI, FL, PX, OUT, IN, PSI, GEOM, CG)                                            hipLaunchKernelGGL((k_mobius_mrhs<P, DAG, EPI, FL, PX>), grid, block,                                                O::mob_lds(h, DAG, EPI, FL, &split), h->st, fld<P>(OUT), cfld<P>(IN),                             cfld<P>(PSI), u, m.partial, GEOM, EPI == EPI_SCHUR ? 1 : 0,                                       m.mob + DAG * nrhs, m.active(), vs, CG, MR_NSCAL)
+  const CgEpi<P, P> none{};
+  O::mob_lds(h, 0, EPI_M5INV, FL_POST_T, &split);
+  if (split) {
+    if constexpr (MobSplitT<P>::value)
+      MOB_MR(0, EPI_M5INV, FL_POST_T | FL_SPLIT_T, P, m.te, in, DVec(), fwd, none);
+  } else {
+    MOB_MR(0, EPI_M5INV, FL_POST_T, P, m.te, in, DVec(), fwd, none);
   }
-  if (scal) {
-    hipLaunchKernelGGL(dwfk::k_reduce_mrhs, dim3(nrhs), dim3(1024), 0, h->st, partial, gx, scal,
-                       (int)dwfk::MR_D, active);
-    HIPCHK(hipGetLastError());
-  }
-  for (int j = 0; j < nrhs; ++j) {
-    const DVec tej = mslice<P>(h, te, j), t1j = mslice<P>(h, t1, j);
-    TRY(O::mob_first(h, masses[j], tej, t1j, 1, active + j));
-    if (cg)
-      TRY(O::template mob_cg_last<P32>(h, masses[j], tej, t1j, mslice<P>(h, *r, j),
-                                       mslice<P>(h, in, j), mslice<P32>(h, *x, j),
-                                       scal + (size_t)j * dwfk::MR_NSCAL,
-                                       partial + (size_t)j * gx, active + j));
-    else
-      TRY(O::mob_second(h, masses[j], mslice<P>(h, out, j), tej, t1j, 1, false, nullptr,
-                        active + j));
-  }
+  MOB_MR(0, EPI_SCHUR, FL_PRE_T | FL_NORM, P, m.t1, m.te, in, back, none);
+  if (scal)
+    hipLaunchKernelGGL(k_reduce_mrhs, dim3(nrhs), dim3(1024), 0, h->st, m.partial, gx, scal,
+                       (int)MR_D, m.active());
+  MOB_MR(1, EPI_M5INV, 0, P, m.te, m.t1, DVec(), fwd, none);
   if (cg) {
-    hipLaunchKernelGGL(dwfk::k_reduce_mrhs, dim3(nrhs), dim3(1024), 0, h->st, partial, gx, scal,
-                       (int)dwfk::MR_RRNEW, active);
-    HIPCHK(hipGetLastError());
+    const CgEpi<P, P32> step{fld<P>(m.rs), cfld<P>(in), fld<P32>(m.xs), scal};
+    MOB_MR(1, EPI_SCHUR, FL_CG, P32, m.te, m.te, m.t1, back, step);
+    hipLaunchKernelGGL(k_reduce_mrhs, dim3(nrhs), dim3(1024), 0, h->st, m.partial, gx, scal,
+                       (int)MR_RRNEW, m.active());
+  } else {
+    MOB_MR(1, EPI_SCHUR, 0, P, out, m.te, m.t1, back, none);
   }
+#undef MOB_MR
+  HIPCHK(hipGetLastError());
   return DWFGPU_OK;
 }
 
@@ -2213,7 +2226,10 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
     HIPCHK(hipMemcpyAsync(m.ibuf, ones.data(), nrhs * sizeof(int), hipMemcpyHostToDevice, h->st));
   }
   MrShape t{h->ns, 1};  // Mobius: the handle's own hop shape, one RHS per work-group
-  if (h->action == DWFGPU_DWF) TRY(mr_tune<PS>(h, nrhs, m, m.active(), &t));
+  if (h->action == DWFGPU_DWF)
+    TRY(mr_tune<PS>(h, nrhs, m, m.active(), &t));
+  else
+    TRY(mr_mob_args<PS>(h, masses, m));
   h->mr_last_ns = t.ns;
   h->mr_last_nr = t.nr;
 
@@ -2257,8 +2273,7 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
       TRY(mr_mdagm<PS>(h, t, nrhs, DVec(), m.ps, m.te, m.t1, m.mass, m.active(), m.partial,
                        m.scal, &m.rs, &m.xs, true));
     else
-      TRY(mr_mdagm_mob<PS>(h, nrhs, DVec(), m.ps, m.te, m.t1, masses, m.active(), m.partial,
-                           m.scal, &m.rs, &m.xs, true));
+      TRY(mr_mdagm_mob<PS>(h, m, DVec(), m.ps, m.scal, true));
     hipLaunchKernelGGL(dwfk::k_cg_scalars_mrhs, dim3(1), dim3(256), 0, h->st, m.scal, m.active(),
                        m.flag(), m.iters(), nrhs);
     HIPCHK(hipGetLastError());
@@ -4030,9 +4045,12 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
       TRY(mr_tune<P>(h, nrhs, m, m.active(), &t));
       TRY(mr_mdagm<P>(h, t, nrhs, m.rs, m.ps, m.te, m.t1, m.mass, m.active(), m.partial,
                       nullptr, nullptr, nullptr, false));
+    } else if (pidx<P>() == DWFGPU_F64 && h->ns64) {  // as a single right-hand side
+      for (int j = 0; j < nrhs; ++j)
+        TRY(Ops<P>::mdagm(h, masses[j], mslice<P>(h, m.rs, j), mslice<P>(h, m.ps, j), nullptr));
     } else {
-      TRY(mr_mdagm_mob<P>(h, nrhs, m.rs, m.ps, m.te, m.t1, masses, m.active(), m.partial,
-                          nullptr, nullptr, nullptr, false));
+      TRY(mr_mob_args<P>(h, masses, m));
+      TRY(mr_mdagm_mob<P>(h, m, m.rs, m.ps, nullptr, false));
     }
     h->mr_last_ns = t.ns;
     h->mr_last_nr = t.nr;

@@ -1218,9 +1218,6 @@ struct MobArgs {
   double kappa_b;
   float fb, fc, fmc, fK, fmK, fkappa_b;
   M5Side m5;
-  // batched solves: the active flag of this launch's right-hand side
-  // (nullptr: always run); a paused one's work-groups leave at once
-  const int* active;
 };
 
 // the coefficient in the compute type R
@@ -1368,11 +1365,12 @@ __host__ __device__ constexpr size_t split_col_offset(int ns) {
 }
 
 template <class P, int DAG, int EPI, int FL, class PX = P>
-__global__ void __launch_bounds__(512)
-k_mobius(Fld<P> out, CFld<P> in, CFld<P> psi, const typename P::S* __restrict__ U,
-         double* __restrict__ partial, Geom g, int p_out, MobArgs a, CgEpi<P, PX> cg) {
+__device__ __forceinline__ void mobius_pass(Fld<P> out, CFld<P> in, CFld<P> psi,
+                                            const typename P::S* __restrict__ U,
+                                            double* __restrict__ partial, const Geom& g,
+                                            int p_out, const MobArgs& a,
+                                            const CgEpi<P, PX>& cg) {
   typedef typename P::R R;
-  if (a.active && *a.active == 0) return;  // uniform: before any barrier
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double sh[16];
   const int ns = blockDim.x, il = threadIdx.x, s = threadIdx.y;
@@ -1530,6 +1528,49 @@ k_mobius(Fld<P> out, CFld<P> in, CFld<P> psi, const typename P::S* __restrict__ 
     }
     st_site<P>(od, osc, g.vh, i, v);
   }
+}
+
+template <class P, int DAG, int EPI, int FL, class PX = P>
+__global__ void __launch_bounds__(512)
+k_mobius(Fld<P> out, CFld<P> in, CFld<P> psi, const typename P::S* __restrict__ U,
+         double* __restrict__ partial, Geom g, int p_out, MobArgs a, CgEpi<P, PX> cg) {
+  mobius_pass<P, DAG, EPI, FL, PX>(out, in, psi, U, partial, g, p_out, a, cg);
+}
+
+template <class P>
+__device__ __forceinline__ Fld<P> fld_at(Fld<P> f, size_t vs, size_t vss, int j) {
+  return Fld<P>{f.d + j * vs, f.sc ? f.sc + j * vss : nullptr};
+}
+template <class P>
+__device__ __forceinline__ CFld<P> fld_at(CFld<P> f, size_t vs, size_t vss, int j) {
+  return CFld<P>{f.d + j * vs, f.sc ? f.sc + j * vss : nullptr};
+}
+
+// one pass of a batch: right-hand side j = blockIdx.y has its own mass, and so
+// its own args[j], its fields j vectors of vs chunks after the first one's,
+// its partials at partial[j * gridDim.x].  A paused one's (active[j] == 0)
+// work-groups leave at once.  One launch for all of them because a pass of one
+// 12^4 Ls 12 vector is 648 work-groups, less than the chip holds at once:
+// launched one after the other, each waited for the last work-groups of the
+// one before.
+template <class P, int DAG, int EPI, int FL, class PX = P>
+__global__ void __launch_bounds__(512)
+k_mobius_mrhs(Fld<P> out, CFld<P> in, CFld<P> psi, const typename P::S* __restrict__ U,
+              double* __restrict__ partial, Geom g, int p_out, const MobArgs* __restrict__ args,
+              const int* __restrict__ active, size_t vs, CgEpi<P, PX> cg, int cg_stride) {
+  const int j = blockIdx.y;
+  if (!active[j]) return;  // uniform: before any barrier
+  const size_t vss = (size_t)g.vh * g.ls;
+  if constexpr ((FL & FL_CG) != 0) {
+    cg.r = fld_at(cg.r, vs, vss, j);
+    cg.p = fld_at(cg.p, vs, vss, j);
+    if constexpr (!std::is_same<PX, NoX>::value)
+      cg.x = fld_at(cg.x, vs * nch<PX>() / nch<P>(), vss, j);
+    cg.scal += (size_t)j * cg_stride;
+  }
+  mobius_pass<P, DAG, EPI, FL, PX>(fld_at(out, vs, vss, j), fld_at(in, vs, vss, j),
+                                   fld_at(psi, vs, vss, j), U,
+                                   partial + (size_t)j * gridDim.x, g, p_out, args[j], cg);
 }
 
 // stand-alone M5^-1 (dag) on a half vector: zmobius_m5inv(out, in, ...)
@@ -2296,15 +2337,6 @@ struct MrArgs {
   Fld<PX> x;
   double* scal;  // [nrhs][MR_NSCAL]
 };
-
-template <class P>
-__device__ __forceinline__ Fld<P> fld_at(Fld<P> f, size_t vs, size_t vss, int j) {
-  return Fld<P>{f.d + j * vs, f.sc ? f.sc + j * vss : nullptr};
-}
-template <class P>
-__device__ __forceinline__ CFld<P> fld_at(CFld<P> f, size_t vs, size_t vss, int j) {
-  return CFld<P>{f.d + j * vs, f.sc ? f.sc + j * vss : nullptr};
-}
 
 // per-RHS (threadIdx.z) sum over a work-group, fixed order; valid in the
 // thread with threadIdx.x == threadIdx.y == 0 of each z

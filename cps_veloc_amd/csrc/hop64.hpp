@@ -284,7 +284,6 @@ __global__ void __launch_bounds__(512)
 k_mobius64(c64* __restrict__ out, const c64* __restrict__ in, const c64* __restrict__ psi,
            const c64* __restrict__ U, double* __restrict__ partial, Geom g, int p_out, MobArgs a,
            c64* __restrict__ r, const double* __restrict__ scal) {
-  if (a.active && *a.active == 0) return;  // uniform: before any barrier
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double sh[16];
   const int ns = blockDim.x >> 1, s = threadIdx.y, ls = g.ls;
