@@ -1343,8 +1343,10 @@ const DVec& api_work(dwfgpu_s* h, int k) { return h->f[h->prec].work[k]; }
 // ===========================================================================
 struct PtcNet {
   int ls = 0, hid = 16;
-  std::vector<std::complex<float>> W[3];  // [9][cout][cin][4][4]
-  std::vector<double> m[3], v[3];         // Adam moments of (re, im)
+  // the three layers' weights [9][cout][cin][4][4] one after the other, the
+  // gradients G likewise, and the Adam moments of (re, im)
+  cx<float>*W = nullptr, *G = nullptr;
+  double2 *m = nullptr, *v = nullptr;
   long adam_t = 0;
   uint16_t* A[3] = {nullptr, nullptr, nullptr};     // bf16 real forms, [9][M'][K']
   uint16_t* Aadj[3] = {nullptr, nullptr, nullptr};  // of the adjoint layers
@@ -1352,93 +1354,56 @@ struct PtcNet {
   uint32_t* gact[2] = {nullptr, nullptr};
   float* gwpart = nullptr;
   int nwg[3] = {0, 0, 0};  // work-groups per direction of each layer's weight gradient
-  cx<float>* G[3] = {nullptr, nullptr, nullptr};
   int cin(int k) const { return k == 0 ? ls : hid; }
   int cout(int k) const { return k == 2 ? ls : hid; }
   size_t nw(int k) const { return (size_t)ptck::NDIR * cout(k) * cin(k) * 16; }
+  size_t first(int k) const {  // of layer k in W, G, m and v; k = 3: their length
+    size_t q = 0;
+    for (int j = 0; j < k; ++j) q += nw(j);
+    return q;
+  }
 };
 
 namespace {
 
 void ptc_free(PtcNet* n) {
   if (!n) return;
+  for (void* p : {(void*)n->W, (void*)n->G, (void*)n->m, (void*)n->v, (void*)n->gwpart})
+    if (p) (void)hipFree(p);
   for (int k = 0; k < 3; ++k) {
     if (n->A[k]) (void)hipFree(n->A[k]);
     if (n->Aadj[k]) (void)hipFree(n->Aadj[k]);
-    if (n->G[k]) (void)hipFree(n->G[k]);
   }
   for (auto p : n->act)
     if (p) (void)hipFree(p);
   for (auto p : n->gact)
     if (p) (void)hipFree(p);
-  if (n->gwpart) (void)hipFree(n->gwpart);
   delete n;
 }
 
-uint16_t bf16_host(float x) {
-  uint32_t u;
-  std::memcpy(&u, &x, 4);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-
-// A_d = [[Re W_d, -Im W_d], [Im W_d, Re W_d]] (rows (part, o, a), columns
-// (part, i, b)) for every d, from W[d][o][i][a][b]; adj: the real form of
-// the adjoint layer, W'_{d'}[i][o][b][a] = conj(W_d[o][i][a][b]), d' = -d
-void ptc_real_form(const std::vector<std::complex<float>>& W, int cin, int cout, bool adj,
-                   std::vector<uint16_t>& out) {
-  const int ci = adj ? cout : cin, co = adj ? cin : cout;
-  const int MP = 8 * co, KP = 8 * ci;
-  out.assign((size_t)ptck::NDIR * MP * KP, 0);
-  for (int d = 0; d < ptck::NDIR; ++d) {
-    const int ds = adj ? (d == 0 ? 0 : (d <= 4 ? d + 4 : d - 4)) : d;  // source direction
-    for (int o = 0; o < co; ++o)
-      for (int i = 0; i < ci; ++i)
-        for (int a = 0; a < 4; ++a)
-          for (int b = 0; b < 4; ++b) {
-            std::complex<float> w;
-            if (!adj)
-              w = W[(((size_t)(ds * cout + o) * cin + i) * 4 + a) * 4 + b];
-            else  // W'[o'=i][i'=o][a'=b][b'=a] = conj(W[o][i][a][b])
-              w = std::conj(W[(((size_t)(ds * cout + i) * cin + o) * 4 + b) * 4 + a]);
-            const int mre = o * 4 + a, mim = co * 4 + o * 4 + a;
-            const int kre = i * 4 + b, kim = ci * 4 + i * 4 + b;
-            uint16_t* Ad = out.data() + (size_t)d * MP * KP;
-            Ad[mre * KP + kre] = bf16_host(w.real());
-            Ad[mre * KP + kim] = bf16_host(-w.imag());
-            Ad[mim * KP + kre] = bf16_host(w.imag());
-            Ad[mim * KP + kim] = bf16_host(w.real());
-          }
-  }
-}
-
-// [9][M'][K'] row-major -> the MFMA fragment order of k_ptc_fwd: 8 bf16
-// A[d][16*blk + l%16][32*kb + 8*(l/16) + e] at (((d*MB + blk)*K32 + kb)*64 + l)*8 + e
-void ptc_fragment_order(std::vector<uint16_t>& buf, int mp, int kp) {
-  const int mb = mp / 16, k32 = kp / 32;
-  std::vector<uint16_t> rm(buf);
-  for (int d = 0; d < ptck::NDIR; ++d)
-    for (int blk = 0; blk < mb; ++blk)
-      for (int kb = 0; kb < k32; ++kb)
-        for (int l = 0; l < 64; ++l)
-          for (int e = 0; e < 8; ++e)
-            buf[((((size_t)d * mb + blk) * k32 + kb) * 64 + l) * 8 + e] =
-                rm[(size_t)d * mp * kp + (size_t)(16 * blk + l % 16) * kp + 32 * kb + 8 * (l / 16) + e];
-}
-
-int ptc_upload(dwfgpu_s* h) {
-  PtcNet* n = h->net;
-  std::vector<uint16_t> buf;
+// an Adam step (count 0: none), and the layers' bf16 real forms from the weights
+int ptc_weights(dwfgpu_s* h, const ptck::AdamStep& step) {
+  const PtcNet* n = h->net;
+  ptck::NetWeights net;
+  size_t most = 0;
   for (int k = 0; k < 3; ++k) {
-    ptc_real_form(n->W[k], n->cin(k), n->cout(k), false, buf);
-    ptc_fragment_order(buf, 8 * n->cout(k), 8 * n->cin(k));
-    HIPCHK(hipMemcpyAsync(n->A[k], buf.data(), buf.size() * 2, hipMemcpyHostToDevice, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
-    ptc_real_form(n->W[k], n->cin(k), n->cout(k), true, buf);
-    ptc_fragment_order(buf, 8 * n->cin(k), 8 * n->cout(k));
-    HIPCHK(hipMemcpyAsync(n->Aadj[k], buf.data(), buf.size() * 2, hipMemcpyHostToDevice, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
+    const size_t q = n->first(k);
+    net.l[k] = ptck::LayerWeights{n->W + q, n->G + q, n->m + q, n->v + q, n->A[k], n->Aadj[k],
+                                  n->cin(k), n->cout(k)};
+    most = std::max(most, n->nw(k));
   }
+  hipLaunchKernelGGL(ptck::k_ptc_weights, dim3((most + 255) / 256, 3), dim3(256), 0, h->st, net,
+                     step);
+  HIPCHK(hipGetLastError());
+  return DWFGPU_OK;
+}
+
+// the weights (re, im) from the host
+int ptc_upload(dwfgpu_s* h, const float* w) {
+  HIPCHK(hipMemcpyAsync(h->net->W, w, h->net->first(3) * sizeof(cx<float>), hipMemcpyHostToDevice,
+                        h->st));
+  TRY(ptc_weights(h, ptck::AdamStep{0, 0.0, 1.0, 1.0}));
+  HIPCHK(hipStreamSynchronize(h->st));
   return DWFGPU_OK;
 }
 
@@ -1568,8 +1533,8 @@ int ptc_grad_pair(dwfgpu_s* h, const DVec& r, const DVec& e, bool accumulate, do
   int cur = 0;
   for (int k = 2; k >= 0; --k) {
     TRY(ptc_gw(h, n->cin(k), n->cout(k), n->gwpart, n->nwg[k], n->gact[cur], n->act[k]));
-    hipLaunchKernelGGL(ptck::k_ptc_gw_reduce, dim3(128), dim3(256), 0, h->st, n->G[k], n->gwpart,
-                       n->nwg[k], n->cin(k), n->cout(k), accumulate ? 1 : 0);
+    hipLaunchKernelGGL(ptck::k_ptc_gw_reduce, dim3(128), dim3(256), 0, h->st, n->G + n->first(k),
+                       n->gwpart, n->nwg[k], n->cin(k), n->cout(k), accumulate ? 1 : 0);
     HIPCHK(hipGetLastError());
     if (k > 0) {
       TRY(ptc_fwd(h, n->cout(k), n->cin(k), n->gact[1 - cur], n->gact[cur], n->Aadj[k]));
@@ -1581,29 +1546,8 @@ int ptc_grad_pair(dwfgpu_s* h, const DVec& r, const DVec& e, bool accumulate, do
 
 // one Adam step with the gradients accumulated over `count` pairs
 int ptc_adam(dwfgpu_s* h, int count, double lr) {
-  PtcNet* n = h->net;
-  const double b1 = 0.9, b2 = 0.999, eps = 1e-8;
-  ++n->adam_t;
-  const double c1 = 1.0 - std::pow(b1, (double)n->adam_t), c2 = 1.0 - std::pow(b2, (double)n->adam_t);
-  for (int k = 0; k < 3; ++k) {
-    std::vector<std::complex<float>> G(n->nw(k));
-    HIPCHK(hipMemcpyAsync(G.data(), n->G[k], G.size() * sizeof(cx<float>), hipMemcpyDeviceToHost,
-                          h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
-    for (size_t q = 0; q < G.size(); ++q) {
-      const double g2[2] = {G[q].real() / count, G[q].imag() / count};
-      double w2[2] = {n->W[k][q].real(), n->W[k][q].imag()};
-      for (int c = 0; c < 2; ++c) {
-        double& m = n->m[k][2 * q + c];
-        double& v = n->v[k][2 * q + c];
-        m = b1 * m + (1.0 - b1) * g2[c];
-        v = b2 * v + (1.0 - b2) * g2[c] * g2[c];
-        w2[c] -= lr * (m / c1) / (std::sqrt(v / c2) + eps);
-      }
-      n->W[k][q] = std::complex<float>((float)w2[0], (float)w2[1]);
-    }
-  }
-  return ptc_upload(h);
+  const double t = (double)++h->net->adam_t;
+  return ptc_weights(h, ptck::AdamStep{count, lr, 1.0 - std::pow(0.9, t), 1.0 - std::pow(0.999, t)});
 }
 
 int ptc_ensure(dwfgpu_s* h) {
@@ -1624,14 +1568,15 @@ int ptc_ensure(dwfgpu_s* h) {
   int st = DWFGPU_OK;
   const size_t V = 2 * (size_t)h->g.vh;
   const int cmax = std::max(ls, n->hid);
+  const size_t nw = n->first(3);
+  st = alloc(h, (void**)&n->W, nw * sizeof(cx<float>));
+  if (!st) st = alloc(h, (void**)&n->G, nw * sizeof(cx<float>));
+  if (!st) st = alloc(h, (void**)&n->m, nw * sizeof(double2));
+  if (!st) st = alloc(h, (void**)&n->v, nw * sizeof(double2));
   for (int k = 0; k < 3 && !st; ++k) {
-    n->W[k].assign(n->nw(k), std::complex<float>(0.f, 0.f));
-    n->m[k].assign(2 * n->nw(k), 0.0);
-    n->v[k].assign(2 * n->nw(k), 0.0);
     const size_t abytes = (size_t)ptck::NDIR * 64 * n->cin(k) * n->cout(k) * 2;
     st = alloc(h, (void**)&n->A[k], abytes);
     if (!st) st = alloc(h, (void**)&n->Aadj[k], abytes);
-    if (!st) st = alloc(h, (void**)&n->G[k], n->nw(k) * sizeof(cx<float>));
   }
   const int chans[4] = {ls, n->hid, n->hid, ls};
   for (int k = 0; k < 4 && !st; ++k) st = alloc(h, (void**)&n->act[k], V * chans[k] * 12 * 4);
@@ -1654,24 +1599,37 @@ int ptc_ensure(dwfgpu_s* h) {
 // default weights: a damped local copy plus small random hops, so that the
 // untrained network is a scaled identity (z = 0.5 r) and training starts
 // from a valid preconditioner
-void ptc_init_weights(PtcNet* n, unsigned long long seed, double scale) {
+int ptc_init_weights(dwfgpu_s* h, unsigned long long seed, double scale) {
+  PtcNet* n = h->net;
+  std::vector<std::complex<float>> W(n->first(3));
+  // Unit normals by the polar method, two a draw: the sequence that
+  // std::normal_distribution gave with this generator.  Its uniforms cost two
+  // long double logarithms each (8-15 ms for Ls 16's 221184 numbers; 3 ms here).
   std::mt19937_64 rng(seed);
-  std::normal_distribution<double> nd(0.0, 1.0);
+  auto uniform = [&]() { return std::min((double)rng() * 0x1p-64, 1.0 - 0x1p-53); };
   for (int k = 0; k < 3; ++k) {
     const int ci = n->cin(k), co = n->cout(k);
-    for (size_t q = 0; q < n->nw(k); ++q)
-      n->W[k][q] = std::complex<float>((float)(scale * nd(rng)), (float)(scale * nd(rng)));
+    std::complex<float>* w = W.data() + n->first(k);
+    for (size_t q = 0; q < n->nw(k); ++q) {
+      double x, y, rr;
+      do {
+        x = 2.0 * uniform() - 1.0;
+        y = 2.0 * uniform() - 1.0;
+        rr = x * x + y * y;
+      } while (rr > 1.0 || rr == 0.0);
+      const double f = std::sqrt(-2.0 * std::log(rr) / rr);
+      w[q] = std::complex<float>((float)(scale * (y * f)), (float)(scale * (x * f)));
+    }
     // d = 0, o = i (channels that exist on both sides), a = b: a real diagonal
     const double diag = k == 2 ? 0.5 : 1.0;
     for (int o = 0; o < std::min(ci, co); ++o)
       for (int a = 0; a < 4; ++a)
-        n->W[k][(((size_t)(0 * co + o) * ci + o) * 4 + a) * 4 + a] += std::complex<float>((float)diag, 0.f);
+        w[(((size_t)(0 * co + o) * ci + o) * 4 + a) * 4 + a] += std::complex<float>((float)diag, 0.f);
   }
-  for (int k = 0; k < 3; ++k) {
-    std::fill(n->m[k].begin(), n->m[k].end(), 0.0);
-    std::fill(n->v[k].begin(), n->v[k].end(), 0.0);
-  }
+  HIPCHK(hipMemsetAsync(n->m, 0, W.size() * sizeof(double2), h->st));
+  HIPCHK(hipMemsetAsync(n->v, 0, W.size() * sizeof(double2), h->st));
   n->adam_t = 0;
+  return ptc_upload(h, reinterpret_cast<const float*>(W.data()));
 }
 
 }  // namespace
@@ -4176,30 +4134,18 @@ size_t dwfgpu_ptc_num_weights(dwfgpu_t h) {
 int dwfgpu_ptc_init(dwfgpu_t h, unsigned long long seed, double scale) {
   if (!h || h->prec != DWFGPU_F64) return DWFGPU_BAD_ARG;
   TRY(ptc_ensure(h));
-  ptc_init_weights(h->net, seed, scale);
-  return ptc_upload(h);
+  return ptc_init_weights(h, seed, scale);
 }
 
 int dwfgpu_ptc_set_weights(dwfgpu_t h, const float* w, size_t n) {
   if (!h || !w || !h->net || n != dwfgpu_ptc_num_weights(h)) return DWFGPU_BAD_ARG;
-  size_t q = 0;
-  for (int k = 0; k < 3; ++k)
-    for (auto& x : h->net->W[k]) {
-      x = std::complex<float>(w[2 * q], w[2 * q + 1]);
-      ++q;
-    }
-  return ptc_upload(h);
+  return ptc_upload(h, w);
 }
 
 int dwfgpu_ptc_get_weights(dwfgpu_t h, float* w, size_t n) {
   if (!h || !w || !h->net || n != dwfgpu_ptc_num_weights(h)) return DWFGPU_BAD_ARG;
-  size_t q = 0;
-  for (int k = 0; k < 3; ++k)
-    for (auto& x : h->net->W[k]) {
-      w[2 * q] = x.real();
-      w[2 * q + 1] = x.imag();
-      ++q;
-    }
+  HIPCHK(hipMemcpyAsync(w, h->net->W, n * sizeof(cx<float>), hipMemcpyDeviceToHost, h->st));
+  HIPCHK(hipStreamSynchronize(h->st));
   return DWFGPU_OK;
 }
 
@@ -4223,12 +4169,8 @@ int dwfgpu_ptc_loss_grad(dwfgpu_t h, const double* r, const double* e, double* l
   TRY(Ops<P32>::to_device(h, b, e));
   TRY(ptc_grad_pair(h, a, b, false, loss));
   if (grads) {
-    size_t off = 0;
-    for (int k = 0; k < 3; ++k) {
-      HIPCHK(hipMemcpyAsync(grads + 2 * off, h->net->G[k], h->net->nw(k) * sizeof(cx<float>),
-                            hipMemcpyDeviceToHost, h->st));
-      off += h->net->nw(k);
-    }
+    HIPCHK(hipMemcpyAsync(grads, h->net->G, h->net->first(3) * sizeof(cx<float>),
+                          hipMemcpyDeviceToHost, h->st));
   }
   HIPCHK(hipStreamSynchronize(h->st));
   return DWFGPU_OK;

@@ -700,6 +700,82 @@ k_ptc_gw_reduce(cx<float>* __restrict__ G, const float* __restrict__ part, int n
   }
 }
 
+// One layer's weights W[d][o][i][a][b] (FP32 complex), its gradient, the Adam
+// moments of (re, im) and the bf16 real forms of the layer and of its adjoint
+// in the fragment order of k_ptc_fwd.
+struct LayerWeights {
+  cx<float>* W;
+  const cx<float>* G;
+  double2 *m, *v;
+  uint16_t *A, *Aadj;
+  int cin, cout;
+};
+struct NetWeights {
+  LayerWeights l[3];
+};
+// Adam's step with the gradient summed over `count` pairs (count 0: none, only
+// the real forms); c1, c2 = 1 - b1^t, 1 - b2^t
+struct AdamStep {
+  int count;
+  double lr, c1, c2;
+};
+
+__host__ __device__ __forceinline__ uint16_t bf16_bits(float x) {  // to nearest even
+  uint32_t u = __builtin_bit_cast(uint32_t, x);
+  u += 0x7fffu + ((u >> 16) & 1u);
+  return (uint16_t)(u >> 16);
+}
+// place of element (row, col) of direction d of an [9][mp][kp] real form
+__device__ __forceinline__ size_t frag_at(int d, int row, int col, int mp, int kp) {
+  const int lane = row % 16 + 16 * (col % 32 / 8);
+  return ((((size_t)d * (mp / 16) + row / 16) * (kp / 32) + col / 32) * 64 + lane) * 8 + col % 8;
+}
+
+// The weights of layer blockIdx.y after an Adam step, and from each of them its
+// four places in A_d = [[Re W_d, -Im W_d], [Im W_d, Re W_d]] and in the
+// adjoint layer's form (W'_{-d}[i][o][b][a] = conj W_d[o][i][a][b]).  On the
+// host, with the gradients fetched and six forms sent, this was 1.5 ms of every
+// mini-batch at Ls 16 with the device idle; here one launch of a few us, bound
+// by its scattered 2-byte stores.
+__global__ void __launch_bounds__(256) k_ptc_weights(NetWeights net, AdamStep st) {
+#pragma clang fp contract(off)
+  const LayerWeights L = net.l[blockIdx.y];
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= NDIR * L.cout * L.cin * 16) return;
+  cx<float> w = L.W[q];
+  if (st.count > 0) {
+    const double b1 = 0.9, b2 = 0.999, eps = 1e-8;
+    const cx<float> g = L.G[q];
+    const double g2[2] = {(double)(g.re / (float)st.count), (double)(g.im / (float)st.count)};
+    const double2 m0 = L.m[q], v0 = L.v[q];
+    double m2[2] = {m0.x, m0.y}, v2[2] = {v0.x, v0.y}, w2[2] = {(double)w.re, (double)w.im};
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      m2[c] = b1 * m2[c] + (1.0 - b1) * g2[c];
+      v2[c] = b2 * v2[c] + (1.0 - b2) * g2[c] * g2[c];
+      w2[c] -= st.lr * (m2[c] / st.c1) / (sqrt(v2[c] / st.c2) + eps);
+    }
+    L.m[q] = double2{m2[0], m2[1]};
+    L.v[q] = double2{v2[0], v2[1]};
+    w = cx<float>{(float)w2[0], (float)w2[1]};
+    L.W[q] = w;
+  }
+  const int b = q % 4, a = q / 4 % 4, i = q / 16 % L.cin, o = q / (16 * L.cin) % L.cout;
+  const int d = q / (16 * L.cin * L.cout), da = d == 0 ? 0 : d <= 4 ? d + 4 : d - 4;
+  const uint16_t re = bf16_bits(w.re), im = bf16_bits(w.im), neg = bf16_bits(-w.im);
+  const int ro = o * 4 + a, ri = i * 4 + b;            // real rows / columns
+  const int co = L.cout * 4 + ro, ci = L.cin * 4 + ri;  // imaginary ones
+  const int mo = 8 * L.cout, mi = 8 * L.cin;
+  L.A[frag_at(d, ro, ri, mo, mi)] = re;
+  L.A[frag_at(d, ro, ci, mo, mi)] = neg;
+  L.A[frag_at(d, co, ri, mo, mi)] = im;
+  L.A[frag_at(d, co, ci, mo, mi)] = re;
+  L.Aadj[frag_at(da, ri, ro, mi, mo)] = re;
+  L.Aadj[frag_at(da, ri, co, mi, mo)] = im;
+  L.Aadj[frag_at(da, ci, ro, mi, mo)] = neg;
+  L.Aadj[frag_at(da, ci, co, mi, mo)] = re;
+}
+
 // Re <x, y> partial sums over a half vector
 template <class P>
 __global__ void __launch_bounds__(dwfk::BLAS_THREADS)
