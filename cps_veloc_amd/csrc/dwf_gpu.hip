@@ -1485,6 +1485,11 @@ int ptc_gw_nwg(dwfgpu_s* h, int cin, int cout, int* nwg) {
   return DWFGPU_BAD_ARG;
 }
 
+// work-groups of the passes over tiles of activations
+dim3 ptc_tiles(const dwfgpu_s* h) {
+  return dim3(std::min(dwfk::BLAS_BLOCKS, h->g.vh / ptck::TS));
+}
+
 // z = |r| net(r/|r|) on sloppy vectors (z must differ from r)
 template <class P>
 int ptc_apply(dwfgpu_s* h, const DVec& z, const DVec& r, double* rnorm_out = nullptr) {
@@ -1495,7 +1500,7 @@ int ptc_apply(dwfgpu_s* h, const DVec& z, const DVec& r, double* rnorm_out = nul
   if (rnorm_out) *rnorm_out = rn;
   if (rn == 0.0) return Ops<P>::copy(h, z, r);  // r = 0: z = 0
   const int action = h->action == DWFGPU_DWF ? 0 : 1;
-  hipLaunchKernelGGL((ptck::k_ptc_embed<P>), dim3(2048), dim3(256), 0, h->st, n->act[0],
+  hipLaunchKernelGGL((ptck::k_ptc_embed<P>), ptc_tiles(h), dim3(256), ptck::act_tile_lds(h->ls), h->st, n->act[0],
                      cfld<P>(r), h->g, action, (float)(1.0 / rn));
   HIPCHK(hipGetLastError());
   for (int k = 0; k < 3; ++k) TRY(ptc_fwd(h, n->cin(k), n->cout(k), n->act[k + 1], n->act[k], n->A[k]));
@@ -1518,22 +1523,22 @@ int ptc_grad_pair(dwfgpu_s* h, const DVec& r, const DVec& e, bool accumulate, do
     return DWFGPU_BAD_ARG;
   }
   const double nt = ee / rr;  // |e/|r||^2
-  hipLaunchKernelGGL((ptck::k_ptc_embed<P32>), dim3(2048), dim3(256), 0, h->st, n->act[0],
+  hipLaunchKernelGGL((ptck::k_ptc_embed<P32>), ptc_tiles(h), dim3(256), ptck::act_tile_lds(h->ls), h->st, n->act[0],
                      cfld<P32>(r), h->g, action, (float)(1.0 / rn));
   HIPCHK(hipGetLastError());
   for (int k = 0; k < 3; ++k) TRY(ptc_fwd(h, n->cin(k), n->cout(k), n->act[k + 1], n->act[k], n->A[k]));
-  hipLaunchKernelGGL(ptck::k_ptc_loss, dim3(dwfk::BLAS_BLOCKS), dim3(256), 0, h->st, n->gact[0],
+  hipLaunchKernelGGL(ptck::k_ptc_loss, ptc_tiles(h), dim3(256), ptck::act_tile_lds(h->ls), h->st, n->gact[0],
                      n->act[3], cfld<P32>(e), (float)(1.0 / rn), h->g, action, (float)(1.0 / nt),
                      h->partial);
   HIPCHK(hipGetLastError());
   double dd;
-  TRY(fetch_sum(h, dwfk::BLAS_BLOCKS, &dd));
+  TRY(fetch_sum(h, ptc_tiles(h).x, &dd));
   if (loss) *loss = dd / nt;
   // backward: layer 2, 1, 0 (gact ping-pong)
   int cur = 0;
   for (int k = 2; k >= 0; --k) {
     TRY(ptc_gw(h, n->cin(k), n->cout(k), n->gwpart, n->nwg[k], n->gact[cur], n->act[k]));
-    hipLaunchKernelGGL(ptck::k_ptc_gw_reduce, dim3(128), dim3(256), 0, h->st, n->G + n->first(k),
+    hipLaunchKernelGGL(ptck::k_ptc_gw_reduce, dim3(n->nw(k) / 64), dim3(256), 0, h->st, n->G + n->first(k),
                        n->gwpart, n->nwg[k], n->cin(k), n->cout(k), accumulate ? 1 : 0);
     HIPCHK(hipGetLastError());
     if (k > 0) {

@@ -90,26 +90,58 @@ __global__ void __launch_bounds__(256) k_gauss_f32(float* __restrict__ out, size
   }
 }
 
+// Activations of TS sites and every channel, staged in LDS between the CG
+// vector (site index fastest) and the activations (a site's C * 12 words
+// contiguous): both sides then move whole rows.  With a thread per (slice, site)
+// storing its 48 bytes a row apart, the embedding of a 16^3x32 Ls 16 vector took
+// 73 us and the loss 114; 34 and 44 us this way (5.8 TB/s).
+// Sites are padded by 4 words against bank conflicts.
+constexpr int TS = 16;
+__host__ __device__ constexpr int act_tile_stride(int C) { return C * 12 + 4; }
+__host__ __device__ constexpr size_t act_tile_lds(int C) {
+  return (size_t)TS * act_tile_stride(C) * 4;
+}
+// rows i0 .. i0 + TS of both parities from the tile: a channel's words on its
+// own parity, zeros on the other
+__device__ __forceinline__ void store_act_tile(uint32_t* __restrict__ act,
+                                               const uint32_t* __restrict__ t, const Geom& g,
+                                               int i0, int action) {
+  const int C = g.ls, quads = C * 3, st = act_tile_stride(C);
+  for (int w = threadIdx.x; w < 2 * TS * quads; w += blockDim.x) {
+    const int p = w / (TS * quads), r = w - p * TS * quads, n = r / quads, q = r - n * quads;
+    u32x4 v = *reinterpret_cast<const u32x4*>(t + n * st + q * 4);
+    if (slice_parity(action, q / 3) != p) v = u32x4{0u, 0u, 0u, 0u};
+    *reinterpret_cast<u32x4*>(act + ((size_t)(p * g.vh + i0 + n) * C) * 12 + q * 4) = v;
+  }
+}
+__device__ __forceinline__ void put_item(uint32_t* t, const uint32_t* w) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    *reinterpret_cast<u32x4*>(t + 4 * k) = u32x4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
+}
+
 // CG half vector (policy P, times `scale`) -> activations with C = ls
-// channels; the other parity of every channel is cleared
+// channels; the other parity of every channel is cleared.  vh is a multiple of TS
 template <class P>
 __global__ void __launch_bounds__(256)
 k_ptc_embed(uint32_t* __restrict__ act, dwfk::CFld<P> in, Geom g, int action, float scale) {
-  const int C = g.ls;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < (size_t)g.vh * g.ls;
-       k += (size_t)gridDim.x * blockDim.x) {
-    const int s = (int)(k / g.vh), i = (int)(k - (size_t)s * g.vh);
-    const int p = slice_parity(action, s);
-    cx<typename P::R> v[12];
-    dwfk::ld_spinor<P>(in.d + (size_t)s * dwfk::nch<P>() * g.vh, in.sc + (size_t)s * g.vh, g.vh,
-                       i, v);
-    uint32_t* dst = act + ((size_t)(p * g.vh + i) * C + s) * 12;
-    uint32_t* zer = act + ((size_t)((1 - p) * g.vh + i) * C + s) * 12;
+  extern __shared__ __align__(16) uint32_t tile[];
+  const int C = g.ls, st = act_tile_stride(C);
+  for (int i0 = blockIdx.x * TS; i0 < g.vh; i0 += gridDim.x * TS) {
+    for (int k = threadIdx.x; k < TS * C; k += blockDim.x) {
+      const int s = k / TS, n = k - s * TS;
+      cx<typename P::R> v[12];
+      dwfk::ld_spinor<P>(in.d + (size_t)s * dwfk::nch<P>() * g.vh, in.sc + (size_t)s * g.vh, g.vh,
+                         i0 + n, v);
+      uint32_t w[12];
 #pragma unroll
-    for (int c = 0; c < 12; ++c) {
-      dst[c] = pack_c(cx<float>{(float)v[c].re * scale, (float)v[c].im * scale});
-      zer[c] = 0u;
+      for (int c = 0; c < 12; ++c)
+        w[c] = pack_c(cx<float>{(float)v[c].re * scale, (float)v[c].im * scale});
+      put_item(tile + n * st + s * 12, w);
     }
+    __syncthreads();
+    store_act_tile(act, tile, g, i0, action);
+    __syncthreads();
   }
 }
 
@@ -144,25 +176,35 @@ __global__ void __launch_bounds__(256)
 k_ptc_loss(uint32_t* __restrict__ gact, const uint32_t* __restrict__ a3,
            dwfk::CFld<dwfk::P32> target, float tscale, Geom g, int action, float gscale,
            double* __restrict__ partial) {
+  extern __shared__ __align__(16) uint32_t tile[];
   __shared__ double sh[16];
-  const int C = g.ls;
+  const int C = g.ls, quads = C * 3, st = act_tile_stride(C);
   double acc = 0.0;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < (size_t)g.vh * g.ls;
-       k += (size_t)gridDim.x * blockDim.x) {
-    const int s = (int)(k / g.vh), i = (int)(k - (size_t)s * g.vh);
-    const int p = slice_parity(action, s);
-    const size_t base = ((size_t)(p * g.vh + i) * C + s) * 12;
-    cx<float> t[12];
-    dwfk::ld_spinor<dwfk::P32>(target.d + (size_t)s * 6 * g.vh, nullptr, g.vh, i, t);
-    uint32_t* zer = gact + ((size_t)((1 - p) * g.vh + i) * C + s) * 12;
-#pragma unroll
-    for (int c = 0; c < 12; ++c) {
-      const cx<float> o = unpack_c(a3[base + c]);
-      const cx<float> d{o.re - tscale * t[c].re, o.im - tscale * t[c].im};
-      acc += (double)d.re * d.re + (double)d.im * d.im;
-      gact[base + c] = pack_c(cx<float>{d.re * gscale, d.im * gscale});
-      zer[c] = 0u;
+  for (int i0 = blockIdx.x * TS; i0 < g.vh; i0 += gridDim.x * TS) {
+    for (int w = threadIdx.x; w < TS * quads; w += blockDim.x) {
+      const int n = w / quads, q = w - n * quads, p = slice_parity(action, q / 3);
+      *reinterpret_cast<u32x4*>(tile + n * st + q * 4) = *reinterpret_cast<const u32x4*>(
+          a3 + ((size_t)(p * g.vh + i0 + n) * C) * 12 + q * 4);
     }
+    __syncthreads();
+    for (int k = threadIdx.x; k < TS * C; k += blockDim.x) {
+      const int s = k / TS, n = k - s * TS;
+      cx<float> t[12];
+      dwfk::ld_spinor<dwfk::P32>(target.d + (size_t)s * 6 * g.vh, nullptr, g.vh, i0 + n, t);
+      uint32_t* o = tile + n * st + s * 12;
+      uint32_t w[12];
+#pragma unroll
+      for (int c = 0; c < 12; ++c) {
+        const cx<float> a = unpack_c(o[c]);
+        const cx<float> d{a.re - tscale * t[c].re, a.im - tscale * t[c].im};
+        acc += (double)d.re * d.re + (double)d.im * d.im;
+        w[c] = pack_c(cx<float>{d.re * gscale, d.im * gscale});
+      }
+      put_item(o, w);
+    }
+    __syncthreads();
+    store_act_tile(gact, tile, g, i0, action);
+    __syncthreads();
   }
   const double tot = dwfk::block_sum(acc, sh);
   if (threadIdx.x == 0) partial[blockIdx.x] = tot;
@@ -669,35 +711,46 @@ k_ptc_gw(float* __restrict__ part, int nwg, const uint32_t* __restrict__ gout,
 }
 
 // G[d][o][i][a][b] (complex, FP32) = 2 * (P_re,re + P_im,im, P_im,re - P_re,im)
-// summed over the nwg partials in a fixed order
+// summed over the nwg partials in a fixed order.  A work-group takes 64
+// elements, the columns (i, b) of a row (o, a) fastest so that its loads are
+// whole rows of a partial, and a quarter of the partials a wave (one thread per
+// element over all of them, 16-byte pieces a load: 44 us at nwg 80, K' = M' =
+// 128; 28 us now).
 __global__ void __launch_bounds__(256)
 k_ptc_gw_reduce(cx<float>* __restrict__ G, const float* __restrict__ part, int nwg, int cin,
                 int cout, int accumulate) {
+  __shared__ double2 sum[3][64];
   const int MP = 8 * cout, KP = 8 * cin;
-  const int n = NDIR * cout * 4 * cin * 4;
-  for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < n; w += gridDim.x * blockDim.x) {
-    int r = w;
-    const int b = r % 4;
-    r /= 4;
-    const int i = r % cin;
-    r /= cin;
-    const int a = r % 4;
-    r /= 4;
-    const int o = r % cout;
-    const int d = r / cout;
-    const int mre = o * 4 + a, mim = cout * 4 + o * 4 + a;
-    const int kre = i * 4 + b, kim = cin * 4 + i * 4 + b;
-    double re = 0.0, im = 0.0;
-    for (int q = 0; q < nwg; ++q) {
-      const float* P = part + ((size_t)d * nwg + q) * MP * KP;
-      re += (double)P[mre * KP + kre] + (double)P[mim * KP + kim];
-      im += (double)P[mim * KP + kre] - (double)P[mre * KP + kim];
-    }
-    // G index [d][o][i][a][b]
-    cx<float>& gv = G[(((size_t)(d * cout + o) * cin + i) * 4 + a) * 4 + b];
-    const cx<float> old = accumulate ? gv : cx<float>{0.f, 0.f};
-    gv = cx<float>{old.re + (float)(2.0 * re), old.im + (float)(2.0 * im)};
+  const int e = threadIdx.x & 63, quarter = threadIdx.x >> 6;
+  int r = blockIdx.x * 64 + e;  // the element count, 9 * 16 * cin * cout, is a multiple of 64
+  const int b = r % 4;
+  r /= 4;
+  const int i = r % cin;
+  r /= cin;
+  const int a = r % 4;
+  r /= 4;
+  const int o = r % cout, d = r / cout;
+  const int mre = o * 4 + a, mim = cout * 4 + o * 4 + a;
+  const int kre = i * 4 + b, kim = cin * 4 + i * 4 + b;
+  double re = 0.0, im = 0.0;
+  const int q1 = nwg * (quarter + 1) / 4;
+#pragma unroll 4
+  for (int q = nwg * quarter / 4; q < q1; ++q) {
+    const float* P = part + ((size_t)d * nwg + q) * MP * KP;
+    re += (double)P[mre * KP + kre] + (double)P[mim * KP + kim];
+    im += (double)P[mim * KP + kre] - (double)P[mre * KP + kim];
   }
+  if (quarter) sum[quarter - 1][e] = double2{re, im};
+  __syncthreads();
+  if (quarter) return;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    re += sum[k][e].x;
+    im += sum[k][e].y;
+  }
+  cx<float>& gv = G[(((size_t)(d * cout + o) * cin + i) * 4 + a) * 4 + b];
+  const cx<float> old = accumulate ? gv : cx<float>{0.f, 0.f};
+  gv = cx<float>{old.re + (float)(2.0 * re), old.im + (float)(2.0 * im)};
 }
 
 // One layer's weights W[d][o][i][a][b] (FP32 complex), its gradient, the Adam
