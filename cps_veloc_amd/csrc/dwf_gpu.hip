@@ -95,6 +95,7 @@ struct dwfgpu_s {
   double* stage4d = nullptr;  // one 4D CANONICAL fermion slice (format calls)
   int* nbt = nullptr;         // neighbour table of the hop kernels (g.nbt)
   double* partial = nullptr;
+  double* partial64 = nullptr;  // <p, A p>'s of a small-lattice CG step
   int npartial = 0;
   double* dscal = nullptr;
   double* hscal = nullptr;   // pinned
@@ -437,13 +438,15 @@ void set_shape64(dwfgpu_s* h) {
 // partials.  masses: nrhs right-hand sides, n/2 components apart (device).
 int dwf64(dwfgpu_s* h, const Geom& g, cx<double>* out, const cx<double>* in, const cx<double>* x0,
           int cb_in, int dag, int epi, bool norm, double nm, double alpha, double* partial,
-          cx<double>* r, const double* scal, const double* masses = nullptr, int nrhs = 1) {
+          cx<double>* r, const dwfk::CgScal64* scal, const double* masses = nullptr,
+          int nrhs = 1) {
   const dim3 grid(h->grid64, nrhs), block(2 * h->ns64, h->ls, 2);
   const size_t lds = lds64(h, h->ns64);
   const cx<double>* u = (const cx<double>*)h->f[DWFGPU_F64].U;
 #define DWF64_LAUNCH(DAG, EPI, NORM, CG)                                                         \
   hipLaunchKernelGGL((dwfk::k_dwf64<DAG, EPI, NORM, CG>), grid, block, lds, h->st, out, in, u,   \
-                     x0, partial, g, cb_in, 2.0 * h->a5inv, nm, alpha, r, scal, masses, h->n / 2)
+                     x0, partial, g, cb_in, 2.0 * h->a5inv, nm, alpha, r,                        \
+                     scal ? *scal : dwfk::CgScal64{}, masses, h->n / 2)
   if (scal) DWF64_LAUNCH(1, 1, false, true);
   else if (epi == 0 && dag) DWF64_LAUNCH(1, 0, false, false);
   else if (epi == 0) DWF64_LAUNCH(0, 0, false, false);
@@ -459,7 +462,7 @@ int dwf64(dwfgpu_s* h, const Geom& g, cx<double>* out, const cx<double>* in, con
 // Small-lattice FP64 Mobius pass; fl: dwfk::FL_*, with FL_CG r and scal as above
 int mob64(dwfgpu_s* h, const Geom& g, const MobArgs& a, cx<double>* out, const cx<double>* in,
           const cx<double>* psi, int p_out, int dag, int epi, int fl, double* partial,
-          cx<double>* r, const double* scal) {
+          cx<double>* r, const dwfk::CgScal64* scal) {
   using namespace dwfk;
   const dim3 grid(h->grid64), block(2 * h->ns64, h->ls, 2);
   const size_t lds = std::max(lds64_cols(h->ns64, h->ls), !dag && !(fl & FL_PRE_T)
@@ -468,7 +471,7 @@ int mob64(dwfgpu_s* h, const Geom& g, const MobArgs& a, cx<double>* out, const c
   const cx<double>* u = (const cx<double>*)h->f[DWFGPU_F64].U;
 #define MOB64_LAUNCH(DAG, EPI, FL)                                                              \
   hipLaunchKernelGGL((k_mobius64<DAG, EPI, FL>), grid, block, lds, h->st, out, in, psi, u,      \
-                     partial, g, p_out, a, r, scal)
+                     partial, g, p_out, a, r, scal ? *scal : CgScal64{})
   if (!dag && epi == EPI_M5INV) MOB64_LAUNCH(0, EPI_M5INV, FL_POST_T);
   else if (!dag && epi == EPI_SCHUR && (fl & FL_NORM)) MOB64_LAUNCH(0, EPI_SCHUR, FL_PRE_T | FL_NORM);
   else if (!dag && epi == EPI_SCHUR) MOB64_LAUNCH(0, EPI_SCHUR, FL_PRE_T);
@@ -614,9 +617,10 @@ struct Ops {
     Geom gm = h->g;
     gm.rev = 1;  // a Schur pass: backwards, as in mob()
     if constexpr (std::is_same<P, P64>::value && std::is_same<PX, dwfk::NoX>::value) {
+      const dwfk::CgScal64 cs{scal, nullptr, 0, nullptr, nullptr};
       if (h->ns64)
         return mob64(h, gm, a, nullptr, (const cx<double>*)te.d, (const cx<double>*)t1.d, 1, 1,
-                     dwfk::EPI_SCHUR, dwfk::FL_CG, partial, (cx<double>*)r.d, scal);
+                     dwfk::EPI_SCHUR, dwfk::FL_CG, partial, (cx<double>*)r.d, &cs);
     }
     const dim3 grid(h->grid_hop), block(h->ns, h->ls);
     const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), scal};
@@ -706,9 +710,10 @@ struct Ops {
       Geom gm = h->g;
       gm.rev = 1;  // an x0 + alpha D pass: backwards, as in dwf()
       if constexpr (std::is_same<P, P64>::value && std::is_same<PX, dwfk::NoX>::value) {
+        const dwfk::CgScal64 cs{h->dscal, nullptr, 0, nullptr, nullptr};
         if (h->ns64)
           return dwf64(h, gm, nullptr, (const cx<double>*)te.d, (const cx<double>*)t1.d, 0, 1, 1,
-                       false, -2.0 * mass * h->a5inv, mk2, h->partial, (cx<double>*)r.d, h->dscal);
+                       false, -2.0 * mass * h->a5inv, mk2, h->partial, (cx<double>*)r.d, &cs);
       }
       const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), h->dscal};
       hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, 1, 1, false, true, PX>), dim3(h->grid_hop),
@@ -730,6 +735,40 @@ struct Ops {
     TRY(mdagm_cg_launch<dwfk::NoX>(h, mass, p, r, DVec()));
     hipLaunchKernelGGL(dwfk::k_reduce_cg_step, dim3(1), dim3(1024), 0, h->st, h->partial, grid(h),
                        h->dscal, alpha, host);
+    HIPCHK(hipGetLastError());
+    return DWFGPU_OK;
+  }
+
+  // cg_step and the next direction `next` = r + beta p on a small lattice
+  // (ns64): five launches, the sums inside those that use them.  |r|^2 is in
+  // dscal[0] before an odd step and in dscal[3] before an even one.
+  static int cg_step64(dwfgpu_s* h, double mass, const DVec& p, const DVec& next, const DVec& r,
+                       int k, double* alpha, double* host) {
+    const DVec& te = F(h).te;
+    const DVec& t1 = F(h).t1;
+    const dwfk::CgScal64 cs{h->dscal + (k & 1 ? 0 : 3), h->partial64, h->grid64, alpha, host};
+    cx<double>* const rd = (cx<double>*)r.d;
+    const cx<double>*ted = (const cx<double>*)te.d, *t1d = (const cx<double>*)t1.d;
+    Geom gm = h->g;
+    gm.rev = 1;
+    if (h->action == DWFGPU_DWF) {
+      const double mk2 = -dwf_kappa(h) * dwf_kappa(h);
+      TRY(dwf(h, mass, te, p, 1, 0, 0, DVec(), 0.0, false));
+      TRY(dwf(h, mass, t1, te, 0, 0, 1, p, mk2, true, h->partial64));
+      TRY(dwf(h, mass, te, t1, 1, 1, 0, DVec(), 0.0, false));
+      TRY(dwf64(h, gm, nullptr, ted, t1d, 0, 1, 1, false, -2.0 * mass * h->a5inv, mk2, h->partial,
+                rd, &cs));
+    } else {
+      TRY(mob_first(h, mass, te, p, 0));
+      TRY(mob_second(h, mass, t1, te, p, 0, true, h->partial64));
+      TRY(mob_first(h, mass, te, t1, 1));
+      TRY(mob64(h, gm, mob_args(h, mass, 1), nullptr, ted, t1d, 1, 1, dwfk::EPI_SCHUR, dwfk::FL_CG,
+                h->partial, rd, &cs));
+    }
+    const size_t n = h->n / 2;
+    hipLaunchKernelGGL(dwfk::k_cg_end64, dim3((n + 255) / 256), dim3(256), 0, h->st,
+                       (cx<double>*)next.d, (const cx<double>*)rd, (const cx<double>*)p.d,
+                       h->partial, h->grid64, cs.rr, h->dscal + (k & 1 ? 3 : 0), host, n);
     HIPCHK(hipGetLastError());
     return DWFGPU_OK;
   }
@@ -874,6 +913,7 @@ struct Ops {
       TRY(ensure_ring<P>(h, NR));
     }
     auto slot = [&](int k) -> const DVec& { return NR == 1 ? dir : F(h).ring[k % NR]; };
+    const bool small = std::is_same<P, P64>::value && h->ns64 && NR > 1;
     EventSet<NEV> ev;
     TRY(ev.create());
     dwfk::XFlush<P> xf;
@@ -891,12 +931,16 @@ struct Ops {
     int itr = 0;
     for (int k = 1; k <= max_itr + LAG; ++k) {
       if (k <= max_itr) {
-        TRY(cg_step(h, mass, slot(k), res, h->dalpha + k % NR, h->hring + 4 * (k % NEV)));
+        double *al = h->dalpha + k % NR, *host = h->hring + 4 * (k % NEV);
+        bool done = false;
+        if constexpr (std::is_same<P, P64>::value)
+          if ((done = small)) TRY(cg_step64(h, mass, slot(k), slot(k + 1), res, k, al, host));
+        if (!done) TRY(cg_step(h, mass, slot(k), res, al, host));
         HIPCHK(hipEventRecord(ev.e[k % NEV], h->st));
       }
       // dir of step k + 1 = res + b dir; in place only after step k's update
       auto next = [&]() -> int {
-        if (k >= max_itr) return DWFGPU_OK;
+        if (small || k >= max_itr) return DWFGPU_OK;
         hipLaunchKernelGGL((dwfk::k_pnext<P>), blas_grid(), blas_block(), 0, h->st,
                            fld<P>(slot(k + 1)), cfld<P>(res), cfld<P>(slot(k)), h->dscal, h->g);
         HIPCHK(hipGetLastError());
@@ -1300,7 +1344,7 @@ void free_all(dwfgpu_s* h) {
     F.ring.clear();
     F.ready = false;
   }
-  void* ptrs[] = {h->cps_stage, h->stage4d, h->partial, h->dscal, h->nbt, h->dalpha};
+  void* ptrs[] = {h->cps_stage, h->stage4d, h->partial, h->partial64, h->dscal, h->nbt, h->dalpha};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (h->hscal) (void)hipHostFree(h->hscal);
@@ -3517,6 +3561,7 @@ int dwfgpu_create(const double* gauge, const int dims[4], int ls, int action, do
   if ((r = ensure_api(h, 0))) return fail(r);
   if ((r = alloc(h, &h->cps_stage, h->n * sizeof(double)))) return fail(r);
   if ((r = alloc(h, (void**)&h->partial, h->npartial * sizeof(double)))) return fail(r);
+  if (h->ns64 && (r = alloc(h, (void**)&h->partial64, h->grid64 * sizeof(double)))) return fail(r);
   if ((r = alloc(h, (void**)&h->dscal, 8 * sizeof(double)))) return fail(r);
   if ((r = alloc(h, (void**)&h->dalpha, 32 * sizeof(double)))) return fail(r);
   if (hipHostMalloc((void**)&h->hring, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess) {

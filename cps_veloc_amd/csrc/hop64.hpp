@@ -200,6 +200,78 @@ __host__ __device__ constexpr size_t lds64_tx(int ns, int ls) {
   return lds64_links(ns, 1) + (size_t)4 * ns * ls * 12 * 16;
 }
 
+// Sum of partials that every work-group forms for itself, without a barrier of
+// its own: the loads at the kernel's start, a value per wave staged before a
+// barrier the kernel has anyway, the total after it.  All work-groups of a
+// launch add in one order and get the same bits.
+struct PartSum {
+  double v = 0.0;
+  __device__ __forceinline__ void load(const double* __restrict__ p, int n, int tid, int nthr) {
+    for (int k = tid; k < n; k += nthr) v += p[k];
+  }
+  __device__ __forceinline__ void stage(double* sh, int tid) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    if ((tid & 63) == 0) sh[tid >> 6] = v;
+  }
+  static __device__ __forceinline__ double total(const double* sh, int nthr) {
+    double t = 0.0;
+    for (int w = 0; w < (nthr + 63) / 64; ++w) t += sh[w];
+    return t;
+  }
+};
+
+// What the last pass of a CG step gets of the scalars: *rr = |r|^2 and the
+// partials of <p, A p> (n > 0), of which work-group 0 leaves alpha and the sum
+// (host: pinned); or, n == 0, rr[1] = <p, A p>.
+struct CgScal64 {
+  const double* rr;
+  const double* dot;
+  int n;
+  double *alpha, *host;
+};
+__device__ __forceinline__ double cg_alpha64(const CgScal64& c, const double* sh, int tid,
+                                             int nthr) {
+  const double d = c.n ? PartSum::total(sh, nthr) : c.rr[1];
+  const double a = d != 0.0 ? c.rr[0] / d : 0.0;
+  if (c.n && blockIdx.x == 0 && tid == 0) {
+    *c.alpha = a;
+    c.host[1] = d;
+  }
+  return a;
+}
+
+// End of a CG step: |r|^2 from its partials into *rr_new and host[0] (pinned),
+// and the next direction pn = r + (|r|^2 / *rr_old) p of n components, one a
+// thread.  The two sums as launches of their own cost an 8^4 Ls 8 DWF step 5.2
+// us and two gaps; inside the last pass (7.5 -> 7.9 us) and here (3.4 -> 3.6 us)
+// the step takes 40.3 us instead of 46.1.  More partials than a small lattice's
+// (at most 1024) would cost every work-group more than the launch saves.
+__global__ void __launch_bounds__(256)
+k_cg_end64(c64* __restrict__ pn, const c64* __restrict__ r, const c64* __restrict__ p,
+           const double* __restrict__ partial, int np, const double* __restrict__ rr_old,
+           double* __restrict__ rr_new, double* __restrict__ host, size_t n) {
+  __shared__ double sh[4];
+  const int tid = threadIdx.x;
+  const size_t e = blockIdx.x * (size_t)256 + tid;
+  c64 rv{0, 0}, pv{0, 0};
+  if (e < n) {
+    rv = r[e];
+    pv = p[e];
+  }
+  const double ro = *rr_old;
+  PartSum s;
+  s.load(partial, np, tid, 256);
+  s.stage(sh, tid);
+  __syncthreads();
+  const double rr = PartSum::total(sh, 256), b = ro != 0.0 ? rr / ro : 0.0;
+  if (e < n) pn[e] = rv + b * pv;
+  if (e == 0) {
+    *rr_new = rr;
+    host[0] = rr;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // DWF (as k_dwf_dslash).  CG: r -= alpha_cg (x0 + alpha D in) instead of `out`.
 // ---------------------------------------------------------------------------
@@ -207,8 +279,8 @@ template <int DAG, int EPI, bool NORM, bool CG>
 __global__ void __launch_bounds__(512)
 k_dwf64(c64* __restrict__ out, const c64* __restrict__ in, const c64* __restrict__ U,
         const c64* __restrict__ x0, double* __restrict__ partial, Geom g, int cb_in,
-        double two_a5, double nm_two_a5, double alpha, c64* __restrict__ r,
-        const double* __restrict__ scal, const double* __restrict__ mass, size_t vs) {
+        double two_a5, double nm_two_a5, double alpha, c64* __restrict__ r, CgScal64 cs,
+        const double* __restrict__ mass, size_t vs) {
   // batched operator: right-hand side blockIdx.y starts vs components further
   // and has its own mass
   if (mass) {
@@ -219,13 +291,14 @@ k_dwf64(c64* __restrict__ out, const c64* __restrict__ in, const c64* __restrict
     nm_two_a5 = -mass[blockIdx.y] * two_a5;
   }
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ double sh[16];
+  __shared__ double sh[16], shd[8];
   const int ns = blockDim.x >> 1, s = threadIdx.y;
   const Own o{(int)threadIdx.x >= ns ? 1 : 0, (int)threadIdx.z};
   const int il = threadIdx.x - o.hf * ns;
   c64* lu = reinterpret_cast<c64*>(smem_raw);  // [2][8][ns][9]
   c64* mycol = lu + il * (g.ls * 12 + 1) + s * 12;
-  const double a_cg = CG ? cg_alpha(scal) : 0.0;
+  const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
+  const int nthr = blockDim.x * blockDim.y * blockDim.z;
   const int blk = xcd_block(g.nxcd, g.rev);
   const int i = blk * ns + il;
   const bool act = i < g.vh;
@@ -243,9 +316,13 @@ k_dwf64(c64* __restrict__ out, const c64* __restrict__ in, const c64* __restrict
     if (EPI == 1) ld_own(x0 + s * slice, g.vh, i, o, x);
     if (CG) ld_own(r + s * slice, g.vh, i, o, rv);
   }
+  PartSum dot;
+  if (CG) dot.load(cs.dot, cs.n, tid, nthr);
   __builtin_amdgcn_sched_barrier(0);
   stage_links64(lu, U, g, blk, ns, 2, (1 + cb_in) & 1);
+  if (CG) dot.stage(shd, tid);
   __syncthreads();
+  const double a_cg = CG ? cg_alpha64(cs, shd, tid, nthr) : 0.0;
   const int set = (s & 1) * 8;
 #pragma unroll
   for (int k = 0; k < 4; ++k) hop.add<DAG>(k, lu + (size_t)((set + hop.dir(k)) * ns + il) * 9);
@@ -283,9 +360,9 @@ template <int DAG, int EPI, int FL>
 __global__ void __launch_bounds__(512)
 k_mobius64(c64* __restrict__ out, const c64* __restrict__ in, const c64* __restrict__ psi,
            const c64* __restrict__ U, double* __restrict__ partial, Geom g, int p_out, MobArgs a,
-           c64* __restrict__ r, const double* __restrict__ scal) {
+           c64* __restrict__ r, CgScal64 cs) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ double sh[16];
+  __shared__ double sh[16], shd[8];
   const int ns = blockDim.x >> 1, s = threadIdx.y, ls = g.ls;
   const Own o{(int)threadIdx.x >= ns ? 1 : 0, (int)threadIdx.z};
   const int il = threadIdx.x - o.hf * ns;
@@ -294,7 +371,8 @@ k_mobius64(c64* __restrict__ out, const c64* __restrict__ in, const c64* __restr
   c64* col = reinterpret_cast<c64*>(smem_raw);  // s-columns, once the hop is done
   c64* mysite = col + il * sst;
   c64* mycol = mysite + s * 12;
-  const double a_cg = (FL & FL_CG) ? cg_alpha(scal) : 0.0;
+  const int ct = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
+  const int cthr = blockDim.x * blockDim.y * blockDim.z;
   const int blk = xcd_block(g.nxcd, g.rev);
   const int i = blk * ns + il;
   const bool act = i < g.vh;
@@ -306,9 +384,13 @@ k_mobius64(c64* __restrict__ out, const c64* __restrict__ in, const c64* __restr
   c64 w[3], rv[3], v[3];
   if (EPI == EPI_SCHUR && act) ld_own(psi + s * slice, g.vh, i, o, w);
   if ((FL & FL_CG) && act) ld_own(r + s * slice, g.vh, i, o, rv);
+  PartSum dot;
+  if (FL & FL_CG) dot.load(cs.dot, cs.n, ct, cthr);
   __builtin_amdgcn_sched_barrier(0);
   stage_links64(lu, U, g, blk, ns, 1, p_out);
+  if (FL & FL_CG) dot.stage(shd, ct);
   __syncthreads();
+  const double a_cg = (FL & FL_CG) ? cg_alpha64(cs, shd, ct, cthr) : 0.0;
   if constexpr (DAG == 0 && !(FL & FL_PRE_T)) {
     // (b + c D5) in of each neighbour: spin hf of slice s - 1 and the second
     // spin (a lower one) of slice s + 1 from those slices' threads, two
