@@ -1920,29 +1920,79 @@ struct MrShape {
   int ns, nr;
 };
 
+// steps of a round of the batched CG, and directions kept for its end: each is
+// a vector per RHS, and the update of x moves (MR_RING + 2) / MR_RING vectors a
+// step where x += alpha p in the last pass of every step moved 3
+constexpr int MR_RING = 4;
+
+// everything a batched call allocates, in one block (nine or more buffers of
+// their own took 1.5-2.5 ms to free)
 template <class PS>
 struct MrState {
-  int nrhs = 0;
-  DVec te, t1, rs, ps, xs;  // xs in P32
-  double* partial = nullptr;
-  double* scal = nullptr;
-  double* mass = nullptr;
-  MobArgs* mob = nullptr;  // Mobius: of each RHS for dag 0, then for dag 1
-  int* ibuf = nullptr;  // active | flag | iters
+  int nrhs = 0, nring = 1;
+  DVec te, t1, rs, ps[MR_RING], xs;  // xs in P32
+  double *partial = nullptr, *scal = nullptr, *mass = nullptr;
+  double* alpha = nullptr;  // [nrhs][nring]
+  MobArgs* mob = nullptr;   // Mobius: of each RHS for dag 0, then for dag 1
+  int* ibuf = nullptr;      // active | flag | iters
   int gx = 0;
+  char* block = nullptr;
   ~MrState() {
-    free_vec(&te);
-    free_vec(&t1);
-    free_vec(&rs);
-    free_vec(&ps);
-    free_vec(&xs);
-    void* p[] = {partial, scal, mass, mob, ibuf};
-    for (void* q : p)
-      if (q) (void)hipFree(q);
+    if (block) (void)hipFree(block);
   }
   int* active() const { return ibuf; }
   int* flag() const { return ibuf + nrhs; }
   int* iters() const { return ibuf + 2 * nrhs; }
+
+  // the buffers, zeroed; cg: rs, xs and a ring of directions too
+  int create(dwfgpu_s* h, int n, int partials, bool cg) {
+    nrhs = n;
+    gx = partials;
+    for (nring = cg ? MR_RING : 1;; nring = 1) {
+      const size_t bytes = carve(h, nullptr, cg);
+      if (hipMalloc((void**)&block, bytes) == hipSuccess) {
+        carve(h, block, cg);
+        HIPCHK(hipMemsetAsync(block, 0, bytes, h->st));
+        return DWFGPU_OK;
+      }
+      block = nullptr;
+      if (nring > 1) {  // without room for the ring
+        (void)hipGetLastError();
+        continue;
+      }
+      HIPCHK(hipGetLastError());
+      return DWFGPU_HIP_ERROR;
+    }
+  }
+
+ private:
+  size_t carve(const dwfgpu_s* h, char* base, bool cg) {
+    size_t off = 0;
+    auto take = [&](size_t bytes) -> void* {
+      void* p = base ? base + off : nullptr;
+      off += (bytes + 255) / 256 * 256;
+      return p;
+    };
+    auto vec = [&](size_t real, bool scaled) {
+      DVec v;
+      v.d = take((size_t)nrhs * h->n * real);
+      if (scaled) v.sc = (float*)take((size_t)nrhs * h->g.vh * h->ls * sizeof(float));
+      return v;
+    };
+    constexpr size_t real = sizeof(typename PS::S) / 2;
+    te = vec(real, PS::kScaled);
+    t1 = vec(real, PS::kScaled);
+    rs = vec(real, PS::kScaled);
+    for (int q = 0; q < nring; ++q) ps[q] = vec(real, PS::kScaled);
+    if (cg) xs = vec(sizeof(float), false);
+    partial = (double*)take((size_t)nrhs * gx * sizeof(double));
+    scal = (double*)take((size_t)nrhs * dwfk::MR_NSCAL * sizeof(double));
+    mass = (double*)take(nrhs * sizeof(double));
+    alpha = (double*)take((size_t)nrhs * nring * sizeof(double));
+    mob = (MobArgs*)take((size_t)2 * nrhs * sizeof(MobArgs));
+    ibuf = (int*)take((size_t)3 * nrhs * sizeof(int));
+    return off;
+  }
 };
 
 size_t mr_lds(const dwfgpu_s* h, const MrShape& t, size_t creal) {
@@ -1970,44 +2020,48 @@ bool mr_shape_ok(const dwfgpu_s* h, const MrShape& t, int nrhs, size_t creal) {
 // kind 2: out = D^dag in (cb 1)      kind 3: x0 + alpha D^dag in -> CG epilogue
 // kind 4: out = x0 + alpha D^dag in (plain batched MatPcDagMatPc)
 template <class P>
-int mr_launch(dwfgpu_s* h, const MrShape& t, int nrhs, dwfk::MrArgs<P, P32> a, int kind) {
+int mr_launch(dwfgpu_s* h, const MrShape& t, int nrhs, dwfk::MrArgs<P> a, int kind) {
   const dim3 grid((h->g.vh + t.ns - 1) / t.ns, (nrhs + t.nr - 1) / t.nr);
   const dim3 block(t.ns, h->ls, t.nr);
   const size_t lds = mr_lds(h, t, sizeof(typename P::R));
   a.cb_in = (kind == 0 || kind == 2) ? 1 : 0;
   switch (kind) {
     case 0:
-      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 0, 0, false, false, P32>), grid, block, lds, h->st, a);
+      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 0, 0, false, false>), grid, block, lds, h->st, a);
       break;
     case 1:
-      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 0, 1, true, false, P32>), grid, block, lds, h->st, a);
+      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 0, 1, true, false>), grid, block, lds, h->st, a);
       break;
     case 2:
-      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 1, 0, false, false, P32>), grid, block, lds, h->st, a);
+      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 1, 0, false, false>), grid, block, lds, h->st, a);
       break;
     case 3:
-      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 1, 1, false, true, P32>), grid, block, lds, h->st, a);
+      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 1, 1, false, true>), grid, block, lds, h->st, a);
       break;
     default:
-      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 1, 1, false, false, P32>), grid, block, lds, h->st, a);
+      hipLaunchKernelGGL((dwfk::k_dwf_mrhs<P, 1, 1, false, false>), grid, block, lds, h->st, a);
       break;
   }
   HIPCHK(hipGetLastError());
   return DWFGPU_OK;
 }
 
-// batched MatPcDagMatPc (cg: the CG step of every active RHS instead of `out`)
+// batched MatPcDagMatPc of `in` (cg: the CG step of every active RHS, r -= alpha
+// A p with |r|^2 partials, instead of `out`)
 template <class P>
-int mr_mdagm(dwfgpu_s* h, const MrShape& t, int nrhs, const DVec& out, const DVec& in,
-             const DVec& te, const DVec& t1, const double* mass, const int* active,
-             double* partial, double* scal, const DVec* r, const DVec* x, bool cg) {
+int mr_mdagm(dwfgpu_s* h, const MrShape& t, const MrState<P>& m, const DVec& out, const DVec& in,
+             double* scal, bool cg) {
+  const DVec &te = m.te, &t1 = m.t1;
+  const int nrhs = m.nrhs;
+  double* const partial = m.partial;
+  const int* const active = m.active();
   const double kap = dwf_kappa(h);
-  dwfk::MrArgs<P, P32> a{};
+  dwfk::MrArgs<P> a{};
   a.U = (const typename P::S*)h->f[pidx<P>()].U;
   a.partial = partial;
   a.g = h->g;
   a.two_a5 = 2.0 * h->a5inv;
-  a.mass = mass;
+  a.mass = m.mass;
   a.active = active;
   a.vs = h->n / 2 / P::kCPC;
   a.nrhs = nrhs;
@@ -2039,13 +2093,8 @@ int mr_mdagm(dwfgpu_s* h, const MrShape& t, int nrhs, const DVec& out, const DVe
   a.x0 = cfld<P>(t1);
   a.alpha = -kap * kap;
   if (cg) {
-    a.r = fld<P>(*r);
-    a.p = cfld<P>(in);
-    a.x = fld<P32>(*x);
+    a.r = fld<P>(m.rs);
     TRY(mr_launch<P>(h, t, nrhs, a, 3));
-    hipLaunchKernelGGL(dwfk::k_reduce_mrhs, dim3(nrhs), dim3(1024), 0, h->st, partial, gx, scal,
-                       (int)dwfk::MR_RRNEW, active);
-    HIPCHK(hipGetLastError());
   } else {
     a.out = fld<P>(out);
     TRY(mr_launch<P>(h, t, nrhs, a, 4));
@@ -2059,7 +2108,6 @@ int mr_mob_args(dwfgpu_s* h, const double* masses, MrState<P>& m) {
   std::vector<MobArgs> a;
   for (int dag = 0; dag < 2; ++dag)
     for (int j = 0; j < m.nrhs; ++j) a.push_back(mob_args(h, masses[j], dag));
-  TRY(alloc(h, (void**)&m.mob, a.size() * sizeof(MobArgs)));
   HIPCHK(hipMemcpyAsync(m.mob, a.data(), a.size() * sizeof(MobArgs), hipMemcpyHostToDevice,
                         h->st));
   HIPCHK(hipStreamSynchronize(h->st));
@@ -2069,9 +2117,8 @@ int mr_mob_args(dwfgpu_s* h, const double* masses, MrState<P>& m) {
 // batched Mobius MatPcDagMatPc: the four hop passes, each one launch for all
 // RHS (k_mobius_mrhs; the M5^-1 and (b + c D5) epilogues keep every s-column
 // of a site in one work-group's LDS, so RHS share a launch but not a
-// work-group).  cg: the CG step of every active RHS (r -= alpha A p,
-// x += alpha p in the last pass, alpha and |r|^2 on the device) instead of
-// `out`.  12^4 Ls 12, 4 RHS, int16: the passes of a step 198 -> 124 us against a launch per
+// work-group).  cg: the CG step of every active RHS (r -= alpha A p, alpha on
+// the device, |r|^2 partials) instead of `out`.  12^4 Ls 12, 4 RHS, int16: the passes of a step 198 -> 124 us against a launch per
 // RHS and pass, a batched MatInv 61 -> 48.5 ms.
 template <class P>
 int mr_mdagm_mob(dwfgpu_s* h, const MrState<P>& m, const DVec& out, const DVec& in, double* scal,
@@ -2085,27 +2132,28 @@ int mr_mdagm_mob(dwfgpu_s* h, const MrState<P>& m, const DVec& out, const DVec& 
   Geom fwd = h->g, back = h->g;
   back.rev = 1;  // the Schur passes, as in Ops::mob()
   bool split;
-#define MOB_MR(DAG, EPI, FL, PX, OUT, IN, PSI, GEOM, CG)                                            hipLaunchKernelGGL((k_mobius_mrhs<P, DAG, EPI, FL, PX>), grid, block,                                                O::mob_lds(h, DAG, EPI, FL, &split), h->st, fld<P>(OUT), cfld<P>(IN),                             cfld<P>(PSI), u, m.partial, GEOM, EPI == EPI_SCHUR ? 1 : 0,                                       m.mob + DAG * nrhs, m.active(), vs, CG, MR_NSCAL)
-  const CgEpi<P, P> none{};
+#define MOB_MR(DAG, EPI, FL, OUT, IN, PSI, GEOM)                                           \
+  hipLaunchKernelGGL((k_mobius_mrhs<P, DAG, EPI, FL>), grid, block,                        \
+                     O::mob_lds(h, DAG, EPI, FL, &split), h->st, fld<P>(OUT), cfld<P>(IN), \
+                     cfld<P>(PSI), u, m.partial, GEOM, EPI == EPI_SCHUR ? 1 : 0,           \
+                     m.mob + DAG * nrhs, m.active(), vs, step, MR_NSCAL)
+  const CgEpi<P, NoX> step{fld<P>(m.rs), CFld<P>{}, Fld<NoX>{}, scal};
   O::mob_lds(h, 0, EPI_M5INV, FL_POST_T, &split);
   if (split) {
     if constexpr (MobSplitT<P>::value)
-      MOB_MR(0, EPI_M5INV, FL_POST_T | FL_SPLIT_T, P, m.te, in, DVec(), fwd, none);
+      MOB_MR(0, EPI_M5INV, FL_POST_T | FL_SPLIT_T, m.te, in, DVec(), fwd);
   } else {
-    MOB_MR(0, EPI_M5INV, FL_POST_T, P, m.te, in, DVec(), fwd, none);
+    MOB_MR(0, EPI_M5INV, FL_POST_T, m.te, in, DVec(), fwd);
   }
-  MOB_MR(0, EPI_SCHUR, FL_PRE_T | FL_NORM, P, m.t1, m.te, in, back, none);
+  MOB_MR(0, EPI_SCHUR, FL_PRE_T | FL_NORM, m.t1, m.te, in, back);
   if (scal)
     hipLaunchKernelGGL(k_reduce_mrhs, dim3(nrhs), dim3(1024), 0, h->st, m.partial, gx, scal,
                        (int)MR_D, m.active());
-  MOB_MR(1, EPI_M5INV, 0, P, m.te, m.t1, DVec(), fwd, none);
+  MOB_MR(1, EPI_M5INV, 0, m.te, m.t1, DVec(), fwd);
   if (cg) {
-    const CgEpi<P, P32> step{fld<P>(m.rs), cfld<P>(in), fld<P32>(m.xs), scal};
-    MOB_MR(1, EPI_SCHUR, FL_CG, P32, m.te, m.te, m.t1, back, step);
-    hipLaunchKernelGGL(k_reduce_mrhs, dim3(nrhs), dim3(1024), 0, h->st, m.partial, gx, scal,
-                       (int)MR_RRNEW, m.active());
+    MOB_MR(1, EPI_SCHUR, FL_CG, m.te, m.te, m.t1, back);
   } else {
-    MOB_MR(1, EPI_SCHUR, 0, P, out, m.te, m.t1, back, none);
+    MOB_MR(1, EPI_SCHUR, 0, out, m.te, m.t1, back);
   }
 #undef MOB_MR
   HIPCHK(hipGetLastError());
@@ -2144,7 +2192,8 @@ int mr_pinned(const dwfgpu_s* h, int nrhs, size_t creal, MrShape* t) {
 // for every candidate shape, twice, and keep the fastest; cached per handle,
 // sloppy precision and RHS count.
 template <class P>
-int mr_tune(dwfgpu_s* h, int nrhs, MrState<P>& m, const int* all_active, MrShape* best) {
+int mr_tune(dwfgpu_s* h, const MrState<P>& m, MrShape* best) {
+  const int nrhs = m.nrhs;
   const int pi = pidx<P>();
   if (h->mr_ns[pi] && h->mr_nrhs[pi] == nrhs) {
     *best = MrShape{h->mr_ns[pi], h->mr_nr[pi]};
@@ -2177,8 +2226,7 @@ int mr_tune(dwfgpu_s* h, int nrhs, MrState<P>& m, const int* all_active, MrShape
     for (int rep = 0; rep < 3 && !st; ++rep) {
       if (hipEventRecord(e0, h->st) != hipSuccess) st = DWFGPU_HIP_ERROR;
       if (!st)
-        st = mr_mdagm<P>(h, t, nrhs, m.rs, m.ps, m.te, m.t1, m.mass, all_active, m.partial, nullptr,
-                         nullptr, nullptr, false);
+        st = mr_mdagm<P>(h, t, m, m.rs, m.ps[0], nullptr, false);
       if (!st && (hipEventRecord(e1, h->st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess))
         st = DWFGPU_HIP_ERROR;
       float ms = 0;
@@ -2215,17 +2263,7 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
   const DVec& r = h->f[DWFGPU_F64].work[0];
   const DVec& ax = h->f[DWFGPU_F64].work[1];
   MrState<PS> m;
-  m.nrhs = nrhs;
-  m.gx = mr_partials_stride(h);
-  TRY(alloc_mvec<PS>(h, nrhs, &m.te));
-  TRY(alloc_mvec<PS>(h, nrhs, &m.t1));
-  TRY(alloc_mvec<PS>(h, nrhs, &m.rs));
-  TRY(alloc_mvec<PS>(h, nrhs, &m.ps));
-  TRY(alloc_mvec<P32>(h, nrhs, &m.xs));
-  TRY(alloc(h, (void**)&m.partial, (size_t)nrhs * m.gx * sizeof(double)));
-  TRY(alloc(h, (void**)&m.scal, (size_t)nrhs * dwfk::MR_NSCAL * sizeof(double)));
-  TRY(alloc(h, (void**)&m.mass, (size_t)nrhs * sizeof(double)));
-  TRY(alloc(h, (void**)&m.ibuf, (size_t)3 * nrhs * sizeof(int)));
+  TRY(m.create(h, nrhs, mr_partials_stride(h), true));
   HIPCHK(hipMemcpyAsync(m.mass, masses, nrhs * sizeof(double), hipMemcpyHostToDevice, h->st));
 
   std::vector<double> sc((size_t)nrhs * dwfk::MR_NSCAL, 0.0), src_nsq(nrhs, 0.0);
@@ -2243,7 +2281,7 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
   }
   MrShape t{h->ns, 1};  // Mobius: the handle's own hop shape, one RHS per work-group
   if (h->action == DWFGPU_DWF)
-    TRY(mr_tune<PS>(h, nrhs, m, m.active(), &t));
+    TRY(mr_tune<PS>(h, m, &t));
   else
     TRY(mr_mob_args<PS>(h, masses, m));
   h->mr_last_ns = t.ns;
@@ -2270,45 +2308,59 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
       if (rr > stp) status[j] = DWFGPU_MAXITER;
       continue;
     }
-    const DVec rsj = mslice<PS>(h, m.rs, j), psj = mslice<PS>(h, m.ps, j);
+    const DVec rsj = mslice<PS>(h, m.rs, j), psj = mslice<PS>(h, m.ps[0], j);
     hipLaunchKernelGGL((dwfk::k_convert<PS, P64>), blas_grid(), blas_block(), 0, h->st, fld<PS>(rsj),
                        cfld<P64>(r), g);
     HIPCHK(hipGetLastError());
     TRY(L::copy(h, psj, rsj));
     act[j] = 1;
   }
-  HIPCHK(hipMemsetAsync(m.xs.d, 0, (size_t)nrhs * (h->n / 2) * sizeof(cx<float>), h->st));
   HIPCHK(hipMemcpyAsync(m.scal, sc.data(), sc.size() * sizeof(double), hipMemcpyHostToDevice, h->st));
   HIPCHK(hipMemcpyAsync(m.ibuf, act.data(), nrhs * sizeof(int), hipMemcpyHostToDevice, h->st));
   HIPCHK(hipMemcpyAsync(m.flag(), flg.data(), nrhs * sizeof(int), hipMemcpyHostToDevice, h->st));
   HIPCHK(hipMemcpyAsync(m.iters(), its.data(), nrhs * sizeof(int), hipMemcpyHostToDevice, h->st));
 
+  // step k of a round: its direction is in slot k % nring.  The steps' updates
+  // of xs are applied together before slot 0 is written again, at the end of the
+  // round (without a ring: of the step)
   const size_t vs = h->n / 2 / PS::kCPC;
-  auto step = [&]() -> int {
+  const int nring = m.nring, gx = h->action == DWFGPU_DWF ? (g.vh + t.ns - 1) / t.ns : h->grid_hop;
+  dwfk::XFlush<PS> xf;
+  xf.cnt = nring;
+  xf.alpha = m.alpha;
+  for (int q = 0; q < nring; ++q) {
+    xf.p[q] = (const typename PS::C*)m.ps[q].d;
+    xf.sc[q] = m.ps[q].sc;
+    xf.ai[q] = q;
+  }
+  const dim3 vgrid(dwfk::BLAS_BLOCKS / 4, nrhs);
+  auto step = [&](int k) -> int {
+    const int slot = k % nring, next = (k + 1) % nring;
     if (h->action == DWFGPU_DWF)
-      TRY(mr_mdagm<PS>(h, t, nrhs, DVec(), m.ps, m.te, m.t1, m.mass, m.active(), m.partial,
-                       m.scal, &m.rs, &m.xs, true));
+      TRY(mr_mdagm<PS>(h, t, m, DVec(), m.ps[slot], m.scal, true));
     else
-      TRY(mr_mdagm_mob<PS>(h, m, DVec(), m.ps, m.scal, true));
-    hipLaunchKernelGGL(dwfk::k_cg_scalars_mrhs, dim3(1), dim3(256), 0, h->st, m.scal, m.active(),
-                       m.flag(), m.iters(), nrhs);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL((dwfk::k_xpby_mrhs<PS>), dim3(dwfk::BLAS_BLOCKS / 4, nrhs), blas_block(), 0,
-                       h->st, fld<PS>(m.ps), cfld<PS>(m.rs), m.scal, m.active(), vs, g);
+      TRY(mr_mdagm_mob<PS>(h, m, DVec(), m.ps[slot], m.scal, true));
+    hipLaunchKernelGGL(dwfk::k_cg_end_mrhs, dim3(nrhs), dim3(1024), 0, h->st, m.partial, gx, m.scal,
+                       m.active(), m.flag(), m.iters(), m.alpha, nring, slot);
+    if (next == 0)
+      hipLaunchKernelGGL((dwfk::k_x_flush_mrhs<PS>), vgrid, blas_block(), 0, h->st,
+                         fld<P32>(m.xs), xf, vs, g);
+    hipLaunchKernelGGL((dwfk::k_xpby_mrhs<PS>), vgrid, blas_block(), 0, h->st, fld<PS>(m.ps[next]),
+                       cfld<PS>(m.ps[slot]), cfld<PS>(m.rs), m.scal, m.active(), vs, g);
     HIPCHK(hipGetLastError());
     return DWFGPU_OK;
   };
 
   // K CG steps per host round, captured once into a graph (no memset or
   // copy inside it) unless DWFGPU_MRHS_EAGER asks for plain launches
-  const int K = 4;
+  const int K = MR_RING;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int st = DWFGPU_OK;
   if (!(flags & DWFGPU_MRHS_EAGER)) {
     HIPCHK(hipStreamSynchronize(h->st));
     HIPCHK(hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < K && !st; ++k) st = step();
+    for (int k = 0; k < K && !st; ++k) st = step(k);
     hipGraph_t gcap = nullptr;
     const hipError_t ec = hipStreamEndCapture(h->st, &gcap);
     if (st || ec != hipSuccess) {
@@ -2336,7 +2388,7 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
     if (exec) {
       if (hipGraphLaunch(exec, h->st) != hipSuccess) st = DWFGPU_HIP_ERROR;
     } else {
-      for (int k = 0; k < K && !st; ++k) st = step();
+      for (int k = 0; k < K && !st; ++k) st = step(k);
     }
     if (st) break;
     std::vector<int> ib(3 * nrhs);
@@ -2350,6 +2402,7 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
     }
     bool changed = false;
     for (int j = 0; j < nrhs && !st; ++j) {
+      const int ran = ib[2 * nrhs + j] - its[j];  // its steps of this round
       act[j] = ib[j];
       flg[j] = ib[nrhs + j];
       its[j] = ib[2 * nrhs + j];
@@ -2357,7 +2410,8 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
       changed = true;
       double* sj = &sc[(size_t)j * dwfk::MR_NSCAL];
       const DVec xj = mslice<P64>(h, sol, j), bj = mslice<P64>(h, src, j);
-      const DVec rsj = mslice<PS>(h, m.rs, j), psj = mslice<PS>(h, m.ps, j);
+      const DVec rsj = mslice<PS>(h, m.rs, j), psj = mslice<PS>(h, m.ps[0], j);
+      const DVec last = mslice<PS>(h, m.ps[(ran - 1) % nring], j);  // its latest direction
       const DVec xsj = mslice<P32>(h, m.xs, j);
       if (flg[j] == 2) {  // <p, A p> == 0: CPS's breakdown
         status[j] = DWFGPU_BREAKDOWN;
@@ -2384,12 +2438,12 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
         flg[j] = 0;
         continue;
       }
-      // continue: r_s = r, p_s = r_s + beta' p_s with beta' = rr / rr_prev
+      // continue: r_s = r, p_s = r_s + beta' (its latest p_s) with beta' = rr / rr_prev
       hipLaunchKernelGGL((dwfk::k_convert<PS, P64>), blas_grid(), blas_block(), 0, h->st,
                          fld<PS>(rsj), cfld<P64>(r), g);
       if (hipGetLastError() != hipSuccess) st = DWFGPU_HIP_ERROR;
       const double beta = sj[dwfk::MR_BETA] * rr / sj[dwfk::MR_RR];
-      if (!st) st = L::axpby(h, psj, rsj, 1.0, beta);
+      if (!st) st = L::axpy_to(h, psj, last, rsj, beta, false);
       sj[dwfk::MR_RR] = rr;
       sj[dwfk::MR_RRUPD] = rr;
       act[j] = 1;
@@ -4025,21 +4079,13 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
     typedef decltype(tag) P;
     TRY(ensure_fields<P>(h));
     MrState<P> m;
-    m.nrhs = nrhs;
-    m.gx = mr_partials_stride(h);
-    TRY(alloc_mvec<P>(h, nrhs, &m.te));
-    TRY(alloc_mvec<P>(h, nrhs, &m.t1));
-    TRY(alloc_mvec<P>(h, nrhs, &m.rs));
-    TRY(alloc_mvec<P>(h, nrhs, &m.ps));
-    TRY(alloc(h, (void**)&m.partial, (size_t)nrhs * m.gx * sizeof(double)));
-    TRY(alloc(h, (void**)&m.mass, (size_t)nrhs * sizeof(double)));
-    TRY(alloc(h, (void**)&m.ibuf, (size_t)3 * nrhs * sizeof(int)));
+    TRY(m.create(h, nrhs, mr_partials_stride(h), false));
     std::vector<int> ones(nrhs, 1);
     HIPCHK(hipMemcpyAsync(m.ibuf, ones.data(), nrhs * sizeof(int), hipMemcpyHostToDevice, h->st));
     HIPCHK(hipMemcpyAsync(m.mass, masses, nrhs * sizeof(double), hipMemcpyHostToDevice, h->st));
     for (int j = 0; j < nrhs; ++j)
       hipLaunchKernelGGL((dwfk::k_convert<P, P64>), blas_grid(), blas_block(), 0, h->st,
-                         fld<P>(mslice<P>(h, m.ps, j)), cfld<P64>(mslice<P64>(h, in->v, j)), h->g);
+                         fld<P>(mslice<P>(h, m.ps[0], j)), cfld<P64>(mslice<P64>(h, in->v, j)), h->g);
     HIPCHK(hipGetLastError());
     MrShape t{h->ns, 1};
     if (h->action == DWFGPU_DWF && pidx<P>() == DWFGPU_F64 && h->ns64) {
@@ -4048,7 +4094,7 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
       const double mk2 = -dwf_kappa(h) * dwf_kappa(h);
       Geom fwd = h->g, back = h->g;
       back.rev = 1;
-      cx<double> *in = (cx<double>*)m.ps.d, *out = (cx<double>*)m.rs.d;
+      cx<double> *in = (cx<double>*)m.ps[0].d, *out = (cx<double>*)m.rs.d;
       cx<double> *te = (cx<double>*)m.te.d, *t1 = (cx<double>*)m.t1.d;
       auto pass = [&](const Geom& g, cx<double>* o, cx<double>* i, cx<double>* x0, int dag) {
         return dwf64(h, g, o, i, x0, x0 ? 0 : 1, dag, x0 ? 1 : 0, false, 0.0, x0 ? mk2 : 0.0,
@@ -4059,15 +4105,14 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
       TRY(pass(fwd, te, t1, nullptr, 1));
       TRY(pass(back, out, te, t1, 1));
     } else if (h->action == DWFGPU_DWF) {
-      TRY(mr_tune<P>(h, nrhs, m, m.active(), &t));
-      TRY(mr_mdagm<P>(h, t, nrhs, m.rs, m.ps, m.te, m.t1, m.mass, m.active(), m.partial,
-                      nullptr, nullptr, nullptr, false));
+      TRY(mr_tune<P>(h, m, &t));
+      TRY(mr_mdagm<P>(h, t, m, m.rs, m.ps[0], nullptr, false));
     } else if (pidx<P>() == DWFGPU_F64 && h->ns64) {  // as a single right-hand side
       for (int j = 0; j < nrhs; ++j)
-        TRY(Ops<P>::mdagm(h, masses[j], mslice<P>(h, m.rs, j), mslice<P>(h, m.ps, j), nullptr));
+        TRY(Ops<P>::mdagm(h, masses[j], mslice<P>(h, m.rs, j), mslice<P>(h, m.ps[0], j), nullptr));
     } else {
       TRY(mr_mob_args<P>(h, masses, m));
-      TRY(mr_mdagm_mob<P>(h, m, m.rs, m.ps, nullptr, false));
+      TRY(mr_mdagm_mob<P>(h, m, m.rs, m.ps[0], nullptr, false));
     }
     h->mr_last_ns = t.ns;
     h->mr_last_nr = t.nr;

@@ -1561,24 +1561,21 @@ __device__ __forceinline__ CFld<P> fld_at(CFld<P> f, size_t vs, size_t vss, int 
 // 12^4 Ls 12 vector is 648 work-groups, less than the chip holds at once:
 // launched one after the other, each waited for the last work-groups of the
 // one before.
-template <class P, int DAG, int EPI, int FL, class PX = P>
+template <class P, int DAG, int EPI, int FL>
 __global__ void __launch_bounds__(512)
 k_mobius_mrhs(Fld<P> out, CFld<P> in, CFld<P> psi, const typename P::S* __restrict__ U,
               double* __restrict__ partial, Geom g, int p_out, const MobArgs* __restrict__ args,
-              const int* __restrict__ active, size_t vs, CgEpi<P, PX> cg, int cg_stride) {
+              const int* __restrict__ active, size_t vs, CgEpi<P, NoX> cg, int cg_stride) {
   const int j = blockIdx.y;
   if (!active[j]) return;  // uniform: before any barrier
   const size_t vss = (size_t)g.vh * g.ls;
   if constexpr ((FL & FL_CG) != 0) {
     cg.r = fld_at(cg.r, vs, vss, j);
-    cg.p = fld_at(cg.p, vs, vss, j);
-    if constexpr (!std::is_same<PX, NoX>::value)
-      cg.x = fld_at(cg.x, vs * nch<PX>() / nch<P>(), vss, j);
     cg.scal += (size_t)j * cg_stride;
   }
-  mobius_pass<P, DAG, EPI, FL, PX>(fld_at(out, vs, vss, j), fld_at(in, vs, vss, j),
-                                   fld_at(psi, vs, vss, j), U,
-                                   partial + (size_t)j * gridDim.x, g, p_out, args[j], cg);
+  mobius_pass<P, DAG, EPI, FL, NoX>(fld_at(out, vs, vss, j), fld_at(in, vs, vss, j),
+                                    fld_at(psi, vs, vss, j), U,
+                                    partial + (size_t)j * gridDim.x, g, p_out, args[j], cg);
 }
 
 // stand-alone M5^-1 (dag) on a half vector: zmobius_m5inv(out, in, ...)
@@ -1781,8 +1778,9 @@ struct XFlush {
   int cnt;
 };
 template <class P, class PX>
-__global__ void __launch_bounds__(BLAS_THREADS)
-k_x_flush(Fld<PX> x, XFlush<P> f, Geom g) {
+__device__ __forceinline__ void x_flush(const Fld<PX>& x, const XFlush<P>& f, const Geom& g,
+                                        const double* __restrict__ alpha, size_t off = 0,
+                                        size_t soff = 0) {
   typedef typename P::R R;
   typedef typename PX::R RX;
   if constexpr (!P::kScaled && std::is_same<P, PX>::value) {
@@ -1795,11 +1793,11 @@ k_x_flush(Fld<PX> x, XFlush<P> f, Geom g) {
         cx<R> pv[4][P::kCPC];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-          if (j + u < f.cnt) ld_chunk<P>(f.p[j + u] + e, pv[u]);
+          if (j + u < f.cnt) ld_chunk<P>(f.p[j + u] + off + e, pv[u]);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
           if (j + u < f.cnt) {
-            const double a = f.alpha[f.ai[j + u]];
+            const double a = alpha[f.ai[j + u]];
 #pragma unroll
             for (int c = 0; c < P::kCPC; ++c)
               xv[c] = cx<R>{(R)(a * pv[u][c].re) + xv[c].re, (R)(a * pv[u][c].im) + xv[c].im};
@@ -1814,14 +1812,19 @@ k_x_flush(Fld<PX> x, XFlush<P> f, Geom g) {
     ld_site<PX>(xv, CFld<PX>{x.d, x.sc}, g, k);
     for (int j = 0; j < f.cnt; ++j) {
       cx<R> pv[12];
-      ld_site<P>(pv, CFld<P>{f.p[j], f.sc[j]}, g, k);
-      const double a = f.alpha[f.ai[j]];
+      ld_site<P>(pv, CFld<P>{f.p[j] + off, f.sc[j] + soff}, g, k);
+      const double a = alpha[f.ai[j]];
 #pragma unroll
       for (int c = 0; c < 12; ++c)
         xv[c] = cx<RX>{(RX)(a * pv[c].re) + xv[c].re, (RX)(a * pv[c].im) + xv[c].im};
     }
     st_site_k<PX>(x, g, k, xv);
   }
+}
+template <class P, class PX>
+__global__ void __launch_bounds__(BLAS_THREADS)
+k_x_flush(Fld<PX> x, XFlush<P> f, Geom g) {
+  x_flush<P, PX>(x, f, g, f.alpha);
 }
 
 // z = a x + y, partial |z|^2 optional
@@ -2325,7 +2328,7 @@ constexpr int MR_NSCAL = 8;
 enum { MR_RR = 0, MR_D = 1, MR_RRNEW = 2, MR_BETA = 3, MR_STOP = 4, MR_RRUPD = 5, MR_DELTA2 = 6,
        MR_MAXIT = 7 };
 
-template <class P, class PX>
+template <class P>
 struct MrArgs {
   Fld<P> out;
   CFld<P> in;
@@ -2339,10 +2342,8 @@ struct MrArgs {
   const int* active;   // [nrhs]
   size_t vs;           // chunks per vector
   int nrhs;
-  // CG epilogue (x in PX)
+  // CG epilogue
   Fld<P> r;
-  CFld<P> p;
-  Fld<PX> x;
   double* scal;  // [nrhs][MR_NSCAL]
 };
 
@@ -2364,8 +2365,8 @@ __device__ __forceinline__ double zslice_sum(double v, double* red) {
   return my[0];
 }
 
-template <class P, int DAG, int EPI, bool NORM, bool CG, class PX>
-__global__ void __launch_bounds__(512) k_dwf_mrhs(MrArgs<P, PX> a) {
+template <class P, int DAG, int EPI, bool NORM, bool CG>
+__global__ void __launch_bounds__(512) k_dwf_mrhs(MrArgs<P> a) {
   typedef typename P::R R;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const Geom& g = a.g;
@@ -2431,10 +2432,9 @@ __global__ void __launch_bounds__(512) k_dwf_mrhs(MrArgs<P, PX> a) {
       for (int c = 0; c < 12; ++c) acc[c] = xv[c] + al * acc[c];
       if (NORM) nrm = norm12(acc);
       if (CG) {
-        const CgEpi<P, PX> cg{fld_at(a.r, a.vs, vss, j), fld_at(a.p, a.vs, vss, j),
-                              fld_at(a.x, a.vs * nch<PX>() / nch<P>(), vss, j),
-                              a.scal + (size_t)j * MR_NSCAL};
-        nrm = cg_epilogue<P, PX>(cg, g, s, i, acc, a_cg);
+        const CgEpi<P, NoX> cg{fld_at(a.r, a.vs, vss, j), CFld<P>{}, Fld<NoX>{},
+                               a.scal + (size_t)j * MR_NSCAL};
+        nrm = cg_epilogue<P, NoX>(cg, g, s, i, acc, a_cg);
       }
     }
     if (!CG) {
@@ -2448,6 +2448,18 @@ __global__ void __launch_bounds__(512) k_dwf_mrhs(MrArgs<P, PX> a) {
   }
 }
 
+// sum of p[0..n) by a work-group of 1024; valid in thread 0
+__device__ __forceinline__ double partial_sum(const double* __restrict__ p, int n, double* sh) {
+  double a0 = 0.0, a1 = 0.0;
+  int k = threadIdx.x;
+  for (; k + 1024 < n; k += 2048) {
+    a0 += p[k];
+    a1 += p[k + 1024];
+  }
+  for (; k < n; k += 1024) a0 += p[k];
+  return block_sum(a0 + a1, sh);
+}
+
 // scal[j][slot] = sum of partial[j][0..n) for every RHS (one work-group each)
 __global__ void __launch_bounds__(1024)
 k_reduce_mrhs(const double* __restrict__ partial, int n, double* __restrict__ scal, int slot,
@@ -2455,67 +2467,85 @@ k_reduce_mrhs(const double* __restrict__ partial, int n, double* __restrict__ sc
   __shared__ double sh[16];
   const int j = blockIdx.x;
   if (!active[j]) return;
-  const double* pj = partial + (size_t)j * n;
-  double a0 = 0.0, a1 = 0.0;
-  int k = threadIdx.x;
-  for (; k + 1024 < n; k += 2048) {
-    a0 += pj[k];
-    a1 += pj[k + 1024];
-  }
-  for (; k < n; k += 1024) a0 += pj[k];
-  const double t = block_sum(a0 + a1, sh);
+  const double t = partial_sum(partial + (size_t)j * n, n, sh);
   if (threadIdx.x == 0) scal[(size_t)j * MR_NSCAL + slot] = t;
 }
 
-// end of a CG step for every active RHS: beta = rr_new / rr, rr = rr_new;
-// an RHS whose residual meets its stop condition, or has dropped by delta
-// since its last reliable update, pauses (active = 0) and raises flag = 1 for
-// the host; <p, A p> == 0 pauses it with flag = 2, reaching the iteration
-// cap with flag = 3.
-__global__ void __launch_bounds__(256)
-k_cg_scalars_mrhs(double* __restrict__ scal, int* __restrict__ active, int* __restrict__ flag,
-                  int* __restrict__ iters, int nrhs) {
-  for (int j = threadIdx.x; j < nrhs; j += blockDim.x) {
-    if (!active[j]) continue;
-    double* sc = scal + (size_t)j * MR_NSCAL;
-    iters[j] += 1;
-    if (sc[MR_D] == 0.0) {
-      active[j] = 0;
-      flag[j] = 2;
-      continue;
-    }
-    const double rrn = sc[MR_RRNEW];
-    sc[MR_BETA] = rrn / sc[MR_RR];
-    sc[MR_RR] = rrn;
-    if (rrn <= sc[MR_STOP] || rrn < sc[MR_DELTA2] * sc[MR_RRUPD]) {
-      active[j] = 0;
-      flag[j] = 1;
-    } else if (iters[j] >= (int)sc[MR_MAXIT]) {
-      active[j] = 0;
-      flag[j] = 3;
-    }
+// end of a CG step for every active RHS (one work-group each): rr_new of the
+// partials, beta = rr_new / rr, rr = rr_new, alpha[j][slot] of the step (0 for a
+// paused RHS) for k_x_flush_mrhs; an RHS whose residual meets its stop
+// condition, or has dropped by delta since its last reliable update, pauses
+// (active = 0) and raises flag = 1 for the host; <p, A p> == 0 pauses it with
+// flag = 2, reaching the iteration cap with flag = 3.
+__global__ void __launch_bounds__(1024)
+k_cg_end_mrhs(const double* __restrict__ partial, int n, double* __restrict__ scal,
+              int* __restrict__ active, int* __restrict__ flag, int* __restrict__ iters,
+              double* __restrict__ alpha, int nslot, int slot) {
+  __shared__ double sh[16];
+  const int j = blockIdx.x;
+  if (!active[j]) {  // uniform: every thread reads it before thread 0 changes it
+    if (threadIdx.x == 0) alpha[(size_t)j * nslot + slot] = 0.0;
+    return;
+  }
+  const double rrn = partial_sum(partial + (size_t)j * n, n, sh);
+  if (threadIdx.x) return;
+  double* sc = scal + (size_t)j * MR_NSCAL;
+  alpha[(size_t)j * nslot + slot] = cg_alpha(sc);
+  sc[MR_RRNEW] = rrn;
+  iters[j] += 1;
+  if (sc[MR_D] == 0.0) {
+    active[j] = 0;
+    flag[j] = 2;
+    return;
+  }
+  sc[MR_BETA] = rrn / sc[MR_RR];
+  sc[MR_RR] = rrn;
+  if (rrn <= sc[MR_STOP] || rrn < sc[MR_DELTA2] * sc[MR_RRUPD]) {
+    active[j] = 0;
+    flag[j] = 1;
+  } else if (iters[j] >= (int)sc[MR_MAXIT]) {
+    active[j] = 0;
+    flag[j] = 3;
   }
 }
 
-// p_j = r_j + beta_j p_j for every active RHS (blockIdx.y = RHS)
+// x_j += sum over the slots of alpha[j][slot] p_slot,j: the steps of a round in
+// one pass over x (f.cnt slots, f.p / f.sc those of the first RHS).  DWF
+// 8^3x32 Ls 12, 12 RHS, FP32: the last pass of a step 166 -> 109 us without
+// x += alpha p in it, this one 27 us a step (5.3 TB/s); int16 Moebius 12^4
+// Ls 12, 4 RHS: 42 -> 29 us and 7.6.
 template <class P>
 __global__ void __launch_bounds__(BLAS_THREADS)
-k_xpby_mrhs(Fld<P> p, CFld<P> r, const double* __restrict__ scal, const int* __restrict__ active,
+k_x_flush_mrhs(Fld<P32> x, XFlush<P> f, size_t vs, Geom g) {
+  const int j = blockIdx.y;
+  const size_t vss = (size_t)g.vh * g.ls;
+  const double* alpha = f.alpha + (size_t)j * f.cnt;
+  bool any = false;
+  for (int q = 0; q < f.cnt; ++q) any = any || alpha[q] != 0.0;
+  if (!any) return;  // paused all the round
+  x_flush<P, P32>(fld_at(x, vs * nch<P32>() / nch<P>(), vss, j), f, g, alpha, j * vs,
+                  P::kScaled ? j * vss : 0);
+}
+
+// pn_j = r_j + beta_j p_j for every active RHS (blockIdx.y = RHS); pn may be p
+template <class P>
+__global__ void __launch_bounds__(BLAS_THREADS)
+k_xpby_mrhs(Fld<P> pn, CFld<P> p, CFld<P> r, const double* __restrict__ scal, const int* __restrict__ active,
             size_t vs, Geom g) {
   typedef typename P::R R;
   const int j = blockIdx.y;
   if (!active[j]) return;
   const size_t vss = (size_t)g.vh * g.ls;
-  const Fld<P> pj = fld_at(p, vs, vss, j);
-  const CFld<P> rj = fld_at(r, vs, vss, j);
+  const Fld<P> nj = fld_at(pn, vs, vss, j);
+  const CFld<P> pj = fld_at(p, vs, vss, j), rj = fld_at(r, vs, vss, j);
   const R b = (R)scal[(size_t)j * MR_NSCAL + MR_BETA];
   DWFK_SITE_LOOP(k, g) {
     cx<R> pv[12], rv[12];
-    ld_site<P>(pv, CFld<P>{pj.d, pj.sc}, g, k);
+    ld_site<P>(pv, pj, g, k);
     ld_site<P>(rv, rj, g, k);
 #pragma unroll
     for (int c = 0; c < 12; ++c) pv[c] = rv[c] + b * pv[c];
-    st_site_k<P>(pj, g, k, pv);
+    st_site_k<P>(nj, g, k, pv);
   }
 }
 
