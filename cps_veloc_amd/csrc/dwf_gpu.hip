@@ -101,11 +101,12 @@ struct dwfgpu_s {
   double* hscal = nullptr;   // pinned
   double* dalpha = nullptr;  // alphas of the pending sloppy CG steps (device)
   double* hring = nullptr;   // pinned copies of the sloppy CG scalars, per step
-  int grid_hop = 0;
+  int grid_hop = 0;  // their most work-groups in any format
   // the small-lattice FP64 hop kernels (hop64.hpp): sites per work-group (0:
   // this lattice takes the general ones) and work-groups
   int ns64 = 0, grid64 = 0;
-  int ns = 16;  // sites per work-group of the hopping kernels (x); y = all slices
+  // sites per work-group of the hopping kernels (x; y = all slices), per format
+  int ns[NPREC] = {16, 16, 16, 16};
   int max_lds = 65536;
   // launch shape of the many-RHS operator chosen by the autotuner, per
   // sloppy precision and RHS count (0: not tuned yet)
@@ -252,18 +253,53 @@ MobArgs mob_args(const dwfgpu_s* h, double mass, int dag) {
 }
 
 // LDS of the s-column buffer (M5^-1 and (b + c D5)^dag epilogues)
-size_t col_lds_bytes(const dwfgpu_s* h, size_t creal) {
-  return (size_t)h->ns * (h->ls * 12 + 1) * 2 * creal;
+size_t col_lds_bytes(int ns, int ls, size_t creal) {
+  return (size_t)ns * (ls * 12 + 1) * 2 * creal;
 }
 // LDS of the staged links and neighbour indices: nsets parities x 8
 // directions x ns sites x (9 complex + 1 int)
-size_t link_lds_bytes(const dwfgpu_s* h, int nsets, size_t creal) {
-  return (size_t)nsets * 8 * h->ns * (9 * 2 * creal + 4);
+size_t link_lds_bytes(int ns, int nsets, size_t creal) {
+  return (size_t)nsets * 8 * ns * (9 * 2 * creal + 4);
 }
-// largest LDS request of any kernel of this handle (FP64 compute is the widest)
-size_t max_lds_bytes(const dwfgpu_s* h) {
-  return h->action == DWFGPU_DWF ? link_lds_bytes(h, 2, 8)
-                                 : std::max(link_lds_bytes(h, 1, 8), col_lds_bytes(h, 8));
+// largest LDS request of a hop kernel with ns sites a work-group
+size_t hop_lds_bytes(int action, int ls, int ns, size_t creal) {
+  return action == DWFGPU_DWF ? link_lds_bytes(ns, 2, creal)
+                              : std::max(link_lds_bytes(ns, 1, creal), col_lds_bytes(ns, ls, creal));
+}
+
+// Sites per work-group of the general hop kernels in format `prec`, found by
+// timing MatPcDagMatPc (ms with 16 / the sites taken):
+//   DWF, whose work-groups only meet at the staged links: FP64 32, or 64 to Ls 8
+//     (24^3x64 Ls 12 4.20 / 3.75, 16^3x32 Ls 16 0.804 / 0.740, Ls 8 0.444 /
+//     0.417): rows of 512 bytes and more from one work-group.  FP32 the shape of
+//     eight whole waves (16^3x32 Ls 16 0.342 / 0.332, 24^3x64 Ls 8 1.32 / 1.19);
+//     where Ls leaves fewer (Ls 10, 12) two such work-groups waste the wave slots
+//     they do not fill (0.108 / 0.112), and 16 stays.  16 bits 16 above Ls 8
+//     (24^3x64 Ls 12 1.18 / 1.30 with 32), 32 to it (16^3x32 Ls 8 0.130 / 0.124)
+//     and 64 to Ls 4 (0.117 / 0.104).
+//   Moebius, whose s-columns take LDS and more barriers: four waves, so 32 for
+//     Ls 5 to 8 (24^3x64 Ls 8 FP64 2.50 / 2.42, FP32 1.20 / 1.15; 16^3x32 Ls 6
+//     int16 0.137 / 0.124), 16 otherwise (24^3x64 Ls 12 3.68 / 4.00, Ls 4 0.248 /
+//     0.251).
+// Never so many that the fullest CU gets more sites than with 16 (12^4 Ls 12
+// DWF FP64, 324 work-groups of 32: 0.125 / 0.141).
+int hop_sites(const dwfgpu_s* h, int prec, int ncu) {
+  const int ls = h->ls;
+  int ns = 16;
+  if (h->action != DWFGPU_DWF)
+    ns = ls > 4 && ls <= 8 ? 32 : 16;
+  else if (prec == DWFGPU_F64)
+    ns = ls <= 8 ? 64 : 32;
+  else if (prec == DWFGPU_F32 && (ls == 8 || ls == 16))
+    ns = 512 / ls;
+  else
+    ns = ls <= 4 ? 64 : ls <= 8 ? 32 : 16;
+  auto fullest = [&](int n) { return ((h->g.vh + n - 1) / n + ncu - 1) / ncu * n; };
+  const size_t creal = prec == DWFGPU_F64 ? 8 : 4;
+  while (ns > 4 && (ns * ls > 512 || hop_lds_bytes(h->action, ls, ns, creal) > (size_t)h->max_lds ||
+                    (ns > 16 && fullest(ns) > fullest(16))))
+    ns /= 2;
+  return ns;
 }
 
 // ---------------------------------------------------------------------------
@@ -493,12 +529,15 @@ struct Ops {
   typedef typename P::R R;
   typedef typename P::S S;
   static PrecFields& F(dwfgpu_s* h) { return h->f[pidx<P>()]; }
+  // sites per work-group and work-groups of the general hop kernels
+  static int sites(const dwfgpu_s* h) { return h->ns[pidx<P>()]; }
+  static int groups(const dwfgpu_s* h) { return (h->g.vh + sites(h) - 1) / sites(h); }
 
   // DWF hop kernel: epi 0 -> out = D in ; epi 1 -> out = x0 + alpha D in
   static int dwf(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, int cb_in, int dag,
                  int epi, const DVec& x0, double alpha, bool norm, double* partial = nullptr) {
     if (!partial) partial = h->partial;
-    const dim3 grid(h->grid_hop), block(h->ns, h->ls);
+    const dim3 grid(groups(h)), block(sites(h), h->ls);
     const double two_a5 = 2.0 * h->a5inv, nm = -2.0 * mass * h->a5inv;
     const S* u = (const S*)F(h).U;
     Geom gm = h->g;
@@ -507,7 +546,7 @@ struct Ops {
       if (h->ns64)
         return dwf64(h, gm, (cx<double>*)out.d, (const cx<double>*)in.d, (const cx<double>*)x0.d,
                      cb_in, dag, epi, norm, nm, alpha, partial, nullptr, nullptr);
-    const size_t lds = link_lds_bytes(h, 2, sizeof(R));
+    const size_t lds = link_lds_bytes(sites(h), 2, sizeof(R));
 #define DWF_LAUNCH(DAG, EPI, NORM)                                                           \
   hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, DAG, EPI, NORM>), grid, block, lds, h->st,       \
                      fld<P>(out), cfld<P>(in), u, cfld<P>(x0), partial, gm, cb_in, two_a5,    \
@@ -527,22 +566,22 @@ struct Ops {
   // LDS of a Mobius pass, and whether it takes the exchange gather
   static size_t mob_lds(const dwfgpu_s* h, int dag, int epi, int fl, bool* split) {
     const bool col = dag || epi == dwfk::EPI_M5INV || epi == dwfk::EPI_SCHUR;
-    const size_t cols = col ? col_lds_bytes(h, sizeof(R)) : 0;
+    const size_t cols = col ? col_lds_bytes(sites(h), h->ls, sizeof(R)) : 0;
     // exchange slots after the links; the M5^-1 / Schur s-columns reuse the
     // LDS from offset 0 once the hop is done
     const size_t split_lds =
-        std::max(cols, dwfk::split_col_offset<R>(h->ns) +
-                           (size_t)h->ls * h->ns * dwfk::TX_SLOT * 2 * sizeof(R));
+        std::max(cols, dwfk::split_col_offset<R>(sites(h)) +
+                           (size_t)h->ls * sites(h) * dwfk::TX_SLOT * 2 * sizeof(R));
     *split = dwfk::MobSplitT<P>::value && !dag && !(fl & dwfk::FL_PRE_T) &&
              split_lds <= (size_t)h->max_lds;
-    return *split ? split_lds : std::max(link_lds_bytes(h, 1, sizeof(R)), cols);
+    return *split ? split_lds : std::max(link_lds_bytes(sites(h), 1, sizeof(R)), cols);
   }
 
   // Mobius hop kernel; fl: dwfk::FL_* flags
   static int mob(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, const DVec& psi,
                  int p_out, int dag, int epi, int fl, double* partial = nullptr) {
     if (!partial) partial = h->partial;
-    const dim3 grid(h->grid_hop), block(h->ns, h->ls);
+    const dim3 grid(groups(h)), block(sites(h), h->ls);
     const MobArgs a = mob_args(h, mass, dag);
     // the Schur passes sweep backwards: they start on the sites the pass
     // before them wrote last, which the last-level cache still holds
@@ -622,9 +661,9 @@ struct Ops {
         return mob64(h, gm, a, nullptr, (const cx<double>*)te.d, (const cx<double>*)t1.d, 1, 1,
                      dwfk::EPI_SCHUR, dwfk::FL_CG, partial, (cx<double>*)r.d, &cs);
     }
-    const dim3 grid(h->grid_hop), block(h->ns, h->ls);
+    const dim3 grid(groups(h)), block(sites(h), h->ls);
     const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), scal};
-    const size_t lds = std::max(link_lds_bytes(h, 1, sizeof(R)), col_lds_bytes(h, sizeof(R)));
+    const size_t lds = std::max(link_lds_bytes(sites(h), 1, sizeof(R)), col_lds_bytes(sites(h), h->ls, sizeof(R)));
     hipLaunchKernelGGL((dwfk::k_mobius<P, 1, dwfk::EPI_SCHUR, dwfk::FL_CG, PX>), grid, block,
                        lds, h->st, fld<P>(te), cfld<P>(te), cfld<P>(t1), (const S*)F(h).U,
                        partial, gm, 1, a, cg);
@@ -634,13 +673,13 @@ struct Ops {
 
   // work-groups of a hop pass: the partial sums it leaves
   static int grid(const dwfgpu_s* h) {
-    return std::is_same<P, P64>::value && h->ns64 ? h->grid64 : h->grid_hop;
+    return std::is_same<P, P64>::value && h->ns64 ? h->grid64 : groups(h);
   }
 
   static int m5inv(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, int dag) {
-    const dim3 grid(h->grid_hop), block(h->ns, h->ls);
+    const dim3 grid(groups(h)), block(sites(h), h->ls);
     const M5Side k = m5_side(h, mass, dag);
-    const size_t lds = col_lds_bytes(h, sizeof(R));
+    const size_t lds = col_lds_bytes(sites(h), h->ls, sizeof(R));
     if (dag)
       hipLaunchKernelGGL((dwfk::k_m5inv<P, 1>), grid, block, lds, h->st, fld<P>(out), cfld<P>(in),
                          h->g, k);
@@ -716,8 +755,8 @@ struct Ops {
                        false, -2.0 * mass * h->a5inv, mk2, h->partial, (cx<double>*)r.d, &cs);
       }
       const dwfk::CgEpi<P, PX> cg{fld<P>(r), cfld<P>(p), fld<PX>(x), h->dscal};
-      hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, 1, 1, false, true, PX>), dim3(h->grid_hop),
-                         dim3(h->ns, h->ls), link_lds_bytes(h, 2, sizeof(R)), h->st, fld<P>(te),
+      hipLaunchKernelGGL((dwfk::k_dwf_dslash<P, 1, 1, false, true, PX>), dim3(groups(h)),
+                         dim3(sites(h), h->ls), link_lds_bytes(sites(h), 2, sizeof(R)), h->st, fld<P>(te),
                          cfld<P>(te), (const S*)F(h).U, cfld<P>(t1), h->partial, gm, 0,
                          2.0 * h->a5inv, -2.0 * mass * h->a5inv, mk2, cg);
     } else {
@@ -2125,8 +2164,8 @@ int mr_mdagm_mob(dwfgpu_s* h, const MrState<P>& m, const DVec& out, const DVec& 
                  bool cg) {
   typedef Ops<P> O;
   using namespace dwfk;
-  const int nrhs = m.nrhs, gx = h->grid_hop;
-  const dim3 grid(gx, nrhs), block(h->ns, h->ls);
+  const int nrhs = m.nrhs, gx = O::groups(h);
+  const dim3 grid(gx, nrhs), block(O::sites(h), h->ls);
   const size_t vs = h->n / 2 / P::kCPC;
   const typename P::S* u = (const typename P::S*)h->f[pidx<P>()].U;
   Geom fwd = h->g, back = h->g;
@@ -2279,7 +2318,7 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
     std::vector<int> ones(nrhs, 1);
     HIPCHK(hipMemcpyAsync(m.ibuf, ones.data(), nrhs * sizeof(int), hipMemcpyHostToDevice, h->st));
   }
-  MrShape t{h->ns, 1};  // Mobius: the handle's own hop shape, one RHS per work-group
+  MrShape t{L::sites(h), 1};  // Mobius: the handle's own hop shape, one RHS per work-group
   if (h->action == DWFGPU_DWF)
     TRY(mr_tune<PS>(h, m, &t));
   else
@@ -2324,7 +2363,7 @@ int invcg_mrhs(dwfgpu_s* h, const dwfgpu_cg_arg* arg, int nrhs, const double* ma
   // of xs are applied together before slot 0 is written again, at the end of the
   // round (without a ring: of the step)
   const size_t vs = h->n / 2 / PS::kCPC;
-  const int nring = m.nring, gx = h->action == DWFGPU_DWF ? (g.vh + t.ns - 1) / t.ns : h->grid_hop;
+  const int nring = m.nring, gx = h->action == DWFGPU_DWF ? (g.vh + t.ns - 1) / t.ns : L::groups(h);
   dwfk::XFlush<PS> xf;
   xf.cnt = nring;
   xf.alpha = m.alpha;
@@ -3573,24 +3612,31 @@ int dwfgpu_create(const double* gauge, const int dims[4], int ls, int action, do
     delete h;
     return rs;
   }
-  // sites per work-group of the hopping kernels; DWFGPU_NS overrides the
-  // default.  Without an override, fewer sites per work-group are taken when
-  // the LDS stage of a long fifth dimension would not fit.
+  // sites per work-group of the hopping kernels; DWFGPU_NS overrides the rule
+  int ncu = 0;
+  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      ncu < 1) {
+    set_err("dwfgpu_create: no compute-unit count of device %d", dev);
+    delete h;
+    return DWFGPU_HIP_ERROR;
+  }
   const char* env_ns = getenv("DWFGPU_NS");
-  if (env_ns) h->ns = atoi(env_ns);
-  while (!env_ns && h->ns > 4 && max_lds_bytes(h) > (size_t)h->max_lds) h->ns /= 2;
-  if (h->ns < 1 || h->ns * ls > 512) {
-    set_err("dwfgpu_create: bad launch shape ns=%d (ns*Ls <= 512)", h->ns);
-    delete h;
-    return DWFGPU_BAD_ARG;
+  for (int k = 0; k < NPREC; ++k) {
+    const int ns = h->ns[k] = env_ns ? atoi(env_ns) : hop_sites(h, k, ncu);
+    if (ns < 1 || ns * ls > 512) {
+      set_err("dwfgpu_create: bad launch shape ns=%d (ns*Ls <= 512)", ns);
+      delete h;
+      return DWFGPU_BAD_ARG;
+    }
+    const size_t lds = hop_lds_bytes(action, ls, ns, k == DWFGPU_F64 ? 8 : 4);
+    if (lds > (size_t)h->max_lds) {
+      set_err("dwfgpu_create: Ls=%d needs %zu bytes of LDS per work-group (limit %d)", ls, lds,
+              h->max_lds);
+      delete h;
+      return DWFGPU_BAD_ARG;
+    }
+    h->grid_hop = std::max(h->grid_hop, (h->g.vh + ns - 1) / ns);
   }
-  if (max_lds_bytes(h) > (size_t)h->max_lds) {
-    set_err("dwfgpu_create: Ls=%d needs %zu bytes of LDS per work-group (limit %d)", ls,
-            max_lds_bytes(h), h->max_lds);
-    delete h;
-    return DWFGPU_BAD_ARG;
-  }
-  h->grid_hop = (h->g.vh + h->ns - 1) / h->ns;
   set_shape64(h);
   h->npartial = std::max({h->grid_hop, h->grid64, dwfk::BLAS_BLOCKS});
   int r = DWFGPU_OK;
@@ -4087,7 +4133,7 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
       hipLaunchKernelGGL((dwfk::k_convert<P, P64>), blas_grid(), blas_block(), 0, h->st,
                          fld<P>(mslice<P>(h, m.ps[0], j)), cfld<P64>(mslice<P64>(h, in->v, j)), h->g);
     HIPCHK(hipGetLastError());
-    MrShape t{h->ns, 1};
+    MrShape t{Ops<P>::sites(h), 1};
     if (h->action == DWFGPU_DWF && pidx<P>() == DWFGPU_F64 && h->ns64) {
       // the passes of a single right-hand side on this lattice, all in one launch
       TRY(mr_pinned(h, nrhs, sizeof(double), &t));
