@@ -391,6 +391,11 @@ constexpr size_t fwd_lds() {
 // CU and runs 11 % faster than on the 2 x 2 grid.
 template <int MB>
 constexpr bool fwd_g4() { return MB == 8; }
+// whether every local index is a block of its wave: then no product stands under
+// a condition on the wave, which the compiler takes for one on the lane (an exec
+// mask and a branch around each product; see k_ptc_gw)
+template <int RM, int MB>
+constexpr bool fwd_full(bool paired) { return fwd_g4<MB>() || paired || 2 * RM == MB; }
 template <int RM, int MB>
 __device__ __forceinline__ int fwd_block(int i, int h, bool paired) {
   if (fwd_g4<MB>()) return i == 0 ? h : MB / 2 + h;
@@ -405,7 +410,7 @@ __device__ __forceinline__ void load_frags(u32x4 (&af)[RM][K32], const u32x4* __
 #pragma unroll
   for (int i = 0; i < RM; ++i) {
     const int blk = fwd_block<RM, MB>(i, h, paired);
-    if (blk < MB)
+    if (fwd_full<RM, MB>(paired) || blk < MB)
 #pragma unroll
       for (int kb = 0; kb < K32; ++kb) af[i][kb] = A[((d * MB + blk) * K32 + kb) * 64 + lane];
   }
@@ -437,6 +442,7 @@ k_ptc_fwd(uint32_t* __restrict__ out, const uint32_t* __restrict__ in,
   constexpr bool G4 = fwd_g4<MB>();
   constexpr int RM = G4 ? 2 : PAIRED ? MB / 2 : (MB + 1) / 2, RH = G4 ? 1 : MB / 4;
   constexpr int RN = G4 ? NB : NB / 2;
+  constexpr bool FULL = fwd_full<RM, MB>(PAIRED);
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t* sB = reinterpret_cast<uint16_t*>(smem);
   float* sC = reinterpret_cast<float*>(smem);  // after the last GEMM (not paired)
@@ -484,7 +490,7 @@ k_ptc_fwd(uint32_t* __restrict__ out, const uint32_t* __restrict__ in,
       for (int j = 0; j < RN; ++j) bfr[j] = ld8(pb + j * 16 * (KP + PADK) + k0);
 #pragma unroll
       for (int i = 0; i < RM; ++i) {
-        if (blk_of(i) < MB) {
+        if (FULL || blk_of(i) < MB) {
           const bf16x8 a8 = __builtin_bit_cast(bf16x8, af[i][kb]);
 #pragma unroll
           for (int j = 0; j < RN; ++j)
@@ -513,7 +519,7 @@ k_ptc_fwd(uint32_t* __restrict__ out, const uint32_t* __restrict__ in,
 #pragma unroll
     for (int i = 0; i < RM; ++i) {
       const int blk = blk_of(i);
-      if (blk < MB) {
+      if (FULL || blk < MB) {
 #pragma unroll
         for (int j = 0; j < RN; ++j)
 #pragma unroll
@@ -608,6 +614,8 @@ k_ptc_gw(float* __restrict__ part, int nwg, const uint32_t* __restrict__ gout,
   static_assert(NCOL % 32 == 0 && (XS * 2) % 8 == 0 && (YS * 2) % 8 == 0, "tile shapes");
   // this wave's output blocks: rows [mb0, mb0 + RM) x columns [kb0, kb0 + RK)
   constexpr int RM = (MB + 1) / 2, RK = (KB2 + 1) / 2;
+  // even block counts: every wave owns all of its RM x RK blocks
+  constexpr bool FM = MB % 2 == 0, FK = KB2 % 2 == 0;
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t* sX = reinterpret_cast<uint16_t*>(smem);  // X^T: [col][M']
   uint16_t* sY = sX + NCOL * XS;                     // Y^T: [col][K']
@@ -682,14 +690,14 @@ k_ptc_gw(float* __restrict__ part, int nwg, const uint32_t* __restrict__ gout,
       bf16x8 yf[RK];
 #pragma unroll
       for (int j = 0; j < RK; ++j)
-        if (kb0 + j < KB2) yf[j] = ld_frag_tr<YS>(sY, (kb0 + j) * 16, cb * 32, lane);
+        if (FK || kb0 + j < KB2) yf[j] = ld_frag_tr<YS>(sY, (kb0 + j) * 16, cb * 32, lane);
 #pragma unroll
       for (int i = 0; i < RM; ++i) {
-        if (mb0 + i < MB) {
+        if (FM || mb0 + i < MB) {
           const bf16x8 xf = ld_frag_tr<XS>(sX, (mb0 + i) * 16, cb * 32, lane);
 #pragma unroll
           for (int j = 0; j < RK; ++j)
-            if (kb0 + j < KB2)
+            if (FK || kb0 + j < KB2)
               acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, yf[j], acc[i][j], 0, 0, 0);
         }
       }
@@ -698,10 +706,10 @@ k_ptc_gw(float* __restrict__ part, int nwg, const uint32_t* __restrict__ gout,
   float* dst = part + ((size_t)d * nwg + x * m + k) * MP * KP;
 #pragma unroll
   for (int i = 0; i < RM; ++i) {
-    if (mb0 + i < MB) {
+    if (FM || mb0 + i < MB) {
 #pragma unroll
       for (int j = 0; j < RK; ++j)
-        if (kb0 + j < KB2)
+        if (FK || kb0 + j < KB2)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             dst[((mb0 + i) * 16 + 4 * (lane >> 4) + r) * KP + (kb0 + j) * 16 + (lane & 15)] =
