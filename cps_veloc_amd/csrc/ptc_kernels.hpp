@@ -216,21 +216,9 @@ k_ptc_loss(uint32_t* __restrict__ gact, const uint32_t* __restrict__ a3,
 // I = (Im M_ab, Re M_ab) (low half first), so that for a colour vector f held as
 // activations (f_b = (Re f_b, Im f_b)):
 //   Re (M f)_a = sum_b dot2(R_ab, f_b),   Im (M f)_a = sum_b dot2(I_ab, f_b).
-// Each bf16 x bf16 product is exact in FP32.  The thread that staged link w
-// (stage_links: thread w stages link w of the tile, w = direction * NT +
-// site) rewrites its 9 complex entries in place, 18 words in the same 72
-// bytes, so no barrier is needed in between (only_dir >= 0: only the NT
-// links of that direction, staged compactly from entry 0, so entry
-// threadIdx.x - only_dir * NT).
-__device__ __forceinline__ void pack_links_dot2(cx<float>* lu, int only_dir = -1) {
-  const int w = (int)threadIdx.x - (only_dir >= 0 ? only_dir * NT : 0);
-  if (w < 0 || w >= (only_dir >= 0 ? NT : 8 * NT)) return;
-  cx<float> u[9];
-#pragma unroll
-  for (int e = 0; e < 9; ++e) u[e] = lu[w * 9 + e];
-  // staged direction 4..7: backward links
-  const bool dag = only_dir >= 0 ? only_dir >= 4 : w >= 4 * NT;
-  uint32_t* q = reinterpret_cast<uint32_t*>(lu + w * 9);
+// Each bf16 x bf16 product is exact in FP32.  u: the link's 9 entries, dag: of
+// a backward direction.
+__device__ __forceinline__ void pack_link(uint32_t* q, const cx<float>* u, bool dag) {
 #pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -239,6 +227,17 @@ __device__ __forceinline__ void pack_links_dot2(cx<float>* lu, int only_dir = -1
       q[(a * 3 + b) * 2] = dwfk::bf16_pair(m.re, -m.im);
       q[(a * 3 + b) * 2 + 1] = dwfk::bf16_pair(m.im, m.re);
     }
+}
+// The thread that staged link w (stage_links: thread w stages link w of the
+// tile, w = direction * NT + site) rewrites its 9 complex entries in place, 18
+// words in the same 72 bytes, so no barrier is needed in between.
+__device__ __forceinline__ void pack_links_dot2(cx<float>* lu) {
+  const int w = (int)threadIdx.x;
+  if (w >= 8 * NT) return;
+  cx<float> u[9];
+#pragma unroll
+  for (int e = 0; e < 9; ++e) u[e] = lu[w * 9 + e];
+  pack_link(reinterpret_cast<uint32_t*>(lu + w * 9), u, w >= 4 * NT);
 }
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -553,7 +552,7 @@ template <int CIN, int COUT>
 constexpr size_t gw_lds() {
   constexpr size_t x = (size_t)NCOL * (8 * COUT + PADW) * 2;
   constexpr size_t y = (size_t)NCOL * (8 * CIN + PADW) * 2;
-  return x + y + (size_t)NT * 9 * 8 + NT * 4;
+  return x + y + (size_t)NT * 18 * 4;
 }
 
 // One MFMA operand fragment (8 bf16: rows r0 + l%16, columns c0 + 8(l/16) ..
@@ -619,8 +618,7 @@ k_ptc_gw(float* __restrict__ part, int nwg, const uint32_t* __restrict__ gout,
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t* sX = reinterpret_cast<uint16_t*>(smem);  // X^T: [col][M']
   uint16_t* sY = sX + NCOL * XS;                     // Y^T: [col][K']
-  cx<float>* lu = reinterpret_cast<cx<float>*>(smem + (size_t)NCOL * (XS + YS) * 2);
-  int* lnb = reinterpret_cast<int*>(reinterpret_cast<unsigned char*>(lu) + (size_t)NT * 9 * 8);
+  uint32_t* lw = reinterpret_cast<uint32_t*>(smem + (size_t)NCOL * (XS + YS) * 2);  // [NT][18]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tiles_per_par = g.vh / NT, ntiles = 2 * tiles_per_par;
   const int nx = nwg % g.nxcd == 0 ? g.nxcd : 1, m = nwg / nx;
@@ -641,16 +639,71 @@ k_ptc_gw(float* __restrict__ part, int nwg, const uint32_t* __restrict__ gout,
   if (PFX && t_first < t_end)
     load_x<COUT>(xv, gout, t_first / tiles_per_par,
                  (t_first - t_first / tiles_per_par * tiles_per_par) * NT, g);
+  // The neighbour-table entries of a tile's items and, in the first NT threads,
+  // links are read one tile ahead, so that a tile's activations, links and
+  // output gradient are all in flight at once: it waits for memory once (entry,
+  // link, barrier and gather one after the other: 274 us at 16^3x32 for 16 -> 16
+  // channels; 248 this way).
+  constexpr int PER = Items<CIN>::PER;
+  const bool hop = d > 0, bwd = d > 4;
+  auto entry = [&](int t, int n) {
+    const int par = t / tiles_per_par, i = (t - par * tiles_per_par) * NT + n;
+    return hop ? g.nbt[(size_t)(par * 8 + d - 1) * g.vh + i] : i;
+  };
+  int ent[PER], lent = 0;
+  auto entries = [&](int t) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int w = threadIdx.x + j * NTHR;
+      if (Items<CIN>::EXACT || w < Items<CIN>::N) ent[j] = entry(t, w / CIN);
+    }
+    if (hop && threadIdx.x < NT) lent = entry(t, threadIdx.x);
+  };
+  if (t_first < t_end) entries(t_first);
   for (int t = t_first; t < t_end; t += m) {
     const int par = t / tiles_per_par;
     const int i0 = (t - par * tiles_per_par) * NT;
+    u32x4 raw[PER][3];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int w = threadIdx.x + j * NTHR;
+      if (Items<CIN>::EXACT || w < Items<CIN>::N) {
+        const size_t y = (size_t)(hop ? 1 - par : par) * g.vh + (ent[j] & 0x7fffffff);
+        const u32x4* src =
+            reinterpret_cast<const u32x4*>(in + (y * CIN + (w - w / CIN * CIN)) * 12);
+        raw[j][0] = src[0];
+        raw[j][1] = src[1];
+        raw[j][2] = src[2];
+      }
+    }
+    cx<float> u[9];
+    const float sg = lent < 0 ? -1.f : 1.f;
+    if (hop && threadIdx.x < NT) {  // U_mu(x) or, of the other parity, U_mu(x - mu)
+      const int site = bwd ? lent & 0x7fffffff : i0 + (int)threadIdx.x;
+      const typename dwfk::P32::S* src =
+          U + (size_t)((((d - 1) & 3) * 2 + (bwd ? 1 - par : par)) * 6) * g.vh + site;
+#pragma unroll
+      for (int e = 0; e < 6; ++e)
+        u[e] = dwfk::Pack<dwfk::P32>::unpack(dwfk::ld_link_elem<dwfk::P32>(src + (size_t)e * g.vh),
+                                             dwfk::link_scale<dwfk::P32>());
+    }
     if (!PFX) load_x<COUT>(xv, gout, par, i0, g);
+    if (t + m < t_end) entries(t + m);
+    __builtin_amdgcn_sched_barrier(0);  // all of them before the first is used
     __syncthreads();  // previous tile's operands consumed
-    // only direction d's links and neighbours are read (none for d = 0),
-    // staged compactly in slot 0
-    if (d > 0) {
-      dwfk::stage_links<dwfk::P32>(lu, lnb, U, g, i0 / NT, NT, 1, par, d - 1, (d - 1) * NT);
-      pack_links_dot2(lu, d - 1);
+    if (hop && threadIdx.x < NT) {
+      // row 2 = conj(row0 x row1) times the boundary sign, fused as the compiler
+      // fuses it in stage_links, so that both kernels round the same link
+      auto mul = [](cx<float> a, cx<float> b) {
+        return cx<float>{fmaf(a.re, b.re, -(a.im * b.im)), fmaf(a.im, b.re, a.re * b.im)};
+      };
+      const cx<float> r0 = mul(u[1], u[5]) - mul(u[2], u[4]);
+      const cx<float> r1 = mul(u[2], u[3]) - mul(u[0], u[5]);
+      const cx<float> r2 = mul(u[0], u[4]) - mul(u[1], u[3]);
+      u[6] = cx<float>{sg * r0.re, -sg * r0.im};
+      u[7] = cx<float>{sg * r1.re, -sg * r1.im};
+      u[8] = cx<float>{sg * r2.re, -sg * r2.im};
+      pack_link(lw + threadIdx.x * 18, u, bwd);
     }
     // X^T of the tile: item (site n, channel o) holds words spin*3 + colour;
     // the 4 spins of a colour are 4 consecutive rows o*4 + spin (real parts)
@@ -673,11 +726,7 @@ k_ptc_gw(float* __restrict__ part, int nwg, const uint32_t* __restrict__ gout,
       }
     }
     __syncthreads();  // links staged
-    {
-      u32x4 raw[Items<CIN>::PER][3];
-      gather_items<CIN>(raw, in, lnb, d, par, i0, g, 0);
-      store_transported<CIN, YS>(sY, raw, reinterpret_cast<const uint32_t*>(lu), d, 0);
-    }
+    store_transported<CIN, YS>(sY, raw, lw, d, 0);
     __syncthreads();
     {
       const int tn = t + m;
