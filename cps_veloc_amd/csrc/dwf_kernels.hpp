@@ -716,8 +716,7 @@ template <class P>
 __device__ __forceinline__ void stage_links(cx<typename P::R>* __restrict__ lu,
                                             int* __restrict__ lnb,
                                             const typename P::S* __restrict__ U, const Geom& g,
-                                            int blk, int ns, int nsets, int p_first,
-                                            int only_dir = -1, int dst_base = 0) {
+                                            int blk, int ns, int nsets, int p_first) {
   typedef typename P::R R;
   constexpr int NE = P::kLinkElems;
   const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
@@ -725,17 +724,17 @@ __device__ __forceinline__ void stage_links(cx<typename P::R>* __restrict__ lu,
   for (int w = tid; w < nsets * 8 * ns; w += nthr) {
     const int il = w % ns, d = (w / ns) % 8, set = w / (8 * ns);
     const int i = blk * ns + il;
-    if (i >= g.vh || (only_dir >= 0 && d != only_dir)) continue;
+    if (i >= g.vh) continue;
     const int p = (p_first + set) & 1;
     const int mu = d & 3;
     const int e = g.nbt[(size_t)(p * 8 + d) * g.vh + i];
     const int nbr = e & 0x7fffffff;
     const bool neg = e < 0;
     const int site = d >= 4 ? nbr : i;
-    lnb[w - dst_base] = nbr;
+    lnb[w] = nbr;
     const int par = d >= 4 ? 1 - p : p;  // U_mu(x - mu) lives on the other parity
     const typename P::S* src = U + (size_t)((mu * 2 + par) * NE) * g.vh + site;
-    cx<R>* dst = lu + (size_t)(w - dst_base) * 9;
+    cx<R>* dst = lu + (size_t)w * 9;
     const float ls = link_scale<P>();
 #pragma unroll
     for (int e = 0; e < NE; ++e) dst[e] = Pack<P>::unpack(ld_link_elem<P>(src + (size_t)e * g.vh), ls);

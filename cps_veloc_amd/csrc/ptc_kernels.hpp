@@ -288,12 +288,10 @@ __device__ __forceinline__ void transport4(const uint32_t* lw, int d, const uint
 }
 
 // site of the activation neighbour of tile site n along d (S index)
-// (lslot: the slot of the staged neighbour list holding direction d, d - 1
-// when all eight directions are staged)
 __device__ __forceinline__ size_t nbr_site(const int* lnb, int d, int n, int par, int i0,
-                                           const Geom& g, int lslot) {
+                                           const Geom& g) {
   if (d == 0) return (size_t)par * g.vh + i0 + n;
-  return (size_t)(1 - par) * g.vh + lnb[lslot * NT + n];
+  return (size_t)(1 - par) * g.vh + lnb[(d - 1) * NT + n];
 }
 
 // (site, channel) items of a tile spread over the work-group: PER per thread
@@ -309,15 +307,13 @@ struct Items {
 template <int CIN>
 __device__ __forceinline__ void gather_items(u32x4 (&raw)[Items<CIN>::PER][3],
                                              const uint32_t* __restrict__ in, const int* lnb,
-                                             int d, int par, int i0, const Geom& g,
-                                             int lslot = -1) {
-  if (lslot < 0) lslot = d - 1;
+                                             int d, int par, int i0, const Geom& g) {
 #pragma unroll
   for (int j = 0; j < Items<CIN>::PER; ++j) {
     const int w = threadIdx.x + j * NTHR;
     if (Items<CIN>::EXACT || w < Items<CIN>::N) {
       const int n = w / CIN, i = w - n * CIN;
-      const size_t y = nbr_site(lnb, d, n, par, i0, g, lslot);
+      const size_t y = nbr_site(lnb, d, n, par, i0, g);
       const u32x4* src = reinterpret_cast<const u32x4*>(in + (y * CIN + i) * 12);
       raw[j][0] = src[0];
       raw[j][1] = src[1];
