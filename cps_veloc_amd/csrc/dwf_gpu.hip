@@ -717,6 +717,17 @@ struct Ops {
     return matpc_w(h, mass, out, in, dag, sum, nullptr, own(h));
   }
 
+  // out = MatPc in with the |out|^2 partials (grid(h) of them) left in h->partial
+  static int matpc_partials(dwfgpu_s* h, double mass, const DVec& out, const DVec& in) {
+    const DVec& te = F(h).te;
+    if (h->action == DWFGPU_DWF) {
+      TRY(dwf(h, mass, te, in, 1, 0, 0, DVec(), 0.0, false));
+      return dwf(h, mass, out, te, 0, 0, 1, in, -dwf_kappa(h) * dwf_kappa(h), true);
+    }
+    TRY(mob_first(h, mass, te, in, 0));
+    return mob_second(h, mass, out, te, in, 0, true);
+  }
+
   // MatPcDagMatPc; *dot (if requested) = |MatPc in|^2 (dwf_mdagm.C:49-55), for
   // which the host waits once, at the end
   static int mdagm_w(dwfgpu_s* h, double mass, const DVec& out, const DVec& in, double* dot,
@@ -2525,7 +2536,8 @@ namespace {
 struct MsWork {
   DVec p;              // directions of all shifts
   void* mem = nullptr;  // the ring of residuals and the live p0
-  dwfk::MsStep* steps = nullptr;   // device
+  dwfk::MsStep* steps = nullptr;   // device, and behind them
+  double* ppart = nullptr;         // |p0|^2's partials
   dwfk::MsStep* hsteps = nullptr;  // pinned, MS_SLOTS flushes
   hipEvent_t ev[4] = {};
   ~MsWork() {
@@ -2554,7 +2566,8 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
   MsWork w;
   Drain drain{h->st};
   HIPCHK(hipMalloc(&w.p.d, (size_t)nshift * vbytes));
-  HIPCHK(hipMalloc((void**)&w.steps, MS_MAXK * sizeof(MsStep)));
+  HIPCHK(hipMalloc((void**)&w.steps, MS_MAXK * sizeof(MsStep) + BLAS_BLOCKS * sizeof(double)));
+  w.ppart = (double*)(w.steps + MS_MAXK);
   HIPCHK(hipHostMalloc((void**)&w.hsteps, MS_SLOTS * MS_MAXK * sizeof(MsStep),
                        hipHostMallocDefault));
   for (auto& e : w.ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -2605,10 +2618,12 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
   // step k: p0 = r_k + a p0, then r_{k+1} = r_k + b (A + sigma) p0
   auto step = [&](int k) -> int {
     hipLaunchKernelGGL(k_ms_p, blas_grid(), blas_block(), 0, h->st, p0, res(k), h->dscal,
-                       k == 0 ? 1 : 0, n, h->partial);
+                       k == 0 ? 1 : 0, n, w.ppart);
     HIPCHK(hipGetLastError());
-    TRY(reduce_to(h, BLAS_BLOCKS, MS_PP));
-    TRY(H::matpc(h, mass, t1, vp0, 0, h->dscal + MS_MP));
+    TRY(H::matpc_partials(h, mass, t1, vp0));
+    hipLaunchKernelGGL(k_ms_dots, dim3(2), dim3(1024), 0, h->st, h->partial, H::grid(h), w.ppart,
+                       (int)BLAS_BLOCKS, h->dscal);
+    HIPCHK(hipGetLastError());
     TRY(H::matpc(h, mass, vap, t1, 1));
     hipLaunchKernelGGL(k_ms_r, blas_grid(), blas_block(), 0, h->st, res(k + 1), res(k), ap, p0,
                        sigma, h->dscal, n, h->partial);
