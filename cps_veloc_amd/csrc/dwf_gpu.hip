@@ -75,7 +75,8 @@ struct PrecFields {
   void* U = nullptr;  // links (18 reals in FP64, first two rows otherwise)
   DVec te, t1;        // opposite-parity temporary, MatPc output inside MdagM
   DVec work[6];       // solver vectors, allocated on first use
-  std::vector<DVec> ring;  // CG directions of the last steps (mixed CG)
+  std::vector<DVec> ring;  // CG directions of the last steps
+  std::vector<void*> ring_mem;  // the blocks they lie in
 };
 
 }  // namespace
@@ -357,10 +358,23 @@ int ensure_work(dwfgpu_s* h, int count) {
 template <class P>
 int ensure_ring(dwfgpu_s* h, int count) {
   TRY(ensure_fields<P>(h));
-  std::vector<DVec>& ring = h->f[pidx<P>()].ring;
-  if ((int)ring.size() < count) ring.resize(count);
-  for (int k = 0; k < count; ++k)
-    if (!ring[k].d) TRY(alloc_vec<P>(h, &ring[k]));
+  PrecFields& f = h->f[pidx<P>()];
+  const int have = (int)f.ring.size();
+  if (have >= count) return DWFGPU_OK;
+  // the missing ones in one block: each allocation costs 0.2 ms to free
+  auto round = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t vb = round(h->n / 2 * sizeof(typename P::S));
+  const size_t sb = P::kScaled ? round((size_t)h->g.vh * h->ls * sizeof(float)) : 0;
+  char* p = nullptr;
+  f.ring_mem.push_back(nullptr);
+  TRY(alloc(h, (void**)&p, (count - have) * (vb + sb)));
+  f.ring_mem.back() = p;
+  for (int k = have; k < count; ++k, p += vb + sb) {
+    DVec v;
+    v.d = p;
+    if (P::kScaled) v.sc = (float*)(p + vb);
+    f.ring.push_back(v);
+  }
   return DWFGPU_OK;
 }
 
@@ -369,8 +383,7 @@ int ensure_ring(dwfgpu_s* h, int count) {
 template <class P>
 int ring_fits(dwfgpu_s* h, int count, int* n) {
   size_t have = 0, total = 0, need = 0;
-  const std::vector<DVec>& ring = h->f[pidx<P>()].ring;
-  for (const DVec& v : ring) have += v.d ? 1 : 0;
+  have = h->f[pidx<P>()].ring.size();
   *n = count;
   if (have >= (size_t)count) return DWFGPU_OK;
   need = (count - have) * (size_t)half_bytes<P>(h);
@@ -1390,7 +1403,9 @@ void free_all(dwfgpu_s* h) {
     free_vec(&F.te);
     free_vec(&F.t1);
     for (auto& w : F.work) free_vec(&w);
-    for (auto& w : F.ring) free_vec(&w);
+    for (void* m : F.ring_mem)
+      if (m) (void)hipFree(m);
+    F.ring_mem.clear();
     F.ring.clear();
     F.ready = false;
   }
