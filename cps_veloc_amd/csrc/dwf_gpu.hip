@@ -2630,7 +2630,10 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
     slot = (slot + 1) % MS_SLOTS;
     return DWFGPU_OK;
   };
-  // step k: p0 = r_k + a p0, then r_{k+1} = r_k + b (A + sigma) p0
+  std::vector<double> rsd_sq(nshift);
+  for (int s = 0; s < nshift; ++s) rsd_sq[s] = chi_norm * rsdcg[s] * rsdcg[s];
+  // step k: p0 = r_k + a p0 (until the first shift has converged), then
+  // r_{k+1} = r_k + b (A + sigma) p0
   auto step = [&](int k) -> int {
     hipLaunchKernelGGL(k_ms_p, blas_grid(), blas_block(), 0, h->st, p0, res(k), h->dscal,
                        k == 0 ? 1 : 0, n, w.ppart);
@@ -2643,7 +2646,7 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
     hipLaunchKernelGGL(k_ms_r, blas_grid(), blas_block(), 0, h->st, res(k + 1), res(k), ap, p0,
                        sigma, h->dscal, n, h->partial);
     hipLaunchKernelGGL(k_ms_reduce, dim3(1), dim3(1024), 0, h->st, h->partial, (int)BLAS_BLOCKS,
-                       sigma, h->dscal, h->hring + 8 * (k % NEV));
+                       sigma, rsd_sq[0], k == 0 ? 1 : 0, h->dscal, h->hring + 8 * (k % NEV));
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(w.ev[k % NEV], h->st));
     return DWFGPU_OK;
@@ -2653,11 +2656,9 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
   HIPCHK(hipMemcpyAsync(h->dscal + MS_C, h->hscal, sizeof(double), hipMemcpyHostToDevice, h->st));
 
   double cp = chi_norm, c = chi_norm, b = 0.0, a = 0.0;
-  std::vector<double> rsd_sq(nshift), bs(nshift), z0(nshift, 1.0), z1(nshift, 1.0), fin(nshift),
-      f(nshift);
+  std::vector<double> bs(nshift), z0(nshift, 1.0), z1(nshift, 1.0), fin(nshift), f(nshift);
   double* z[2] = {z0.data(), z1.data()};
   std::vector<int> convs(nshift, 0), conv_at(nshift, 0);
-  for (int s = 0; s < nshift; ++s) rsd_sq[s] = chi_norm * rsdcg[s] * rsdcg[s];
   int iz = 1, convp = 0;
   unsigned todo = 0;  // shifts whose psi update by f is pending
   // the entry of step k for the flush: the pending psi update, and the

@@ -2260,7 +2260,10 @@ k_ms_flush(MsFlush a, const MsStep* __restrict__ st) {
 
 // Scalars of the step on the device: |r|^2, |MatPc p0|^2, |p0|^2 and the
 // previous |r|^2; d = <p0, (A + sigma) p0> = |MatPc p0|^2 + sigma |p0|^2.
-enum { MS_C = 0, MS_MP = 1, MS_PP = 2, MS_CP = 3 };
+// MS_HOLD: 1 once the first shift has converged.  Its direction is then left as
+// it is like any converged shift's (minvcg.C:210-222), and the steps that the
+// other shifts still need go on with that p0.
+enum { MS_C = 0, MS_MP = 1, MS_PP = 2, MS_CP = 3, MS_HOLD = 4 };
 
 // ro = r + b (ap + sigma p), b = -|r|^2 / d; |ro|^2 partials
 __global__ void __launch_bounds__(BLAS_THREADS)
@@ -2282,11 +2285,13 @@ k_ms_r(cx<double>* ro, const cx<double>* r, const cx<double>* __restrict__ ap,
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// p = r + (|r|^2 / previous |r|^2) p; |p|^2 partials.  first: p = r
+// p = r + (|r|^2 / previous |r|^2) p; |p|^2 partials.  first: p = r.  Held (MS_HOLD):
+// p and its partials stay those of the last step.
 __global__ void __launch_bounds__(BLAS_THREADS)
 k_ms_p(cx<double>* __restrict__ p, const cx<double>* __restrict__ r,
        const double* __restrict__ scal, int first, size_t n, double* __restrict__ partial) {
   __shared__ double sh[16];
+  if (!first && scal[MS_HOLD] != 0.0) return;  // uniform
   const double a = first ? 0.0 : scal[MS_C] / scal[MS_CP];
   double acc = 0.0;
   for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
@@ -2315,10 +2320,11 @@ k_ms_dots(const double* __restrict__ mp, int nmp, const double* __restrict__ pp,
 }
 
 // the end of a step: |r|^2 of the partials becomes the current one; host
-// (pinned) receives it and d
+// (pinned) receives it and d.  stop: the first shift's stop condition on |r|^2,
+// (the first step's own test ends the whole solve and is the host's)
 __global__ void __launch_bounds__(1024)
-k_ms_reduce(const double* __restrict__ partial, int n, double sigma, double* __restrict__ scal,
-            double* __restrict__ host) {
+k_ms_reduce(const double* __restrict__ partial, int n, double sigma, double stop, int first,
+            double* __restrict__ scal, double* __restrict__ host) {
   __shared__ double sh[16];
   double a0 = 0.0;
   for (int k = threadIdx.x; k < n; k += 1024) a0 += partial[k];
@@ -2328,6 +2334,10 @@ k_ms_reduce(const double* __restrict__ partial, int n, double sigma, double* __r
     host[0] = t;
     scal[MS_CP] = scal[MS_C];
     scal[MS_C] = t;
+    if (first)
+      scal[MS_HOLD] = 0.0;
+    else if (t < stop)
+      scal[MS_HOLD] = 1.0;
   }
 }
 
