@@ -2665,19 +2665,18 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
   // directions of step k from r_k
   auto entry = [&](int k, bool directions) {
     MsStep* e = pending();
-    unsigned moves = todo;
+    e->psi = todo;
+    e->p = 0;
     for (int s = 0; s < nshift; ++s) {
-      e->f[s] = (todo >> s) & 1u ? f[s] : 0.0;
-      e->zr[s] = 0.0;
-      e->ap[s] = 1.0;
+      e->f[s] = f[s];
       // without a ring the first shift's direction is the live one
       if (!directions || convs[s] || (s == 0 && !w.mem)) continue;
-      moves |= 1u << s;
+      e->p |= 1u << s;
       e->zr[s] = s == 0 ? 1.0 : z[iz][s];
       e->ap[s] = s == 0 ? a : a * (z[iz][s] * bs[s]) / (z[1 - iz][s] * b);
     }
     F.r[F.cnt++] = res(k);
-    F.active |= moves;
+    F.active |= e->psi | e->p;
     todo = 0;
   };
   // the recurrences of step k from its scalars

@@ -2209,11 +2209,13 @@ k_compress_links(typename P::S* __restrict__ dst, const cx<double>* __restrict__
 constexpr int MAXSHIFT = 32;
 constexpr int MS_MAXK = 8;
 
-// one pending step: psi_s += f[s] p_s (the end of the step before), then
-// p_s = zr[s] r + ap[s] p_s (minvcg.C:266-285, :210-222); 0, 0, 1 for a shift
-// that takes no part any more
+// one pending step: psi_s += f[s] p_s (the end of the step before) for the
+// shifts of psi's bits, then p_s = zr[s] r + ap[s] p_s for those of p's
+// (minvcg.C:266-285, :210-222).  A shift that takes no part any more is skipped,
+// not multiplied by 0: after a breakdown r is not finite.
 struct MsStep {
   double f[MAXSHIFT], zr[MAXSHIFT], ap[MAXSHIFT];
+  unsigned psi, p;
 };
 struct MsFlush {
   cx<double>* psi;        // shift s at psi + s * vs (SINGLE: one psi for all)
@@ -2248,8 +2250,8 @@ k_ms_flush(MsFlush a, const MsStep* __restrict__ st) {
 #pragma unroll
       for (int j = 0; j < K; ++j)
         if (j < a.cnt) {
-          acc = st[j].f[s] * p + acc;
-          p = st[j].zr[s] * r[j] + st[j].ap[s] * p;
+          if ((st[j].psi >> s) & 1u) acc = st[j].f[s] * p + acc;
+          if ((st[j].p >> s) & 1u) p = st[j].zr[s] * r[j] + st[j].ap[s] * p;
         }
       *ps = p;
       if (!a.single) *qs = acc;

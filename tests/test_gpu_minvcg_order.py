@@ -1,9 +1,10 @@
 """GPU MInvCG where a shift stops before the others need it to: the first shift
 converges first (shifts in falling order, or looser stop residuals of its own),
 which freezes the direction that every later step uses (minvcg.C:210-222 skips
-a converged shift 0 too).  Against the oracle: the same iteration counts, psi
-within 1e-10 relative a shift and the residuals to 1e-7 (relative link errors of
-1e-14 move the oracle's own by 4e-14 and 1e-12)."""
+a converged shift 0 too), and a recurrence that breaks down a few steps after a
+shift converged, which leaves that shift's solution alone.  Against the oracle:
+the same iteration counts, psi within 1e-10 relative a shift and the residuals to
+1e-7 (relative link errors of 1e-14 move the oracle's own by 4e-14 and 1e-12)."""
 import numpy as np
 import pytest
 
@@ -53,4 +54,21 @@ def test_general_lattice(action):
         assert gk == ok and np.array_equal(git, oit) and np.allclose(grs, ors, rtol=1e-7)
         for s in range(len(shifts)):
             assert np.linalg.norm(gp[s] - op[s]) <= 1e-10 * np.linalg.norm(op[s])
+    g.close()
+
+
+@pytest.mark.parametrize("action", ["dwf", "mobius"])
+def test_breakdown_after_a_shift_converged(action):
+    """|chi|^2 of 1e-295 underflows within seven steps, the second shift having
+    converged in the first: 0 / 0 from there on in the first shift only."""
+    print(f"[gpu] MInvCG {action}: |r|^2 runs into underflow", flush=True)
+    g, o = make(action, (4, 2, 2, 6), 4)
+    chi = 1e-149 * np.random.default_rng(9).standard_normal(g.n)
+    shifts, rsd = [300.0, 600.0], [1e-200, 1e-2]
+    gp, gk, grs, git, _ = g.MInvCG(chi, 0.1, shifts, rsd, max_iter=20)
+    op, ok, ors, oit = o.minvcg(chi, 0.1, shifts, rsd, max_iter=20)
+    assert np.isnan(op[0]).all() and np.isfinite(op[1]).all()
+    assert gk == ok and np.array_equal(git, oit) and abs(grs[1] - ors[1]) <= 1e-7 * ors[1]
+    got, want = gp[1] * 1e149, op[1] * 1e149
+    assert np.linalg.norm(got - want) <= 1e-10 * np.linalg.norm(want)
     g.close()
