@@ -109,6 +109,7 @@ struct dwfgpu_s {
   // sites per work-group of the hopping kernels (x; y = all slices), per format
   int ns[NPREC] = {16, 16, 16, 16};
   int max_lds = 65536;
+  size_t ring_max = SIZE_MAX;  // most bytes of a solve's ring (DWFGPU_RING_MB)
   // launch shape of the many-RHS operator chosen by the autotuner, per
   // sloppy precision and RHS count (0: not tuned yet)
   int mr_ns[NPREC] = {0, 0, 0, 0}, mr_nr[NPREC] = {0, 0, 0, 0}, mr_nrhs[NPREC] = {0, 0, 0, 0};
@@ -378,18 +379,12 @@ int ensure_ring(dwfgpu_s* h, int count) {
   return DWFGPU_OK;
 }
 
-// vectors of a ring (*n = count), or one where they would take more than a
-// quarter of the device's free memory
-template <class P>
-int ring_fits(dwfgpu_s* h, int count, int* n) {
-  size_t have = 0, total = 0, need = 0;
-  have = h->f[pidx<P>()].ring.size();
-  *n = count;
-  if (have >= (size_t)count) return DWFGPU_OK;
-  need = (count - have) * (size_t)half_bytes<P>(h);
-  size_t avail = 0;
+// whether a solve may take `bytes` more for a ring of vectors: within the
+// handle's limit, and a quarter of the device's free memory at most
+int ring_room(const dwfgpu_s* h, size_t bytes, bool* ok) {
+  size_t avail = 0, total = 0;
   HIPCHK(hipMemGetInfo(&avail, &total));
-  if (need > avail / 4) *n = 1;
+  *ok = bytes <= h->ring_max && bytes <= avail / 4;
   return DWFGPU_OK;
 }
 
@@ -933,7 +928,7 @@ struct Ops {
         if (stop) break;
       }
     } else if (max_itr > 0) {
-      TRY(invcg_steps(h, mass, sol, dir, res, stp_cnd, max_itr, &itr, &status));
+      TRY(invcg_steps(h, mass, sol, dir, res, stp_cnd, rr, max_itr, &itr, &status));
     }
     // true residual |src - A sol| / |src|  (inv_cg.C:403-415)
     TRY(mdagm(h, mass, mmp, sol, nullptr));
@@ -947,36 +942,65 @@ struct Ops {
     return status;
   }
 
-  // The steps of the plain CG: res holds the residual and dscal[0] its square.
+  // The steps of the plain CG without a ring: sol += a dir and dir = res + b dir
+  // in one pass after every step (5 vectors), for which the host waits.  Moebius
+  // 24^3x64 Ls 12 in FP64: 4.72 ms a step; k_pnext and k_x_flush of the one step (6
+  // vectors, two launches) 4.90.
+  static int invcg_in_place(dwfgpu_s* h, double mass, const DVec& sol, const DVec& dir,
+                            const DVec& res, double stp_cnd, double rr, int max_itr, int* itr,
+                            int* status) {
+    TRY(copy(h, dir, res));
+    for (*itr = 1;; ++*itr) {
+      TRY(cg_step(h, mass, dir, res, h->dalpha, h->hring));
+      HIPCHK(hipStreamSynchronize(h->st));
+      const double rr_prv = rr, d = h->hring[1];
+      rr = h->hring[0];
+      if (d == 0.0) {  // alpha = 0 was used: res is unchanged
+        *status = DWFGPU_BREAKDOWN;
+        return DWFGPU_OK;
+      }
+      const double a = rr_prv / d;  // the epilogue's alpha (cg_alpha)
+      const bool last = rr <= stp_cnd || *itr == max_itr;
+      if (last)
+        hipLaunchKernelGGL((dwfk::k_cg_xp<P, P, false>), blas_grid(), blas_block(), 0, h->st,
+                           fld<P>(sol), fld<P>(dir), cfld<P>(res), a, 0.0, h->g);
+      else
+        hipLaunchKernelGGL((dwfk::k_cg_xp<P, P, true>), blas_grid(), blas_block(), 0, h->st,
+                           fld<P>(sol), fld<P>(dir), cfld<P>(res), a, rr / rr_prv, h->g);
+      HIPCHK(hipGetLastError());
+      if (last) return DWFGPU_OK;
+    }
+  }
+
+  // The steps of the plain CG: res holds the residual, dscal[0] and rr0 its
+  // square.
   // alpha and beta stay on the device, and the host looks at the scalars of a
   // step (CPS's stop test, inv_cg.C:354) while the GPU runs the next, so that the
   // GPU never waits for the host; one step past the last is run and not used.
   // The directions of the last steps stay in a ring and sol += alpha_j dir_j is
-  // applied CG_KRING steps at a time (k_x_flush, the order and rounding of one
-  // update per step): 4.3 vectors move per step beside the operator where
-  // sol += a dir and dir = res + b dir in every step moved 5, and no speculative
-  // step ever reaches sol.  Moebius 24^3x64 Ls 12: 1004 -> 836 us a step (5.1
-  // TB/s); DWF 8^4 Ls 8, where the wait for the host and k_cg_xp's 12 components
-  // a thread cost more than the traffic: 5.3 -> 4.3 ms for 92 steps.  Without room
-  // for the ring (a quarter of the free memory), or for CG_SHORT steps, every step
-  // is waited for and applied at once, dir in place.
+  // applied CG_KRING steps at a time (k_x_flush, in the order of one update per
+  // step; the 16-bit formats round sol once a flush): 4.3 vectors move per step
+  // beside the operator where sol += a dir and dir = res + b dir in every step
+  // move 5, and no speculative step ever reaches sol.  Moebius 24^3x64 Ls 12: 1004
+  // -> 836 us a step (5.1 TB/s); DWF 8^4 Ls 8, where the wait for the host and
+  // k_cg_xp's 12 components a thread cost more than the traffic: 5.3 -> 4.3 ms for
+  // 92 steps.  Without room for the ring (ring_room), or for CG_SHORT steps:
+  // invcg_in_place.
   static int invcg_steps(dwfgpu_s* h, double mass, const DVec& sol, const DVec& dir,
-                         const DVec& res, double stp_cnd, int max_itr, int* itr_out,
+                         const DVec& res, double stp_cnd, double rr0, int max_itr, int* itr_out,
                          int* status) {
-    constexpr int NEV = 4;
-    int K = CG_KRING, LAG = 1, NR = K + LAG + 1;
-    if (max_itr <= CG_SHORT)
-      NR = 1;
-    else
-      TRY(ring_fits<P>(h, NR, &NR));
-    if (NR == 1) {
-      K = 1;
-      LAG = 0;
-    } else {
-      TRY(ensure_ring<P>(h, NR));
+    constexpr int NEV = 4, K = CG_KRING, LAG = 1, NR = K + LAG + 1;
+    const int have = (int)F(h).ring.size();
+    bool room = max_itr > CG_SHORT;
+    if (room && have < NR) TRY(ring_room(h, (NR - have) * (size_t)half_bytes<P>(h), &room));
+    if (room && ensure_ring<P>(h, NR) != DWFGPU_OK) {  // no block of that size
+      (void)hipGetLastError();
+      room = false;
     }
-    auto slot = [&](int k) -> const DVec& { return NR == 1 ? dir : F(h).ring[k % NR]; };
-    const bool small = std::is_same<P, P64>::value && h->ns64 && NR > 1;
+    if (!room)
+      return invcg_in_place(h, mass, sol, dir, res, stp_cnd, rr0, max_itr, itr_out, status);
+    auto slot = [&](int k) -> const DVec& { return F(h).ring[k % NR]; };
+    const bool small = std::is_same<P, P64>::value && h->ns64;
     EventSet<NEV> ev;
     TRY(ev.create());
     dwfk::XFlush<P> xf;
@@ -1001,15 +1025,11 @@ struct Ops {
         if (!done) TRY(cg_step(h, mass, slot(k), res, al, host));
         HIPCHK(hipEventRecord(ev.e[k % NEV], h->st));
       }
-      // dir of step k + 1 = res + b dir; in place only after step k's update
-      auto next = [&]() -> int {
-        if (small || k >= max_itr) return DWFGPU_OK;
+      if (!small && k < max_itr) {  // dir of step k + 1 = res + b dir
         hipLaunchKernelGGL((dwfk::k_pnext<P>), blas_grid(), blas_block(), 0, h->st,
                            fld<P>(slot(k + 1)), cfld<P>(res), cfld<P>(slot(k)), h->dscal, h->g);
         HIPCHK(hipGetLastError());
-        return DWFGPU_OK;
-      };
-      if (LAG) TRY(next());
+      }
       const int j = k - LAG;
       if (j < 1) continue;
       HIPCHK(hipEventSynchronize(ev.e[j % NEV]));
@@ -1026,7 +1046,6 @@ struct Ops {
       xf.cnt++;
       if (xf.cnt == K) TRY(flush());
       if (rr <= stp_cnd) break;
-      if (!LAG) TRY(next());
     }
     TRY(flush());
     *itr_out = itr;
@@ -3641,6 +3660,18 @@ int dwfgpu_create(const double* gauge, const int dims[4], int ls, int action, do
   if (int rs = scratch_setup(dev)) {
     delete h;
     return rs;
+  }
+  // DWFGPU_RING_MB: most MiB of device memory that a solve's ring of vectors may
+  // take (0: the solvers run without)
+  if (const char* env = getenv("DWFGPU_RING_MB")) {
+    char* end = nullptr;
+    const unsigned long long mb = strtoull(env, &end, 10);
+    if (end == env || *end || mb > SIZE_MAX >> 20) {
+      set_err("DWFGPU_RING_MB=%s: need a number of MiB", env);
+      delete h;
+      return DWFGPU_BAD_ARG;
+    }
+    h->ring_max = (size_t)mb << 20;
   }
   // sites per work-group of the hopping kernels; DWFGPU_NS overrides the rule
   int ncu = 0;

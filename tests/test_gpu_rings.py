@@ -1,0 +1,49 @@
+"""GPU: the rings of vectors that the CG solvers keep their last steps in.
+
+With DWFGPU_RING_MB=0 (no ring: every step applied at once, the directions in
+place) a solve agrees with the oracle as with a ring.  Bars of the iterates: FP64
+1e-12, FP32 1e-5 and int16 2e-3 of the oracle's after the same steps."""
+import numpy as np
+import pytest
+
+from cps_veloc_amd import lattice as lat
+from cps_veloc_amd.dwf import BAD_ARG, CgArg, DiracOpDwfGpu, DiracOpMobiusGpu, DwfGpuError
+from oracle.oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+BAR = {"f64": 1e-12, "f32": 1e-5, "i16": 2e-3}
+
+
+def make(action, dims, ls, precision="f64", oracle=True):
+    U = lat.random_gauge(dims, 0.3, 7)
+    cls, kw = (DiracOpDwfGpu, {}) if action == "dwf" else (DiracOpMobiusGpu, {"b": 1.5, "c": 0.5})
+    g = cls(U, dims, ls, m5=1.8, precision=precision, **kw)
+    return g, (Oracle(dims, ls, action, m5=1.8, b=1.5, c=0.5, gauge_canonical=U) if oracle
+               else None)
+
+
+@pytest.mark.parametrize("ring", ["0", None])
+@pytest.mark.parametrize("action,precision", [("dwf", "f64"), ("mobius", "f64"), ("dwf", "f32"),
+                                              ("mobius", "i16")])
+def test_invcg(monkeypatch, action, precision, ring):
+    if ring is not None:
+        monkeypatch.setenv("DWFGPU_RING_MB", ring)
+    # a small-lattice and (36864 pairs) a general one
+    for dims, ls, mass in (((4, 2, 2, 6), 4, 0.2), ((8, 8, 8, 18), 8, 0.2)):
+        g, o = make(action, dims, ls, precision)
+        src = np.random.default_rng(11).standard_normal(g.n)
+        for cap in (3, 6, 10) if precision != "f64" else (2, 5, 6, 12, 21):
+            print(f"[gpu] InvCg ring={ring} {action} {precision} {dims} cap={cap}", flush=True)
+            sol = np.zeros(g.n)
+            it, _, _ = g.InvCg(sol, src, CgArg(mass, cap, 1e-15))
+            xo, oit, _, _ = o.invcg(src, mass, stop_rsd=1e-15, max_iter=cap)
+            assert it == oit
+            assert np.linalg.norm(sol - xo) <= BAR[precision] * np.linalg.norm(xo)
+        g.close()
+
+
+def test_limit_is_a_number(monkeypatch):
+    monkeypatch.setenv("DWFGPU_RING_MB", "lots")
+    with pytest.raises(DwfGpuError) as e:
+        make("dwf", (4, 2, 2, 6), 4, oracle=False)
+    assert e.value.code == BAD_ARG
