@@ -362,13 +362,14 @@ int ensure_ring(dwfgpu_s* h, int count) {
   PrecFields& f = h->f[pidx<P>()];
   const int have = (int)f.ring.size();
   if (have >= count) return DWFGPU_OK;
-  // the missing ones in one block: each allocation costs 0.2 ms to free
+  // the missing ones in one block (each allocation costs 0.2 ms to free), not
+  // cleared: every slot is written before it is read
   auto round = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t vb = round(h->n / 2 * sizeof(typename P::S));
   const size_t sb = P::kScaled ? round((size_t)h->g.vh * h->ls * sizeof(float)) : 0;
   char* p = nullptr;
   f.ring_mem.push_back(nullptr);
-  TRY(alloc(h, (void**)&p, (count - have) * (vb + sb)));
+  HIPCHK(hipMalloc((void**)&p, (count - have) * (vb + sb)));
   f.ring_mem.back() = p;
   for (int k = have; k < count; ++k, p += vb + sb) {
     DVec v;
@@ -378,6 +379,25 @@ int ensure_ring(dwfgpu_s* h, int count) {
   }
   return DWFGPU_OK;
 }
+
+// A block of more than RING_KEEP that a solve added to the ring goes back when
+// the solve ends, so that what it leaves to other users of the device does not
+// shrink with the lattice: hipMalloc and hipFree of 2 or 10 GiB take 0.3 ms each
+// (of a solve of 250 ms and more), of 256 MiB 0.03 and 0.3 ms, which a short
+// solve on a smaller lattice would notice.
+constexpr size_t RING_KEEP = (size_t)256 << 20;
+struct RingLoan {
+  dwfgpu_s* h;
+  PrecFields* f;
+  size_t count, blocks, bytes;  // the ring's length and blocks before, the bytes it may grow by
+  ~RingLoan() {
+    if (bytes <= RING_KEEP || f->ring_mem.size() == blocks) return;
+    (void)hipStreamSynchronize(h->st);
+    f->ring.resize(count);
+    for (; f->ring_mem.size() > blocks; f->ring_mem.pop_back())
+      if (f->ring_mem.back()) (void)hipFree(f->ring_mem.back());
+  }
+};
 
 // whether a solve may take `bytes` more for a ring of vectors: within the
 // handle's limit, and a quarter of the device's free memory at most
@@ -991,8 +1011,10 @@ struct Ops {
                          int* status) {
     constexpr int NEV = 4, K = CG_KRING, LAG = 1, NR = K + LAG + 1;
     const int have = (int)F(h).ring.size();
+    const size_t grow = have < NR ? (NR - have) * (size_t)half_bytes<P>(h) : 0;
     bool room = max_itr > CG_SHORT;
-    if (room && have < NR) TRY(ring_room(h, (NR - have) * (size_t)half_bytes<P>(h), &room));
+    if (room && grow) TRY(ring_room(h, grow, &room));
+    const RingLoan loan{h, &F(h), F(h).ring.size(), F(h).ring_mem.size(), grow};
     if (room && ensure_ring<P>(h, NR) != DWFGPU_OK) {  // no block of that size
       (void)hipGetLastError();
       room = false;

@@ -1,11 +1,15 @@
 """GPU: the rings of vectors that the CG solvers keep their last steps in.
 
 With DWFGPU_RING_MB=0 (no ring: every step applied at once, the directions in
-place) a solve agrees with the oracle as with a ring.  Bars of the iterates: FP64
+place) a solve agrees with the oracle as with a ring.  A solve gives a ring of
+more than 256 MiB back when it ends, and takes none above the limit.  Bars of the iterates: FP64
 1e-12, FP32 1e-5 and int16 2e-3 of the oracle's after the same steps."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from cps_veloc_amd import dwf
 from cps_veloc_amd import lattice as lat
 from cps_veloc_amd.dwf import BAD_ARG, CgArg, DiracOpDwfGpu, DiracOpMobiusGpu, DwfGpuError
 from oracle.oracle import Oracle
@@ -20,6 +24,12 @@ def make(action, dims, ls, precision="f64", oracle=True):
     g = cls(U, dims, ls, m5=1.8, precision=precision, **kw)
     return g, (Oracle(dims, ls, action, m5=1.8, b=1.5, c=0.5, gauge_canonical=U) if oracle
                else None)
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert dwf.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
 
 
 @pytest.mark.parametrize("ring", ["0", None])
@@ -47,3 +57,20 @@ def test_limit_is_a_number(monkeypatch):
     with pytest.raises(DwfGpuError) as e:
         make("dwf", (4, 2, 2, 6), 4, oracle=False)
     assert e.value.code == BAD_ARG
+
+
+def test_large_ring_is_given_back(monkeypatch):
+    # 16^3x32 Ls 8 FP64: 96 MiB a vector, 960 MiB of ring
+    for ring in (None, "100"):
+        if ring is not None:
+            monkeypatch.setenv("DWFGPU_RING_MB", ring)
+        g, _ = make("dwf", (16, 16, 16, 32), 8, oracle=False)
+        x, b = g.vector(), g.vector(np.random.default_rng(3).standard_normal(g.n))
+        g.InvCg_dev(x, b, CgArg(0.1, 3, 1e-15))  # allocates the work vectors
+        before = free_bytes()
+        g.InvCg_dev(x, b, CgArg(0.1, 14, 1e-15))
+        print(f"[gpu] ring={ring}: {(before - free_bytes()) / 2**20:.0f} MiB kept", flush=True)
+        assert before - free_bytes() <= 256 << 20
+        x.free()
+        b.free()
+        g.close()
