@@ -399,12 +399,15 @@ struct RingLoan {
   }
 };
 
-// whether a solve may take `bytes` more for a ring of vectors: within the
-// handle's limit, and a quarter of the device's free memory at most
-int ring_room(const dwfgpu_s* h, size_t bytes, bool* ok) {
+// Whether a solve may take `bytes` more for a ring of vectors: within the
+// handle's limit, and at most a quarter of the device memory that is free beside
+// the `rest` which the solve allocates in any case.  Every solver with a ring asks
+// this and runs without one otherwise, so that a ring never takes what a graph, a
+// caller's next vectors or another handle needs.
+int ring_room(const dwfgpu_s* h, size_t bytes, size_t rest, bool* ok) {
   size_t avail = 0, total = 0;
   HIPCHK(hipMemGetInfo(&avail, &total));
-  *ok = bytes <= h->ring_max && bytes <= avail / 4;
+  *ok = bytes <= h->ring_max && rest <= avail && bytes <= (avail - rest) / 4;
   return DWFGPU_OK;
 }
 
@@ -1013,7 +1016,7 @@ struct Ops {
     const int have = (int)F(h).ring.size();
     const size_t grow = have < NR ? (NR - have) * (size_t)half_bytes<P>(h) : 0;
     bool room = max_itr > CG_SHORT;
-    if (room && grow) TRY(ring_room(h, grow, &room));
+    if (room && grow) TRY(ring_room(h, grow, 0, &room));
     const RingLoan loan{h, &F(h), F(h).ring.size(), F(h).ring_mem.size(), grow};
     if (room && ensure_ring<P>(h, NR) != DWFGPU_OK) {  // no block of that size
       (void)hipGetLastError();
@@ -2050,25 +2053,31 @@ struct MrState {
   int* flag() const { return ibuf + nrhs; }
   int* iters() const { return ibuf + 2 * nrhs; }
 
-  // the buffers, zeroed; cg: rs, xs and a ring of directions too
+  // the buffers, zeroed; cg: rs, xs and a ring of directions too, if there is room
   int create(dwfgpu_s* h, int n, int partials, bool cg) {
     nrhs = n;
     gx = partials;
-    for (nring = cg ? MR_RING : 1;; nring = 1) {
-      const size_t bytes = carve(h, nullptr, cg);
-      if (hipMalloc((void**)&block, bytes) == hipSuccess) {
-        carve(h, block, cg);
-        HIPCHK(hipMemsetAsync(block, 0, bytes, h->st));
-        return DWFGPU_OK;
-      }
-      block = nullptr;
-      if (nring > 1) {  // without room for the ring
+    size_t bytes = carve(h, nullptr, cg);
+    if (cg) {
+      const size_t least = bytes;
+      nring = MR_RING;
+      bytes = carve(h, nullptr, cg);
+      bool room = false;
+      TRY(ring_room(h, bytes - least, least, &room));
+      if (room && hipMalloc((void**)&block, bytes) != hipSuccess) {
         (void)hipGetLastError();
-        continue;
+        block = nullptr;
+        room = false;
       }
-      HIPCHK(hipGetLastError());
-      return DWFGPU_HIP_ERROR;
+      if (!room) {
+        nring = 1;
+        bytes = least;
+      }
     }
+    if (!block) HIPCHK(hipMalloc((void**)&block, bytes));
+    carve(h, block, cg);
+    HIPCHK(hipMemsetAsync(block, 0, bytes, h->st));
+    return DWFGPU_OK;
   }
 
  private:
@@ -2628,11 +2637,13 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
                        hipHostMallocDefault));
   for (auto& e : w.ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   // K pending steps and LAG steps ahead need K + LAG + 1 residuals; the live
-  // p0 is one vector more.  Where they do not fit, or the solve is too short to
-  // gain from them: every step flushed at once, the residual in place and p0
-  // the first shift's own direction.
+  // p0 is one vector more.  Without room for them (ring_room), or in a solve too
+  // short to gain from them: every step flushed at once, the residual in place
+  // and p0 the first shift's own direction.
   int K = MS_MAXK, LAG = 2, NR = K + LAG + 1;
-  if (max_num_iter <= 4 || hipMalloc(&w.mem, (size_t)(NR + 1) * vbytes) != hipSuccess) {
+  bool room = max_num_iter > 4;
+  if (room) TRY(ring_room(h, (NR + 1) * vbytes, 0, &room));
+  if (!room || hipMalloc(&w.mem, (NR + 1) * vbytes) != hipSuccess) {
     (void)hipGetLastError();
     w.mem = nullptr;
     K = NR = 1;
