@@ -3896,8 +3896,7 @@ int dwfgpu_vec_create(dwfgpu_t h, dwfgpu_vec_t* v) {
 
 int dwfgpu_vec_destroy(dwfgpu_vec_t v) {
   if (!v) return DWFGPU_BAD_ARG;
-  (void)hipStreamSynchronize(v->h->st);
-  free_vec(&v->v);
+  free_vec(&v->v);  // hipFree waits for the device; v->h may be destroyed already
   delete v;
   return DWFGPU_OK;
 }
@@ -4192,8 +4191,7 @@ int dwfgpu_mvec_create(dwfgpu_t h, int nrhs, dwfgpu_mvec_t* out) {
 
 int dwfgpu_mvec_destroy(dwfgpu_mvec_t v) {
   if (!v) return DWFGPU_BAD_ARG;
-  (void)hipStreamSynchronize(v->h->st);
-  free_vec(&v->v);
+  free_vec(&v->v);  // hipFree waits for the device; v->h may be destroyed already
   delete v;
   return DWFGPU_OK;
 }
