@@ -3731,7 +3731,7 @@ int dwfgpu_create(const double* gauge, const int dims[4], int ls, int action, do
     }
     h->grid_hop = std::max(h->grid_hop, (h->g.vh + ns - 1) / ns);
   }
-  set_shape64(h);
+  if (!env_ns) set_shape64(h);  // DWFGPU_NS: the general hop kernels on every lattice
   h->npartial = std::max({h->grid_hop, h->grid64, dwfk::BLAS_BLOCKS});
   int r = DWFGPU_OK;
   auto fail = [&](int code) {
@@ -4225,10 +4225,11 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
       hipLaunchKernelGGL((dwfk::k_convert<P, P64>), blas_grid(), blas_block(), 0, h->st,
                          fld<P>(mslice<P>(h, m.ps[0], j)), cfld<P64>(mslice<P64>(h, in->v, j)), h->g);
     HIPCHK(hipGetLastError());
-    MrShape t{Ops<P>::sites(h), 1};
-    if (h->action == DWFGPU_DWF && pidx<P>() == DWFGPU_F64 && h->ns64) {
-      // the passes of a single right-hand side on this lattice, all in one launch
-      TRY(mr_pinned(h, nrhs, sizeof(double), &t));
+    // the small-lattice passes of a single right-hand side, unless a shape is pinned
+    const bool small = pidx<P>() == DWFGPU_F64 && h->ns64 &&
+                       !(h->action == DWFGPU_DWF && getenv("DWFGPU_MRHS_SHAPE"));
+    MrShape t{small ? h->ns64 : Ops<P>::sites(h), 1};
+    if (h->action == DWFGPU_DWF && small) {  // all of them in one launch
       const double mk2 = -dwf_kappa(h) * dwf_kappa(h);
       Geom fwd = h->g, back = h->g;
       back.rev = 1;
@@ -4245,7 +4246,7 @@ int dwfgpu_matpcdagmatpc_mrhs_dev(dwfgpu_t h, int precision, const double* masse
     } else if (h->action == DWFGPU_DWF) {
       TRY(mr_tune<P>(h, m, &t));
       TRY(mr_mdagm<P>(h, t, m, m.rs, m.ps[0], nullptr, false));
-    } else if (pidx<P>() == DWFGPU_F64 && h->ns64) {  // as a single right-hand side
+    } else if (small) {
       for (int j = 0; j < nrhs; ++j)
         TRY(Ops<P>::mdagm(h, masses[j], mslice<P>(h, m.rs, j), mslice<P>(h, m.ps[0], j), nullptr));
     } else {
