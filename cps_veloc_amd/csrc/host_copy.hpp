@@ -5,11 +5,12 @@
 // reached 10 GB/s into a freshly allocated array (its pages are touched for the
 // first time by that thread), 16 GB/s into a used one and 27 GB/s to the
 // device, against 57 GB/s of the link from pinned memory.  Here the link moves
-// chunks between the device and a ring of pinned buffers while WORKERS threads
+// chunks between the device and a ring of pinned buffers while up to 8 threads
 // move them between the ring and the caller's array.  Measured, 1.02 GB: 97 ->
 // 24 ms into a fresh array (43 GB/s), 35 -> 22 ms to the device (45 GB/s).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <sched.h>
 
 #include <algorithm>
 #include <atomic>
@@ -25,7 +26,7 @@ namespace hostcopy {
 constexpr size_t CHUNK = (size_t)4 << 20;  // the largest chunk, one buffer of the ring
 constexpr int NBUF = 8;                    // 32 MiB of pinned memory in all
 constexpr int LAG = 4;                     // chunks on the link before the oldest is waited for
-constexpr int WORKERS = 8;
+constexpr int WORKERS = 8;                 // at most: see workers()
 // Smaller copies are left to hipMemcpy: starting the threads costs about 0.1 ms
 // (9.4 MB: 0.57 -> 0.43 ms to the host, but 0.29 -> 0.42 ms to the device, where
 // hipMemcpy itself reaches 29-32 GB/s; 201 MB to the device 7.0 -> 4.7 ms).
@@ -59,6 +60,17 @@ inline void release() {
   }
 }
 
+// Threads of a copy: one for each core that the caller may run on beside its own,
+// since threads that wait do so on the core (a waiting thread that sleeps would
+// be woken for every chunk of 0.1 ms).  0, a single core: hipMemcpy's one thread.
+inline int workers() {
+  cpu_set_t set;
+  const int n = sched_getaffinity(0, sizeof set, &set) == 0
+                    ? CPU_COUNT(&set)
+                    : (int)std::thread::hardware_concurrency();
+  return std::max(0, std::min(WORKERS, n - 1));
+}
+
 // (to the device: in order on st, whose work the callers wait for before they
 // return to their own)
 inline hipError_t direct(void* dev, void* host, size_t bytes, bool to_host, hipStream_t st) {
@@ -80,9 +92,10 @@ inline bool pinned(const void* host) {
 inline hipError_t copy(void* dev, void* host, size_t bytes, bool to_host, hipStream_t st) {
   if (bytes < (to_host ? MIN_TO_HOST : MIN_TO_DEVICE) || pinned(host))
     return direct(dev, host, bytes, to_host, st);
+  const int nworker = workers();
   Ring& r = ring();
   std::unique_lock<std::mutex> own(r.mu, std::try_to_lock);
-  if (!own.owns_lock()) return direct(dev, host, bytes, to_host, st);
+  if (nworker == 0 || !own.owns_lock()) return direct(dev, host, bytes, to_host, st);
   if (!r.pin && hipHostMalloc((void**)&r.pin, NBUF * CHUNK, hipHostMallocPortable) != hipSuccess) {
     (void)hipGetLastError();
     r.pin = nullptr;
@@ -127,7 +140,7 @@ inline hipError_t copy(void* dev, void* host, size_t bytes, bool to_host, hipStr
   std::thread pool[WORKERS];
   int started = 0;
   try {
-    for (; started < WORKERS; ++started) pool[started] = std::thread(worker);
+    for (; started < nworker; ++started) pool[started] = std::thread(worker);
   } catch (...) {  // fewer threads than asked for
   }
   hipError_t err = hipSuccess;
