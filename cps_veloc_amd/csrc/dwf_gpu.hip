@@ -2666,6 +2666,7 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
   F.vs = F.n = n;
   F.nshift = nshift;
   F.single = multi ? 0 : 1;
+  F.all = ~0u;
   int slot = 0;
   auto pending = [&]() { return w.hsteps + (size_t)slot * MS_MAXK + F.cnt; };
   auto flush = [&]() -> int {
@@ -2678,6 +2679,7 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
     HIPCHK(hipGetLastError());
     F.cnt = 0;
     F.active = 0;
+    F.all = ~0u;
     F.chi = nullptr;
     slot = (slot + 1) % MS_SLOTS;
     return DWFGPU_OK;
@@ -2729,6 +2731,7 @@ int minvcg_run(dwfgpu_s* h, double mass, const double* shift, int nshift, const 
     }
     F.r[F.cnt++] = res(k);
     F.active |= e->psi | e->p;
+    F.all &= e->psi & e->p;
     todo = 0;
   };
   // the recurrences of step k from its scalars

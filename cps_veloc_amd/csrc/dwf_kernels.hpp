@@ -2225,6 +2225,7 @@ struct MsFlush {
   size_t vs, n;           // vector stride and length
   int cnt, nshift, single;
   unsigned active;        // shifts that any of the steps moves
+  unsigned all;           // shifts whose psi and p every step moves
 };
 
 template <int K>
@@ -2247,12 +2248,22 @@ k_ms_flush(MsFlush a, const MsStep* __restrict__ st) {
         acc = cx<double>{0, 0};
         if (!a.chi) acc = *qs;
       }
+      if ((a.all >> s) & 1u) {  // no test in each step (12^3x24 Ls 8, 10
+        // shifts: 182 us a flush with them in all, 177 this way)
 #pragma unroll
-      for (int j = 0; j < K; ++j)
-        if (j < a.cnt) {
-          if ((st[j].psi >> s) & 1u) acc = st[j].f[s] * p + acc;
-          if ((st[j].p >> s) & 1u) p = st[j].zr[s] * r[j] + st[j].ap[s] * p;
-        }
+        for (int j = 0; j < K; ++j)
+          if (j < a.cnt) {
+            acc = st[j].f[s] * p + acc;
+            p = st[j].zr[s] * r[j] + st[j].ap[s] * p;
+          }
+      } else {
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+          if (j < a.cnt) {
+            if ((st[j].psi >> s) & 1u) acc = st[j].f[s] * p + acc;
+            if ((st[j].p >> s) & 1u) p = st[j].zr[s] * r[j] + st[j].ap[s] * p;
+          }
+      }
       *ps = p;
       if (!a.single) *qs = acc;
     }
