@@ -273,12 +273,15 @@ size_t hop_lds_bytes(int action, int ls, int ns, size_t creal) {
 // timing MatPcDagMatPc (ms with 16 / the sites taken):
 //   DWF, whose work-groups only meet at the staged links: FP64 32, or 64 to Ls 8
 //     (24^3x64 Ls 12 4.20 / 3.75, 16^3x32 Ls 16 0.804 / 0.740, Ls 8 0.444 /
-//     0.417): rows of 512 bytes and more from one work-group.  FP32 the shape of
-//     eight whole waves (16^3x32 Ls 16 0.342 / 0.332, 24^3x64 Ls 8 1.32 / 1.19);
-//     where Ls leaves fewer (Ls 10, 12) two such work-groups waste the wave slots
-//     they do not fill (0.108 / 0.112), and 16 stays.  16 bits 16 above Ls 8
-//     (24^3x64 Ls 12 1.18 / 1.30 with 32), 32 to it (16^3x32 Ls 8 0.130 / 0.124)
-//     and 64 to Ls 4 (0.117 / 0.104).
+//     0.417): rows of 512 bytes and more from one work-group.  FP32 at Ls 8 and 16
+//     the shape of eight whole waves (16^3x32 Ls 16 0.343 / 0.327, Ls 8 0.189 /
+//     0.174, 24^3x64 Ls 8 1.32 / 1.19); where Ls leaves fewer (Ls 10, 12) 32
+//     sites are within 4 % either way (0.108 / 0.112; 16^3x32 Ls 10 0.230 /
+//     0.224, Ls 12 0.255 / 0.254), and 16 stays.  FP32 at Ls 4 and 6 as 16 bits:
+//     64 to Ls 4 (16^3x32 0.124 / 0.118; eight waves would be 128 sites, not
+//     measured) and 32 to Ls 8 (Ls 6 0.161 / 0.154, 64 sites 0.162).  16 bits 16
+//     above Ls 8 (24^3x64 Ls 12 1.18 / 1.30 with 32), 32 to it (16^3x32 Ls 8
+//     0.130 / 0.124, Ls 6 0.129 / 0.119) and 64 to Ls 4 (0.117 / 0.104).
 //   Moebius, whose s-columns take LDS and more barriers: four waves, so 32 for
 //     Ls 5 to 8 (24^3x64 Ls 8 FP64 2.50 / 2.42, FP32 1.20 / 1.15; 16^3x32 Ls 6
 //     int16 0.137 / 0.124), 16 otherwise (24^3x64 Ls 12 3.68 / 4.00, Ls 4 0.248 /

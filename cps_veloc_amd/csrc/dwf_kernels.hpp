@@ -1065,9 +1065,10 @@ struct CgEpi {
   const double* scal;
 };
 
-// PX = NoX: the epilogue updates r only; x += alpha p is left to the pass
-// that forms the next direction (k_cg_xp), which reads p anyway.  This keeps
-// the x traffic and its arithmetic out of the hop kernel.
+// PX = NoX: the epilogue updates r only; x += alpha p is left to a pass over
+// several steps' directions (k_x_flush) or, without a ring of them, to the one
+// that forms the next direction (k_cg_xp).  This keeps the x traffic and its
+// arithmetic out of the hop kernel.
 struct NoX {
   typedef float R;
   typedef float S;
@@ -1765,8 +1766,9 @@ k_pnext(Fld<P> pn, CFld<P> r, CFld<P> p, const double* __restrict__ scal, Geom g
   }
 }
 
-// x += a_0 p_0, then += a_1 p_1, ... (the order and the rounding of one
-// update per CG step, k_cg_xp): the x updates of cnt steps in one pass
+// x += a_0 p_0, then += a_1 p_1, ... (the order of one update per CG step and,
+// in FP64 and FP32, its rounding; a 16-bit x is rounded once): the x updates of
+// cnt steps in one pass
 constexpr int XFLUSH_MAX = 16;
 template <class P>
 struct XFlush {
@@ -2363,8 +2365,7 @@ k_ms_reduce(const double* __restrict__ partial, int n, double sigma, double stop
 // is how a converged RHS retires without changing any launch shape.
 // ---------------------------------------------------------------------------
 constexpr int MR_NSCAL = 8;
-enum { MR_RR = 0, MR_D = 1, MR_RRNEW = 2, MR_BETA = 3, MR_STOP = 4, MR_RRUPD = 5, MR_DELTA2 = 6,
-       MR_MAXIT = 7 };
+enum { MR_RR = 0, MR_D = 1, MR_BETA = 2, MR_STOP = 3, MR_RRUPD = 4, MR_DELTA2 = 5, MR_MAXIT = 6 };
 
 template <class P>
 struct MrArgs {
@@ -2529,7 +2530,6 @@ k_cg_end_mrhs(const double* __restrict__ partial, int n, double* __restrict__ sc
   if (threadIdx.x) return;
   double* sc = scal + (size_t)j * MR_NSCAL;
   alpha[(size_t)j * nslot + slot] = cg_alpha(sc);
-  sc[MR_RRNEW] = rrn;
   iters[j] += 1;
   if (sc[MR_D] == 0.0) {
     active[j] = 0;

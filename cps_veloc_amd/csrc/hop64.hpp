@@ -245,8 +245,9 @@ __device__ __forceinline__ double cg_alpha64(const CgScal64& c, const double* sh
 // and the next direction pn = r + (|r|^2 / *rr_old) p of n components, one a
 // thread.  The two sums as launches of their own cost an 8^4 Ls 8 DWF step 5.2
 // us and two gaps; inside the last pass (7.5 -> 7.9 us) and here (3.4 -> 3.6 us)
-// the step takes 40.3 us instead of 46.1.  More partials than a small lattice's
-// (at most 1024) would cost every work-group more than the launch saves.
+// the step takes 40.3 us instead of 46.1.  Every work-group reads
+// all partials, one for each 8 or 4 sites: 256 here, 2048 at the line of
+// set_shape64() (Ls 2), and on a larger lattice more than the launch saves.
 __global__ void __launch_bounds__(256)
 k_cg_end64(c64* __restrict__ pn, const c64* __restrict__ r, const c64* __restrict__ p,
            const double* __restrict__ partial, int np, const double* __restrict__ rr_old,
