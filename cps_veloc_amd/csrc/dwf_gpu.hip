@@ -24,6 +24,15 @@
 #include "ptc_kernels.hpp"
 #include "roofline.h"
 
+// 256 work-groups: 16 to 64 of them took 75.5 MB in 1.96 to 1.77 ms, 256 in 1.72
+hipError_t hostcopy::to_pinned(void* pin, const void* dev, size_t bytes, hipStream_t st) {
+  if (((uintptr_t)pin | (uintptr_t)dev | bytes) % 16)
+    return hipMemcpyAsync(pin, dev, bytes, hipMemcpyDeviceToHost, st);
+  hipLaunchKernelGGL(dwfk::k_copy16, dim3(256), dim3(256), 0, st, (uint4*)pin, (const uint4*)dev,
+                     bytes / 16);
+  return hipGetLastError();
+}
+
 using dwfk::cx;
 using dwfk::Geom;
 using dwfk::M5Side;

@@ -6,8 +6,9 @@
 // first time by that thread), 16 GB/s into a used one and 27 GB/s to the
 // device, against 57 GB/s of the link from pinned memory.  Here the link moves
 // chunks between the device and a ring of pinned buffers while up to 8 threads
-// move them between the ring and the caller's array.  Measured, 1.02 GB: 97 ->
-// 24 ms into a fresh array (43 GB/s), 35 -> 22 ms to the device (45 GB/s).
+// move them between the ring and the caller's array.  Measured, 1.02 GB: 98 ->
+// 24 ms into a fresh array (43 GB/s), 58 -> 20 ms into a used one, 34 -> 22 ms to
+// the device (45 GB/s).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <sched.h>
@@ -28,12 +29,13 @@ constexpr int NBUF = 8;                    // 32 MiB of pinned memory in all
 constexpr int LAG = 4;                     // chunks on the link before the oldest is waited for
 constexpr int WORKERS = 8;                 // at most: see workers()
 // Smaller copies are left to hipMemcpy: starting the threads costs about 0.1 ms
-// (9.4 MB: 0.57 -> 0.43 ms to the host, but 0.29 -> 0.42 ms to the device, where
-// hipMemcpy itself reaches 29-32 GB/s; 201 MB to the device 7.0 -> 4.7 ms).
+// (to the host 4.7 MB 0.28 / 0.28 ms, 9.4 MB 0.57 -> 0.37; to the device 9.4 MB
+// 0.29 -> 0.42, where hipMemcpy itself reaches 29-32 GB/s, 201 MB 7.0 -> 4.7).
 constexpr size_t MIN_TO_HOST = (size_t)4 << 20, MIN_TO_DEVICE = (size_t)64 << 20;
 // An eighth of a small copy a chunk, so that the threads start early; 4 MiB of
 // a large one, because each chunk costs the link about 15 us beside its bytes
-// (1 GiB to a fresh array: 30, 38 and 43 GB/s with chunks of 1, 2 and 4 MiB).
+// (1 GiB to a fresh array, moved by hipMemcpyAsync: 30, 38 and 43 GB/s with chunks
+// of 1, 2 and 4 MiB).
 constexpr size_t MIN_CHUNK = (size_t)512 << 10;
 
 // The pinned ring: one for the process, kept while any handle is alive.  A
@@ -87,6 +89,16 @@ inline bool pinned(const void* host) {
   (void)hipGetLastError();  // an unknown address is not an error here
   return false;
 }
+
+// bytes of device memory into a pinned buffer, by a kernel (dwf_gpu.hip).  Not
+// hipMemcpyAsync: that is the DMA engine's, and with an event behind each copy
+// the engine and the stream's queue wait for each other, 25 us a chunk and, in
+// phases such as the 30 ms after a batched operator call, 130 us (copy trace; the
+// copy of 0.7 MB itself takes 17).  5.8 MB to the host 0.36 and, in such a phase,
+// 1.26 ms, where one hipMemcpy took 0.35; 151 MB 8.0 ms.  By kernel 0.29 and 3.2
+// ms, in either state.
+__attribute__((visibility("hidden"))) hipError_t to_pinned(void* pin, const void* dev,
+                                                          size_t bytes, hipStream_t st);
 
 // dev <-> host, after the work queued on st; to the host complete on return
 inline hipError_t copy(void* dev, void* host, size_t bytes, bool to_host, hipStream_t st) {
@@ -154,7 +166,7 @@ inline hipError_t copy(void* dev, void* host, size_t bytes, bool to_host, hipStr
       if (t < n) {
         if (to_host ? t >= NBUF : true) wait(to_host ? t - NBUF : t);
         char *p = pin + (t % NBUF) * CHUNK, *d = (char*)dev + t * chunk;
-        err = to_host ? hipMemcpyAsync(p, d, len(t), hipMemcpyDeviceToHost, st)
+        err = to_host ? to_pinned(p, d, len(t), st)
                       : hipMemcpyAsync(d, p, len(t), hipMemcpyHostToDevice, st);
         if (err == hipSuccess) err = hipEventRecord(ev.e[t % NBUF], st);
       }
