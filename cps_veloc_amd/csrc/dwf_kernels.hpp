@@ -441,6 +441,17 @@ __host__ __device__ __forceinline__ Nbr neighbours(const Geom& g, int i, int par
   return n;
 }
 
+// The size of the work-group, from the packet.  blockDim's reads also ask whether
+// the group is a partial last one (there is none), which the compiler only folds
+// away where it knows the kernel around them: in kernels whose body is a device
+// function shared by two (mobius_pass, x_flush) it chose between two 16-bit values
+// in memory by vector loads, before anything else of the work-group.  Moebius
+// MatPcDagMatPc 24^3x64 Ls 12: FP64 3.542 -> 3.485 ms, bf16 1.190 -> 1.177, int16
+// 1.188 -> 1.173, FP32 1.733 -> 1.716.
+__device__ __forceinline__ int wg_x() { return __builtin_amdgcn_workgroup_size_x(); }
+__device__ __forceinline__ int wg_y() { return __builtin_amdgcn_workgroup_size_y(); }
+__device__ __forceinline__ int wg_z() { return __builtin_amdgcn_workgroup_size_z(); }
+
 // Work-groups are dispatched round-robin over the XCDs (hardware id b runs on
 // XCD b % nxcd).  Renumber them so that XCD k receives one contiguous range of
 // logical ids; neighbouring sites then share that XCD's L2.
@@ -719,8 +730,8 @@ __device__ __forceinline__ void stage_links(cx<typename P::R>* __restrict__ lu,
                                             int blk, int ns, int nsets, int p_first) {
   typedef typename P::R R;
   constexpr int NE = P::kLinkElems;
-  const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-  const int nthr = blockDim.x * blockDim.y * blockDim.z;
+  const int tid = threadIdx.x + wg_x() * (threadIdx.y + wg_y() * threadIdx.z);
+  const int nthr = wg_x() * wg_y() * wg_z();
   for (int w = tid; w < nsets * 8 * ns; w += nthr) {
     const int il = w % ns, d = (w / ns) % 8, set = w / (8 * ns);
     const int i = blk * ns + il;
@@ -900,8 +911,8 @@ __device__ __forceinline__ void stage_links_pq(LinkPQ* __restrict__ lu, int* __r
                                                const uint32_t* __restrict__ U, const Geom& g,
                                                int blk, int ns, int nsets, int p_first) {
   constexpr int NE = PI16::kLinkElems;
-  const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-  const int nthr = blockDim.x * blockDim.y * blockDim.z;
+  const int tid = threadIdx.x + wg_x() * (threadIdx.y + wg_y() * threadIdx.z);
+  const int nthr = wg_x() * wg_y() * wg_z();
   for (int w = tid; w < nsets * 8 * ns; w += nthr) {
     const int il = w % ns, d = (w / ns) % 8, set = w / (8 * ns);
     const int i = blk * ns + il;
@@ -1030,8 +1041,8 @@ __device__ __forceinline__ void hop4(cx<R>* acc, const LD& ld, const cx<R>* lu, 
 // sum over the work-group; result valid in thread 0.  Fixed order, so the
 // total is reproducible run to run.
 __device__ __forceinline__ double block_sum(double v, double* sh) {
-  const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-  const int nthr = blockDim.x * blockDim.y * blockDim.z;
+  const int tid = threadIdx.x + wg_x() * (threadIdx.y + wg_y() * threadIdx.z);
+  const int nthr = wg_x() * wg_y() * wg_z();
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
   if ((tid & 63) == 0) sh[tid >> 6] = v;
@@ -1126,7 +1137,7 @@ k_dwf_dslash(Fld<P> out, CFld<P> in, const typename P::S* __restrict__ U, CFld<P
   typedef typename P::R R;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double sh[16];
-  const int ns = blockDim.x, il = threadIdx.x, s = threadIdx.y;
+  const int ns = wg_x(), il = threadIdx.x, s = threadIdx.y;
   int* lnb = reinterpret_cast<int*>(smem_raw);                   // [2][8][ns]
   cx<R>* lu = reinterpret_cast<cx<R>*>(smem_raw + 2 * 8 * ns * 4);  // [2][8][ns][9]
   const double a_cg = CG ? cg_alpha(cg.scal) : 0.0;
@@ -1281,8 +1292,8 @@ __device__ __forceinline__ void m5inv_column_reg(cx<R>* v, bool upper, const M5S
 template <int DAG, typename R>
 __device__ __forceinline__ void m5inv_columns(cx<R>* col, int sst, int ns, int nvalid, int ls,
                                               const M5Side& k) {
-  const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-  const int nthr = blockDim.x * blockDim.y * blockDim.z;
+  const int tid = threadIdx.x + wg_x() * (threadIdx.y + wg_y() * threadIdx.z);
+  const int nthr = wg_x() * wg_y() * wg_z();
   for (int w = tid; w < ns * 12; w += nthr) {
     const int cc = w / ns, sl = w - cc * ns;
     if (sl >= nvalid) continue;
@@ -1381,7 +1392,7 @@ __device__ __forceinline__ void mobius_pass(Fld<P> out, CFld<P> in, CFld<P> psi,
   typedef typename P::R R;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double sh[16];
-  const int ns = blockDim.x, il = threadIdx.x, s = threadIdx.y;
+  const int ns = wg_x(), il = threadIdx.x, s = threadIdx.y;
   int* lnb = reinterpret_cast<int*>(smem_raw);                   // neighbours [8][ns]
   cx<R>* lu = reinterpret_cast<cx<R>*>(smem_raw + 8 * ns * 4);  // staged links [8][ns][9]
   // s-columns [ns][sst] reuse the LDS of the links and neighbour indices,
@@ -1586,7 +1597,7 @@ k_m5inv(Fld<P> out, CFld<P> in, Geom g, M5Side k) {
   typedef typename P::R R;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cx<R>* col = reinterpret_cast<cx<R>*>(smem_raw);
-  const int ns = blockDim.x, il = threadIdx.x, s = threadIdx.y;
+  const int ns = wg_x(), il = threadIdx.x, s = threadIdx.y;
   const int sst = g.ls * 12 + 1;
   const int blk = xcd_block(g.nxcd, g.rev);
   const int i = blk * ns + il;
@@ -1629,8 +1640,8 @@ __device__ __forceinline__ void st_site_k(Fld<P> f, const Geom& g, size_t k,
 }
 
 #define DWFK_SITE_LOOP(k, g) \
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < (size_t)(g).vh * (g).ls; \
-       k += (size_t)gridDim.x * blockDim.x)
+  for (size_t k = blockIdx.x * (size_t)dwfk::wg_x() + threadIdx.x; k < (size_t)(g).vh * (g).ls; \
+       k += (size_t)gridDim.x * dwfk::wg_x())
 
 template <class P>
 __global__ void __launch_bounds__(BLAS_THREADS)
@@ -1788,8 +1799,8 @@ __device__ __forceinline__ void x_flush(const Fld<PX>& x, const XFlush<P>& f, co
   typedef typename PX::R RX;
   if constexpr (!P::kScaled && std::is_same<P, PX>::value) {
     const size_t n = (size_t)nch<P>() * g.vh * g.ls;
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
-         e += (size_t)gridDim.x * blockDim.x) {
+    for (size_t e = blockIdx.x * (size_t)wg_x() + threadIdx.x; e < n;
+         e += (size_t)gridDim.x * wg_x()) {
       cx<R> xv[P::kCPC];
       ld_chunk<P>(x.d + e, xv);
       for (int j = 0; j < f.cnt; j += 4) {  // four directions in flight
