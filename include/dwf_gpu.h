@@ -116,6 +116,7 @@ int dwfgpu_matinv(dwfgpu_t h, const dwfgpu_cg_arg *arg, double *out, const doubl
                   double *true_res, int *iters);
 
 /* ---- device-resident vectors (no PCIe traffic per call) --------------- */
+/* A vector may be destroyed after its handle, but not used.                 */
 int dwfgpu_vec_create(dwfgpu_t h, dwfgpu_vec_t *v);
 int dwfgpu_vec_destroy(dwfgpu_vec_t v);
 int dwfgpu_vec_upload(dwfgpu_vec_t v, const double *host_cps_order);
